@@ -3031,16 +3031,130 @@ __global__ void __launch_bounds__(256) k_blit(const float *color, uint64_t plane
     }
 }
 
+// ---------------------------------------------------------------------------
+// Workgroup sort in registers: ascending bitonic sort of the first m of
+// blockDim.x * E values, E per thread (value e of a thread is element wave *
+// 64 E + 64 e + lane); m a power of two, and all of them unless E is 1.  Exchanges at a distance below 64
+// are lane exchanges, below 64 E register exchanges; only those between
+// waves go through LDS (sh, one word per element) with barriers.
+// ---------------------------------------------------------------------------
+// Lane l's value from lane l ^ J: a DPP move where the hardware has one, else
+// a swizzle (within 32 lanes) or a permute.
+template <int J> __device__ __forceinline__ int32_t lane_xor(int32_t v) {
+    if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);          // quad_perm 1 0 3 2
+    else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);     // quad_perm 2 3 0 1
+    else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);    // row_ror 8
+    else if constexpr (J < 32) return __builtin_amdgcn_ds_swizzle(v, (J << 10) | 0x1F);       // xor within 32 lanes
+    else return __shfl_xor(v, J, 64);
+}
+
+template <int J, class T, int E> __device__ __forceinline__ void sort_lanes(T (&v)[E], uint32_t i0, uint32_t k) {
+    const bool low = (threadIdx.x & J) == 0u;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        T o = lane_xor<J>(v[e]);
+        bool up = ((i0 + 64u * e) & k) == 0u;
+        if ((o < v[e]) == (low == up)) v[e] = o;
+    }
+}
+
+template <int Q, class T, int E> __device__ __forceinline__ void sort_regs(T (&v)[E], uint32_t i0, uint32_t k) {
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if ((e & Q) == 0 && e + Q < E) {
+            bool up = ((i0 + 64u * e) & k) == 0u;
+            T a = v[e], b = v[e + Q];
+            if ((b < a) == up) {
+                v[e] = b;
+                v[e + Q] = a;
+            }
+        }
+    }
+}
+
+template <class T, int E> __device__ __forceinline__ void block_sort(T (&v)[E], T *sh, uint32_t m) {
+    static_assert(E == 1 || E == 2 || E == 4 || E == 8, "values per thread");
+    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
+    for (uint32_t k = 2; k <= m; k <<= 1) {
+        for (uint32_t j = k >> 1; j >= 64u * E; j >>= 1) {
+#pragma unroll
+            for (int e = 0; e < E; e++) sh[i0 + 64u * e] = v[e];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                uint32_t i = i0 + 64u * e;
+                T o = sh[i ^ j];
+                bool low = (i & j) == 0u, up = (i & k) == 0u;
+                if ((o < v[e]) == (low == up)) v[e] = o;
+            }
+            __syncthreads();
+        }
+        if (E >= 8 && k >= 512u) sort_regs<4>(v, i0, k);
+        if (E >= 4 && k >= 256u) sort_regs<2>(v, i0, k);
+        if (E >= 2 && k >= 128u) sort_regs<1>(v, i0, k);
+        if (k >= 64u) sort_lanes<32>(v, i0, k);
+        if (k >= 32u) sort_lanes<16>(v, i0, k);
+        if (k >= 16u) sort_lanes<8>(v, i0, k);
+        if (k >= 8u) sort_lanes<4>(v, i0, k);
+        if (k >= 4u) sort_lanes<2>(v, i0, k);
+        sort_lanes<1>(v, i0, k);
+    }
+}
+
 // Renderer::update_auto_exposure (src/renderer.rs:258-290) on the device: one
-// workgroup sorts the tiles' log luminance in LDS (bitonic, on the order of
-// f32::total_cmp), one lane sums the trimmed middle in sorted order and
-// steps the exposure.  state = {ev, target, exposure}; with use_host the
-// step starts from (host_ev, host_target) instead of the stored state.
-// The device's log2f / expf / powf may differ from the host libm's by an
-// ulp, so the exposure agrees with the host step to a few ulps.
+// workgroup sorts the tiles' log luminance (on the order of f32::total_cmp),
+// one wave sums the trimmed middle in sorted order and steps the exposure.
+// state = {ev, target, exposure}; with use_host the step starts from
+// (host_ev, host_target) instead of the stored state.  The device's log2f /
+// expf / powf may differ from the host libm's by an ulp, so the exposure
+// agrees with the host step to a few ulps.
+//
+// Bound by latency: one workgroup, a sort of 36 to 91 dependent stages and a
+// chain of 0.8 n dependent additions (the sum's order is part of its value).
+// Four values a thread keep all but the widest exchanges in registers (none
+// reach LDS up to 256 tiles), and the chain reads ahead of itself.  Against a
+// bitonic sort in LDS with one lane adding from LDS: 17.4 -> 7.6 us at 240
+// tiles (720p), 28.8 -> 10.3 at 510 (1080p), 94.6 -> 21.4 at 2040 (2160p).  Up
+// to 64 tiles one value a lane, sorted only as far as there are tiles (3.7 ->
+// 2.7 us at 6; four values a lane make 36 stages of it and were slower).
+__device__ __forceinline__ float add_bits(float sum, int4 a) {
+    return (((sum + __int_as_float(a.x)) + __int_as_float(a.y)) + __int_as_float(a.z)) + __int_as_float(a.w);
+}
+
+// v[i] + ... + v[end - 1] in order; v holds float bits.
+__device__ __forceinline__ float exposure_sum(const int32_t *v, uint32_t i, uint32_t end) {
+    float sum = 0.0f;
+    for (; i < end && (i & 3u); i++) sum += __int_as_float(v[i]);
+    const int4 *q = reinterpret_cast<const int4 *>(v);
+    if (i + 16u <= end) {
+        int4 a[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = q[(i >> 2) + j];
+        for (; i + 32u <= end; i += 16u) {
+            int4 b[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) b[j] = q[(i >> 2) + 4 + j];
+#pragma unroll
+            for (int j = 0; j < 4; j++) sum = add_bits(sum, a[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) a[j] = b[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) sum = add_bits(sum, a[j]);
+        i += 16u;
+    }
+    for (; i < end; i++) sum += __int_as_float(v[i]);
+    return sum;
+}
+
+template <int E>
 __global__ void __launch_bounds__(1024) k_exposure(const float *lum, uint32_t n, float dt, int use_host, float host_ev,
-                                                   float host_target, float *state) {
-    __shared__ int32_t key[SR_EXPOSURE_MAX];
+                                                   float host_target, float *state, uint32_t m) {
+    __shared__ __align__(16) int32_t key[E == 1 ? 64 : 1024 * E];
+    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
+    float lv[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) lv[e] = i0 + 64u * e < n ? lum[i0 + 64u * e] : 0.0f;
     float ev = use_host ? host_ev : state[0];
     float target = use_host ? host_target : state[1];
     float dtc = maxps(dt, 0.0f);
@@ -3054,41 +3168,21 @@ __global__ void __launch_bounds__(1024) k_exposure(const float *lum, uint32_t n,
         }
         return;
     }
-    uint32_t m = 1;
-    while (m < n) m <<= 1;
-    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
-        int32_t k = 0x7FFFFFFF;
-        if (i < n) {
-            float sv = log2f(maxps(lum[i], 1e-4f));
-            int32_t b = __float_as_int(sv);
-            k = b ^ (int32_t)(((uint32_t)(b >> 31)) >> 1);
-        }
-        key[i] = k;
+    int32_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        int32_t b = __float_as_int(log2f(maxps(lv[e], 1e-4f)));
+        v[e] = i0 + 64u * e < n ? b ^ (int32_t)(((uint32_t)(b >> 31)) >> 1) : 0x7FFFFFFF;
     }
+    block_sort(v, key, m);
+    // (no wave reads the sort's last exchange here: its barrier has passed)
+#pragma unroll
+    for (int e = 0; e < E; e++) key[i0 + 64u * e] = v[e] ^ (int32_t)(((uint32_t)(v[e] >> 31)) >> 1);
     __syncthreads();
-    for (uint32_t k = 2; k <= m; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
-                uint32_t l = i ^ j;
-                if (l > i) {
-                    int32_t a = key[i], b = key[l];
-                    bool up = (i & k) == 0;
-                    if ((a > b) == up) {
-                        key[i] = b;
-                        key[l] = a;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         uint32_t trim = sat_u32(floorf((float)n * 0.10f));
         trim = min(trim, (n - 1) / 2);
-        float sum = 0.0f;
-        for (uint32_t i = trim; i < n - trim; i++) {
-            int32_t k = key[i];
-            sum += __int_as_float(k ^ (int32_t)(((uint32_t)(k >> 31)) >> 1));
-        }
+        float sum = exposure_sum(key, trim, n - trim);
         float mean = sum / (float)(n - 2 * trim);
         float y = minps(maxps(0.45f, 0.0f), 1.0f);
         float kk = 0.2f;
@@ -3097,9 +3191,12 @@ __global__ void __launch_bounds__(1024) k_exposure(const float *lum, uint32_t n,
         float tev = log2f(meter) - mean;
         float t = minps(maxps(powf(2.0f, tev), 0.05f), 32.0f);
         float nev = ev + (log2f(t) - ev) * alpha;
-        state[0] = nev;
-        state[1] = t;
-        state[2] = powf(2.0f, nev);
+        float exposure = powf(2.0f, nev);
+        if (threadIdx.x == 0) {
+            state[0] = nev;
+            state[1] = t;
+            state[2] = exposure;
+        }
     }
 }
 
@@ -3346,7 +3443,17 @@ hipError_t launch_blit(const float *color, uint64_t plane, int32_t W, int32_t H,
 hipError_t launch_exposure(const float *lum, uint32_t n, float dt, bool use_host, float ev, float target, float *state,
                            hipStream_t st) {
     if (n == 0 || n > SR_EXPOSURE_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_exposure, dim3(1), dim3(1024), 0, st, lum, n, dt, use_host ? 1 : 0, ev, target, state);
+    // one wave up to 64 tiles; then four values a thread up to 4096 tiles
+    // (4K UHD has 2040) in as many waves as they fill, else eight
+    uint32_t m = 1;
+    while (m < n) m <<= 1;
+    if (n > 64) m = std::max(m, 256u);
+#define SR_EXPOSURE(E, threads)                                                                                       \
+    hipLaunchKernelGGL(k_exposure<E>, dim3(1), dim3(threads), 0, st, lum, n, dt, use_host ? 1 : 0, ev, target, state, m)
+    if (n <= 64) SR_EXPOSURE(1, 64);
+    else if (n <= 4096) SR_EXPOSURE(4, m / 4);
+    else SR_EXPOSURE(8, m / 8);
+#undef SR_EXPOSURE
     return hipGetLastError();
 }
 
