@@ -58,7 +58,7 @@ struct FrameArgs {
     uint32_t *tr_start;           // tr_slots
     uint32_t *tr_end;             // tr_slots (cursor, then end)
     uint32_t *tr_list;            // tr_cap record ids
-    unsigned long long *tr_scratch;  // tr_cap: sort room for lists longer than LDS holds
+    unsigned long long *tr_scratch;  // tr_cap x 20 B: sort room for lists longer than LDS holds
     uint32_t tr_cap;
     float4 *center_color;         // 4 (colour, depth) per 64px tile
     int32_t persistent_blocks;    // 0 = one block per item

@@ -2688,153 +2688,394 @@ __device__ __forceinline__ uint32_t z_desc_key(float z) {
     return ~asc;
 }
 
-// Ascending bitonic sort of v[0..P), P a power of two, by the whole workgroup.
-__device__ void bitonic_sort(unsigned long long *v, int P) {
-    for (int k = 2; k <= P; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < P; i += blockDim.x) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    unsigned long long a = v[i], b = v[ixj];
-                    if ((a > b) == ((i & k) == 0)) {
-                        v[i] = b;
-                        v[ixj] = a;
-                    }
-                }
-            }
-            __syncthreads();
-        }
+// ---------------------------------------------------------------------------
+// Workgroup sort in registers: ascending bitonic sort of the first m of
+// blockDim.x * E values, E per thread (value e of a thread is element wave *
+// 64 E + 64 e + lane); m a power of two, and all of them unless E is 1.  Exchanges at a distance below 64
+// are lane exchanges, below 64 E register exchanges; only those between
+// waves go through LDS (sh, one word per element) with barriers.
+// ---------------------------------------------------------------------------
+// Lane l's value from lane l ^ J: a DPP move where the hardware has one, else
+// a swizzle (within 32 lanes) or a permute.
+template <int J> __device__ __forceinline__ int32_t lane_xor(int32_t v) {
+    if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);          // quad_perm 1 0 3 2
+    else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);     // quad_perm 2 3 0 1
+    else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);    // row_ror 8
+    else if constexpr (J < 32) return __builtin_amdgcn_ds_swizzle(v, (J << 10) | 0x1F);       // xor within 32 lanes
+    else return __shfl_xor(v, J, 64);
 }
 
-// Ascending heap sort of v[0..n) by one thread.
-__device__ void heap_sort(unsigned long long *v, int n) {
-    auto sift = [&](int root, int end) {
-        for (;;) {
-            int c = 2 * root + 1;
-            if (c >= end) return;
-            if (c + 1 < end && v[c] < v[c + 1]) c++;
-            if (!(v[root] < v[c])) return;
-            unsigned long long t = v[root];
-            v[root] = v[c];
-            v[c] = t;
-            root = c;
-        }
-    };
-    for (int r = n / 2 - 1; r >= 0; r--) sift(r, n);
-    for (int end = n - 1; end > 0; end--) {
-        unsigned long long t = v[0];
-        v[0] = v[end];
-        v[end] = t;
-        sift(0, end);
+template <int J> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    const uint32_t lo = (uint32_t)lane_xor<J>((int32_t)(uint32_t)v), hi = (uint32_t)lane_xor<J>((int32_t)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+template <int J, class T, int E> __device__ __forceinline__ void sort_lanes(T (&v)[E], uint32_t i0, uint32_t k) {
+    const bool low = (threadIdx.x & J) == 0u;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        T o = lane_xor<J>(v[e]);
+        bool up = ((i0 + 64u * e) & k) == 0u;
+        if ((o < v[e]) == (low == up)) v[e] = o;
     }
 }
 
-// BumpQueue::sort_by (src/bumpqueue.rs:155-200) by one thread: Lomuto
-// quicksort with the rightmost element as pivot, an element moving left when
-// it compares Less, i.e. its z key is below the pivot's (its avg_z above).
-// The two parts of a partition are disjoint, so their order of processing
-// does not change the result: the smaller is sorted first and the larger
-// stacked, which bounds the stack by log2(n) ranges.  Keys in the low 32 bits.
-__device__ void lomuto_sort(unsigned long long *v, int n, int *stack) {
-    int sp = 0, lo = 0, hi = n - 1;
-    for (;;) {
-        while (lo < hi) {
-            uint32_t pivot = (uint32_t)v[hi];
-            int i = lo;
-            for (int j = lo; j < hi; j++) {
-                unsigned long long x = v[j];
-                if ((uint32_t)x < pivot) {
-                    if (i != j) {
-                        v[j] = v[i];
-                        v[i] = x;
-                    }
-                    i++;
-                }
-            }
-            if (i != hi) {
-                unsigned long long t = v[i];
-                v[i] = v[hi];
-                v[hi] = t;
-            }
-            if (i - lo < hi - i) {
-                stack[sp++] = i + 1;
-                stack[sp++] = hi;
-                hi = i - 1;
-            } else {
-                stack[sp++] = lo;
-                stack[sp++] = i - 1;
-                lo = i + 1;
+template <int Q, class T, int E> __device__ __forceinline__ void sort_regs(T (&v)[E], uint32_t i0, uint32_t k) {
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if ((e & Q) == 0 && e + Q < E) {
+            bool up = ((i0 + 64u * e) & k) == 0u;
+            T a = v[e], b = v[e + Q];
+            if ((b < a) == up) {
+                v[e] = b;
+                v[e + Q] = a;
             }
         }
-        if (sp == 0) break;
-        hi = stack[--sp];
-        lo = stack[--sp];
+    }
+}
+
+template <class T, int E> __device__ __forceinline__ void block_sort(T (&v)[E], T *sh, uint32_t m) {
+    static_assert(E == 1 || E == 2 || E == 4 || E == 8, "values per thread");
+    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
+    for (uint32_t k = 2; k <= m; k <<= 1) {
+        for (uint32_t j = k >> 1; j >= 64u * E; j >>= 1) {
+#pragma unroll
+            for (int e = 0; e < E; e++) sh[i0 + 64u * e] = v[e];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                uint32_t i = i0 + 64u * e;
+                T o = sh[i ^ j];
+                bool low = (i & j) == 0u, up = (i & k) == 0u;
+                if ((o < v[e]) == (low == up)) v[e] = o;
+            }
+            __syncthreads();
+        }
+        if (E >= 8 && k >= 512u) sort_regs<4>(v, i0, k);
+        if (E >= 4 && k >= 256u) sort_regs<2>(v, i0, k);
+        if (E >= 2 && k >= 128u) sort_regs<1>(v, i0, k);
+        if (k >= 64u) sort_lanes<32>(v, i0, k);
+        if (k >= 32u) sort_lanes<16>(v, i0, k);
+        if (k >= 16u) sort_lanes<8>(v, i0, k);
+        if (k >= 8u) sort_lanes<4>(v, i0, k);
+        if (k >= 4u) sort_lanes<2>(v, i0, k);
+        sort_lanes<1>(v, i0, k);
     }
 }
 
 // k_tr_sort: one workgroup per 64-px tile orders its list back to front as
-// the reference does.  With no two different triangles on the same key every
-// correct sort gives the reference's order, and a bitonic sort of
-// (z key, id) in LDS is final.  Otherwise Lomuto's result depends on the
-// starting order, which is the canonical submission order (ascending record
-// id, the copies of a wrapped entry adjacent and identical): the list is put
-// in that order and quicksorted as the reference does.  Lists longer than
-// the LDS holds are sorted in global scratch by one thread.
-#define TR_SORT_MAX 4096
-__global__ void __launch_bounds__(256) k_tr_sort(const uint32_t *tr_start, const uint32_t *tr_end, uint32_t *list,
-                                                 uint32_t cap, unsigned long long *scratch, const float4 *raster,
-                                                 TriSource src) {
+// the reference does: BumpQueue::sort_by (src/bumpqueue.rs:155-200), a Lomuto
+// quicksort with the rightmost element as pivot, an element moving left when
+// its z key is below the pivot's (its avg_z above), from the canonical
+// submission order (ascending record id; the copies of a wrapped entry are
+// adjacent and identical).  With no two different triangles on one key every
+// correct sort gives that order, and the sort of (z key, id) is final.
+// Otherwise the elements that share a key with another are taken from a run
+// of the quicksort itself, in which only the ranges that hold such elements
+// are partitioned.
+//
+// A wave partitions a range 64 elements at a time.  Behind the scan the range
+// holds first the elements below the pivot, then (from slot i) the others;
+// each element below the pivot that the scan meets is swapped with the one at
+// slot i, and i advances.  While the scan meets no more of them than there
+// are others queued, their targets all lie before the part being scanned, so
+// their swaps are independent and the lanes do them at once.  A longer run
+// of them moves down as a whole past the queue, which it turns.
+//
+// One lane used to run the whole quicksort, an LDS round trip per comparison:
+// 32 spheres, half of them glass (20,480 translucent triangles) at 1600x900
+// (lists of up to 560, a hundred on equal keys in the worst) took 767 us and
+// take 91: the two sorts 21, the partitions, a chain of LDS round trips, the
+// rest.
+#define TR_SORT_MAX 4096            // lists up to this long are sorted in LDS
+#define TR_SORT_NT 512              // threads: eight waves share the ranges
+static_assert(TR_SORT_MAX == 8 * TR_SORT_NT, "eight values a thread at most");
+
+// Partitions v[lo..hi] (lo < hi); returns the pivot's slot.  Called by a whole
+// wave with uniform arguments.
+template <class V> __device__ __forceinline__ int lomuto_partition(V v, int lo, int hi) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t pivot = (uint32_t)v[hi];
+    int i = lo;
+    for (int j0 = lo; j0 < hi; j0 += 64) {
+        const int c = min(64, hi - j0);
+        unsigned long long x = 0ull;
+        if (lane < c) x = v[j0 + lane];
+        const uint64_t part = c == 64 ? ~0ull : (1ull << c) - 1ull;
+        const uint64_t less = __ballot(lane < c && (uint32_t)x < pivot);
+        int s = 0;
+        while (s < c) {
+            const int queued = j0 + s - i;
+            if (queued == 0) {
+                // the elements below the pivot stay where they are up to the
+                // first other one; that one and those next to it are queued
+                const uint64_t other = ~less & part & (~0ull << s);
+                const int t = other ? __ffsll((unsigned long long)other) - 1 : c;
+                i += t - s;
+                const uint64_t after = t < 64 ? less & (~0ull << t) : 0ull;
+                s = after ? __ffsll((unsigned long long)after) - 1 : c;
+                continue;
+            }
+            const uint64_t rest = less & (~0ull << s);
+            const uint64_t gap = ~less & part & (~0ull << s);
+            const int t = gap ? __ffsll((unsigned long long)gap) - 1 : c;      // end of the run below the pivot
+            if (t - s > queued) {
+                // a run longer than the queue: it moves down by the queue's
+                // length, and the queue, whose front went to its back once
+                // for each of the run, follows it, turned by the run's length
+                unsigned long long y = 0ull;
+                if (lane < queued) y = v[i + lane];
+                wave_lds_sync();
+                if (lane >= s && lane < t) v[j0 + lane - queued] = x;
+                int q = lane - (t - s) % queued;
+                if (q < 0) q += queued;
+                if (lane < queued) v[i + (t - s) + q] = y;
+                wave_lds_sync();
+                i += t - s;
+                s = t;
+                continue;
+            }
+            // up to the (queued + 1)-th element below the pivot
+            const int rank = __popcll(rest & ((1ull << lane) - 1ull));
+            const uint64_t stop = __ballot(((rest >> lane) & 1ull) && rank == queued);
+            const int e = stop ? __ffsll((unsigned long long)stop) - 1 : c;
+            const bool mine = lane < e && ((rest >> lane) & 1ull);
+            unsigned long long y = 0ull;
+            if (mine) y = v[i + rank];
+            wave_lds_sync();
+            if (mine) {
+                v[i + rank] = x;
+                v[j0 + lane] = y;
+            }
+            wave_lds_sync();
+            i += min(queued, __popcll(rest));
+            s = e;
+        }
+    }
+    if (i != hi && lane == 0) {
+        unsigned long long t = v[i];
+        v[i] = v[hi];
+        v[hi] = t;
+    }
+    wave_lds_sync();
+    return i;
+}
+
+// v[lo..hi], all on one key: every step swaps the range's ends (nothing is
+// below the pivot) and goes on behind the first, which in all turns the range
+// by one: its last element first, the others after it in order.
+template <class V> __device__ __forceinline__ void lomuto_rotate(V v, int lo, int hi) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long last = v[hi];
+    for (int e = hi; e > lo; e -= 64) {
+        const int p = e - lane;
+        unsigned long long x = 0ull;
+        if (p > lo) x = v[p - 1];
+        wave_lds_sync();
+        if (p > lo) v[p] = x;
+        wave_lds_sync();
+    }
+    if (lane == 0) v[lo] = last;
+    wave_lds_sync();
+}
+
+// Ranges still to partition, two lists used in turn.
+struct TrRangesLds {                // lists of up to TR_SORT_MAX: 16-bit bounds
+    uint32_t *p;
+    __device__ __forceinline__ void get(int k, int &lo, int &hi) const {
+        lo = (int)(p[k] & 0xFFFFu);
+        hi = (int)(p[k] >> 16);
+    }
+    __device__ __forceinline__ void set(int k, int lo, int hi) const { p[k] = (uint32_t)lo | ((uint32_t)hi << 16); }
+};
+struct TrRangesMem {
+    uint2 *p;
+    __device__ __forceinline__ void get(int k, int &lo, int &hi) const {
+        lo = (int)p[k].x;
+        hi = (int)p[k].y;
+    }
+    __device__ __forceinline__ void set(int k, int lo, int hi) const { p[k] = make_uint2((uint32_t)lo, (uint32_t)hi); }
+};
+
+// Quicksorts v[0..n) as far as it decides the order of equal keys; ties[q]
+// counts, up to sorted position q, the positions whose key equals the one
+// before.  A range holds the keys of its sorted positions, so it holds ties
+// if the count grows over it, and its first element has its key before the
+// range if the count grows there.  cnt: two words.
+template <class V, class C, class R>
+__device__ __forceinline__ void lomuto_ties(V v, int n, const C *ties, R cur, R nxt, int *cnt) {
+    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) {
+        cur.set(0, 0, n - 1);
+        cnt[0] = 1;
+        cnt[1] = 0;
+    }
+    __syncthreads();
+    for (int k = 0;; k ^= 1) {
+        const int c = cnt[k];
+        if (c == 0) break;
+        for (int r = wave; r < c; r += nw) {
+            int lo, hi;
+            cur.get(r, lo, hi);
+            lo = __builtin_amdgcn_readfirstlane(lo);
+            hi = __builtin_amdgcn_readfirstlane(hi);
+            if ((int)ties[hi] - (int)ties[lo] == hi - lo) {
+                lomuto_rotate(v, lo, hi);
+                continue;
+            }
+            const int i = lomuto_partition(v, lo, hi);
+            if (lane < 2) {
+                const int a = lane ? i + 1 : lo, b = lane ? hi : i - 1;
+                if (a < b && (int)ties[b] - (a > 0 ? (int)ties[a - 1] : 0) > 0) nxt.set(atomicAdd(&cnt[k ^ 1], 1), a, b);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) cnt[k] = 0;
+        R t = cur;
+        cur = nxt;
+        nxt = t;
+        __syncthreads();
+    }
+}
+
+// Sorts v[0..n) (n <= 512 E) through registers; sh: exchange room of 512 E
+// values (may be v).
+template <int E, class V> __device__ __forceinline__ void tr_block_sort(V v, unsigned long long *sh, int n, uint32_t m) {
+    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
+    unsigned long long r[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) r[e] = i0 + 64u * e < (uint32_t)n ? v[i0 + 64u * e] : ~0ull;
+    __syncthreads();
+    block_sort(r, sh, m);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        if (i0 + 64u * e < (uint32_t)n) v[i0 + 64u * e] = r[e];
+    __syncthreads();
+}
+
+// Sorts a list of up to TR_SORT_MAX values in LDS: one value a thread, as far
+// as the list reaches, up to 512.
+__device__ __forceinline__ void tr_sort_lds(unsigned long long *sk, int n) {
+    if (n <= TR_SORT_NT) {
+        uint32_t m = 1;
+        while (m < (uint32_t)n) m <<= 1;
+        tr_block_sort<1>(sk, sk, n, m);
+    } else if (n <= 2 * TR_SORT_NT) {
+        tr_block_sort<2>(sk, sk, n, 2 * TR_SORT_NT);
+    } else if (n <= 4 * TR_SORT_NT) {
+        tr_block_sort<4>(sk, sk, n, 4 * TR_SORT_NT);
+    } else {
+        tr_block_sort<8>(sk, sk, n, 8 * TR_SORT_NT);
+    }
+}
+
+// Sorts a longer list in memory: blocks of TR_SORT_MAX sorted through
+// registers and merged by bitonic steps whose comparisons all ascend (so the
+// missing end of the last block needs no padding); each step's exchanges
+// within a block are done by sorting the block again.
+__device__ void tr_sort_mem(unsigned long long *v, int n, unsigned long long *sh) {
+    auto blocks = [&] {
+        for (int b = 0; b < n; b += TR_SORT_MAX) tr_block_sort<8>(v + b, sh, min(n - b, TR_SORT_MAX), TR_SORT_MAX);
+    };
+    auto order = [&](int i, int l) {
+        unsigned long long a = v[i], b = v[l];
+        if (b < a) {
+            v[i] = b;
+            v[l] = a;
+        }
+    };
+    blocks();
+    for (int k = 2 * TR_SORT_MAX; k / 2 < n; k <<= 1) {
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            int l = (i & ~(k - 1)) + (k - 1) - (i & (k - 1));
+            if ((i & (k >> 1)) == 0 && l < n) order(i, l);
+        }
+        __syncthreads();
+        for (int j = k >> 2; j >= TR_SORT_MAX; j >>= 1) {
+            for (int i = threadIdx.x; i < n; i += blockDim.x)
+                if ((i & j) == 0 && i + j < n) order(i, i + j);
+            __syncthreads();
+        }
+        blocks();
+    }
+}
+
+// The list's order from its sorted keys v = (z key << 32 | id): writes the
+// ids, then, if different triangles share a key, reorders those.  sort sorts
+// v[0..n); sh: 17 words for the count's scan, then flags and counters.
+template <class V, class C, class R, class F>
+__device__ __forceinline__ void tr_order(V v, int n, uint32_t *out, C *ties, R cur, R nxt, uint32_t *sh, int *cnt,
+                                         int *serial, F sort) {
+    if (threadIdx.x == 0) *serial = 0;
+    __syncthreads();
+    uint32_t carry = 0u;
+    for (int i0 = 0; i0 < n; i0 += (int)blockDim.x) {
+        const int i = i0 + (int)threadIdx.x;
+        uint32_t tie = 0u;
+        if (i < n) {
+            const unsigned long long x = v[i];
+            out[i] = (uint32_t)x;
+            if (i > 0) {
+                const unsigned long long b = v[i - 1];
+                tie = (b >> 32) == (x >> 32) ? 1u : 0u;
+                if (tie && (uint32_t)b != (uint32_t)x) *serial = 1;
+            }
+        }
+        uint32_t ex;
+        const uint32_t tot = block_excl_scan(tie, ex, sh);
+        if (i < n) ties[i] = (C)(carry + ex + tie);
+        carry += tot;
+    }
+    __syncthreads();
+    if (!*serial) return;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const unsigned long long x = v[i];
+        v[i] = (x << 32) | (x >> 32);           // (id, z key)
+    }
+    __syncthreads();
+    sort();
+    lomuto_ties(v, n, ties, cur, nxt, cnt);
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const bool tied = (i > 0 && ties[i] != ties[i - 1]) || (i + 1 < n && ties[i + 1] != ties[i]);
+        if (tied) out[i] = (uint32_t)(v[i] >> 32);
+    }
+}
+
+// scratch (for lists longer than the LDS holds): cap values, then cap ranges,
+// then cap counts.
+__global__ void __launch_bounds__(TR_SORT_NT) k_tr_sort(const uint32_t *tr_start, const uint32_t *tr_end,
+                                                        uint32_t *list, uint32_t cap, unsigned long long *scratch,
+                                                        const float4 *raster, TriSource src) {
     __shared__ unsigned long long sk[TR_SORT_MAX];
-    __shared__ int stack[2 * 40];
-    __shared__ int serial;
+    __shared__ uint16_t ties[TR_SORT_MAX];
+    __shared__ uint32_t ranges[TR_SORT_MAX];
+    __shared__ uint32_t sh[17];
+    __shared__ int cnt[2], serial;
     uint32_t slot = blockIdx.x;
     uint32_t s = tr_start[slot], e = min(tr_end[slot], cap);
     if (e <= s + 1) return;
-    int n = (int)(e - s);
+    const int n = (int)(e - s);
+    auto key_of = [&](int i) {
+        uint32_t id = list[s + i];
+        return ((unsigned long long)z_desc_key(tri_avg_z(src, raster + 4 * (size_t)id)) << 32) | id;
+    };
     if (n <= TR_SORT_MAX) {
-        int P = 1;
-        while (P < n) P <<= 1;
-        for (int i = threadIdx.x; i < P; i += blockDim.x) {
-            unsigned long long key = ~0ull;
-            if (i < n) {
-                uint32_t id = list[s + i];
-                key = ((unsigned long long)z_desc_key(tri_avg_z(src, raster + 4 * (size_t)id)) << 32) | id;
-            }
-            sk[i] = key;
-        }
-        if (threadIdx.x == 0) serial = 0;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) sk[i] = key_of(i);
         __syncthreads();
-        bitonic_sort(sk, P);
-        for (int i = threadIdx.x; i + 1 < n; i += blockDim.x)
-            if ((sk[i] >> 32) == (sk[i + 1] >> 32) && (uint32_t)sk[i] != (uint32_t)sk[i + 1]) serial = 1;
-        __syncthreads();
-        if (!serial) {
-            for (int i = threadIdx.x; i < n; i += blockDim.x) list[s + i] = (uint32_t)sk[i];
-            return;
-        }
-        for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            unsigned long long x = sk[i];
-            sk[i] = (x << 32) | (x >> 32);          // (id, z key)
-        }
-        __syncthreads();
-        bitonic_sort(sk, P);
-        if (threadIdx.x == 0) lomuto_sort(sk, n, stack);
-        __syncthreads();
-        for (int i = threadIdx.x; i < n; i += blockDim.x) list[s + i] = (uint32_t)(sk[i] >> 32);
+        tr_sort_lds(sk, n);
+        tr_order(sk, n, list + s, ties, TrRangesLds{ranges}, TrRangesLds{ranges + TR_SORT_MAX / 2}, sh, cnt, &serial,
+                 [&] { tr_sort_lds(sk, n); });
         return;
     }
     unsigned long long *v = scratch + s;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        uint32_t id = list[s + i];
-        v[i] = ((unsigned long long)id << 32) | z_desc_key(tri_avg_z(src, raster + 4 * (size_t)id));
-    }
+    uint2 *mr = reinterpret_cast<uint2 *>(scratch + cap) + s;
+    uint32_t *mt = reinterpret_cast<uint32_t *>(scratch + 2 * (size_t)cap) + s;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) v[i] = key_of(i);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        heap_sort(v, n);
-        lomuto_sort(v, n, stack);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) list[s + i] = (uint32_t)(v[i] >> 32);
+    tr_sort_mem(v, n, sk);
+    tr_order(v, n, list + s, mt, TrRangesMem{mr}, TrRangesMem{mr + n / 2}, sh, cnt, &serial,
+             [&] { tr_sort_mem(v, n, sk); });
 }
 
 struct TrArgs {
@@ -3028,76 +3269,6 @@ __global__ void __launch_bounds__(256) k_blit(const float *color, uint64_t plane
         }
         uint32_t v = (sat_u8(c[0] * 255.0f) << 24) | (sat_u8(c[1] * 255.0f) << 16) | (sat_u8(c[2] * 255.0f) << 8) | 0xFFu;
         out[i] = frame_bytes ? __builtin_bswap32(v) : v;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Workgroup sort in registers: ascending bitonic sort of the first m of
-// blockDim.x * E values, E per thread (value e of a thread is element wave *
-// 64 E + 64 e + lane); m a power of two, and all of them unless E is 1.  Exchanges at a distance below 64
-// are lane exchanges, below 64 E register exchanges; only those between
-// waves go through LDS (sh, one word per element) with barriers.
-// ---------------------------------------------------------------------------
-// Lane l's value from lane l ^ J: a DPP move where the hardware has one, else
-// a swizzle (within 32 lanes) or a permute.
-template <int J> __device__ __forceinline__ int32_t lane_xor(int32_t v) {
-    if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);          // quad_perm 1 0 3 2
-    else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);     // quad_perm 2 3 0 1
-    else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);    // row_ror 8
-    else if constexpr (J < 32) return __builtin_amdgcn_ds_swizzle(v, (J << 10) | 0x1F);       // xor within 32 lanes
-    else return __shfl_xor(v, J, 64);
-}
-
-template <int J, class T, int E> __device__ __forceinline__ void sort_lanes(T (&v)[E], uint32_t i0, uint32_t k) {
-    const bool low = (threadIdx.x & J) == 0u;
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        T o = lane_xor<J>(v[e]);
-        bool up = ((i0 + 64u * e) & k) == 0u;
-        if ((o < v[e]) == (low == up)) v[e] = o;
-    }
-}
-
-template <int Q, class T, int E> __device__ __forceinline__ void sort_regs(T (&v)[E], uint32_t i0, uint32_t k) {
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        if ((e & Q) == 0 && e + Q < E) {
-            bool up = ((i0 + 64u * e) & k) == 0u;
-            T a = v[e], b = v[e + Q];
-            if ((b < a) == up) {
-                v[e] = b;
-                v[e + Q] = a;
-            }
-        }
-    }
-}
-
-template <class T, int E> __device__ __forceinline__ void block_sort(T (&v)[E], T *sh, uint32_t m) {
-    static_assert(E == 1 || E == 2 || E == 4 || E == 8, "values per thread");
-    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
-    for (uint32_t k = 2; k <= m; k <<= 1) {
-        for (uint32_t j = k >> 1; j >= 64u * E; j >>= 1) {
-#pragma unroll
-            for (int e = 0; e < E; e++) sh[i0 + 64u * e] = v[e];
-            __syncthreads();
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                uint32_t i = i0 + 64u * e;
-                T o = sh[i ^ j];
-                bool low = (i & j) == 0u, up = (i & k) == 0u;
-                if ((o < v[e]) == (low == up)) v[e] = o;
-            }
-            __syncthreads();
-        }
-        if (E >= 8 && k >= 512u) sort_regs<4>(v, i0, k);
-        if (E >= 4 && k >= 256u) sort_regs<2>(v, i0, k);
-        if (E >= 2 && k >= 128u) sort_regs<1>(v, i0, k);
-        if (k >= 64u) sort_lanes<32>(v, i0, k);
-        if (k >= 32u) sort_lanes<16>(v, i0, k);
-        if (k >= 16u) sort_lanes<8>(v, i0, k);
-        if (k >= 8u) sort_lanes<4>(v, i0, k);
-        if (k >= 4u) sort_lanes<2>(v, i0, k);
-        sort_lanes<1>(v, i0, k);
     }
 }
 
@@ -3384,7 +3555,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_tr_bins, dim3(g), dim3(256), 0, st, a.views, a.rec_geo, a.rec_cap, a.tr_end, a.tr_list,
                            a.tr_cap, a.status);
-        hipLaunchKernelGGL(k_tr_sort, dim3(a.tr_slots), dim3(256), 0, st, a.tr_start, a.tr_end, a.tr_list, a.tr_cap,
+        hipLaunchKernelGGL(k_tr_sort, dim3(a.tr_slots), dim3(TR_SORT_NT), 0, st, a.tr_start, a.tr_end, a.tr_list, a.tr_cap,
                            a.tr_scratch, a.rec_raster, src);
     }
     RasterArgs P;

@@ -332,7 +332,7 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
         if (sort_passes > 1 && (r = pair_vals2.ensure((size_t)pair_cap * 4))) return r;
         if ((r = sort_hist.ensure((size_t)bin_sort_tiles(pair_cap) * 256 * 4))) return r;
         if (has_tr && (r = tr_list.ensure((size_t)tr_cap * 4))) return r;
-        if (has_tr && (r = tr_scratch.ensure((size_t)tr_cap * 8))) return r;
+        if (has_tr && (r = tr_scratch.ensure((size_t)tr_cap * 20))) return r;
         FrameArgs a;
         memset(&a, 0, sizeof(a));
         a.views = (const DevView *)views.ptr;

@@ -31,3 +31,47 @@ def test_device_exposure_tile_counts(sr, scenes, env, tiles):
     host = r.exposure
     r.close()
     assert abs(dev - host) <= 1e-5 * host, (dev, host)
+
+
+def _glass_layers(sr, scenes, n, levels, seed):
+    """n small translucent triangles facing the camera in one 64-px tile, at
+    `levels` distinct depths (few levels: long runs of equal sort keys)."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    c = rng.uniform(-0.8, 0.8, (n, 1, 2))
+    a = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2])
+    xy = c + 0.25 * np.stack([np.cos(a), np.sin(a)], -1)
+    z = -2.0 - 0.5 * rng.permutation(np.arange(n) % levels) / levels
+    pos = np.concatenate([xy, np.broadcast_to(z[:, None, None], (n, 3, 1))], -1).astype(np.float32).reshape(-1, 3)
+    prims, mats, nodes, meshes = [], [], [], []
+    for k, part in enumerate(np.array_split(np.arange(n), min(n, 5))):
+        p = pos.reshape(n, 3, 3)[part].reshape(-1, 3)
+        prims.append({"positions": p, "normals": np.tile(np.float32([0, 0, 1]), (len(p), 1)), "texcoords": None,
+                      "tangents": None, "indices": np.arange(len(p), dtype=np.uint32), "material": k})
+        mats.append({"base_color": tuple(rng.uniform(0.5, 1, 3)) + (1.0,), "metallic": 0.1, "roughness": 0.4,
+                     "is_translucent": 1, "transmission": 0.7})
+        meshes.append((k, 1))
+        nodes.append((np.eye(4, dtype=np.float32), k))
+    return sr.SceneData(prims, meshes, nodes, mats, [], name=f"glass_{n}_{levels}")
+
+
+# the sort's sizes (one, two, four and eight values a thread, in LDS up to
+# 4096, then blocks of 4096 merged in memory), each without and with runs of
+# equal keys, down to one key for all
+@pytest.mark.parametrize("n,levels", [(2, 1), (63, 63), (65, 7), (512, 512), (513, 40), (1025, 1), (2049, 2049),
+                                      (2500, 700), (4096, 3), (4096, 4000), (4097, 4097), (5000, 1), (9001, 2500)])
+def test_translucent_sort_sizes(sr, orc, scenes, env, n, levels):
+    """Lists of 2 to 9001 translucent triangles in one tile blend in the
+    oracle's order: the linear colour, which the order decides, is the
+    oracle's bit for bit."""
+    W = H = 60
+    scene = _glass_layers(sr, scenes, n, levels, n + levels)
+    scene.prepare(env, grid=16)
+    cam = scenes.make_camera(scenes.camera_spec((0, 0, 0), 0.0, 0.0, np.pi / 3, W, H, 20.0))
+    r = sr.Renderer(W, H)
+    r.render_scene(sr.Scene(scene), cam)
+    rgb = r.read_color()
+    r.close()
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()["rgb"]
+    assert np.array_equal(rgb.view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32))
