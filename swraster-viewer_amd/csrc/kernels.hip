@@ -3085,11 +3085,11 @@ struct TrArgs {
     uint32_t cap;
 };
 
-// Staged entry fields for k_translucent (one 256-wide row each).
-enum {
-    G_A = 0, G_B = 3, G_C = 6, G_SX = 9, G_SY = 12,
-    G_OOA = 15, G_OA, G_ODA, G_ODB, G_ZA, G_ZDA, G_ZDB, G_ID, G_ORG, G_LIM, G_COARSE, G_COUNT
-};
+// A staged entry of k_translucent: the entry's edges, depth interpolators,
+// record id and walk limits (TR_ROW float4).  [0] A0 B0 C0 SX0, [1] SY0 A1 B1
+// C1, [2] SX1 SY1 A2 B2, [3] C2 SX2 SY2 ooa, [4] oa oda odb za, [5] zda zdb id
+// origin(ox0 | oy0 << 16), [6] limits(cmxx | cmxy << 16) coarse.
+#define TR_ROW 7
 
 __device__ __forceinline__ int find_view_tile(const RasterArgs &P, uint32_t slot) {
     int lo = 0, hi = P.num_views - 1;
@@ -3101,18 +3101,54 @@ __device__ __forceinline__ int find_view_tile(const RasterArgs &P, uint32_t slot
     return lo;
 }
 
+__device__ __forceinline__ void tr_stage(const TriSetup &ts, uint32_t id, float4 *row) {
+    row[0] = make_float4(ts.A[0], ts.B[0], ts.C[0], ts.SX[0]);
+    row[1] = make_float4(ts.SY[0], ts.A[1], ts.B[1], ts.C[1]);
+    row[2] = make_float4(ts.SX[1], ts.SY[1], ts.A[2], ts.B[2]);
+    row[3] = make_float4(ts.C[2], ts.SX[2], ts.SY[2], ts.ooa);
+    row[4] = make_float4(ts.oa, ts.oda, ts.odb, ts.za);
+    row[5] = make_float4(ts.zda, ts.zdb, __uint_as_float(id),
+                         __uint_as_float((uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16)));
+    row[6] = make_float4(__uint_as_float((uint32_t)ts.cmxx | ((uint32_t)ts.cmxy << 16)),
+                         __uint_as_float(ts.coarse ? 1u : 0u), 0.0f, 0.0f);
+}
+
+__device__ __forceinline__ uint32_t tr_unstage(const float4 *row, TriSetup &ts) {
+    float4 r0 = row[0], r1 = row[1], r2 = row[2], r3 = row[3], r4 = row[4], r5 = row[5], r6 = row[6];
+    ts.A[0] = r0.x; ts.B[0] = r0.y; ts.C[0] = r0.z; ts.SX[0] = r0.w; ts.SY[0] = r1.x;
+    ts.A[1] = r1.y; ts.B[1] = r1.z; ts.C[1] = r1.w; ts.SX[1] = r2.x; ts.SY[1] = r2.y;
+    ts.A[2] = r2.z; ts.B[2] = r2.w; ts.C[2] = r3.x; ts.SX[2] = r3.y; ts.SY[2] = r3.z;
+    ts.ooa = r3.w; ts.oa = r4.x; ts.oda = r4.y; ts.odb = r4.z; ts.za = r4.w; ts.zda = r5.x; ts.zdb = r5.y;
+    uint32_t org = __float_as_uint(r5.w), lim = __float_as_uint(r6.x);
+    ts.ox0 = (int)(org & 0xFFFFu); ts.oy0 = (int)(org >> 16);
+    ts.cmxx = (int)(lim & 0xFFFFu); ts.cmxy = (int)(lim >> 16);
+    ts.coarse = __float_as_uint(r6.y) != 0u;
+    return __float_as_uint(r5.z);
+}
+
 // k_translucent: the forward pass of each 64-px tile's sorted list
 // (src/tilerasterizer.rs:96-101 with TranslucentForwardShader,
 // src/shader.rs:66-76).  Sixteen workgroups per tile, each a 16x16 pixel
-// block with one thread per pixel in 2x2-quad order, walk the list in order:
-// the reference's quad walk and coverage of the entry (the same walk as the
-// opaque pass), the depth test against the opaque depth without writing it,
-// and on passing samples the translucent shader over the current colour.
-// A pixel's colour depends only on its own samples and its quad's
-// barycentrics, so threads never wait on each other.  The block holding the
-// tile's centre quad also updates it (on screen or not) and the tile
-// luminance.
-__device__ __forceinline__ void translucent_block(const RasterArgs &P, const TrArgs &Q, uint32_t *st) {
+// block with one thread per pixel, in four waves of 8x8 pixels in 2x2-quad
+// order.  The workgroup takes 256 list entries at a time and keeps, in order,
+// those whose walk meets its block, set up once each.  A wave then goes over
+// the kept entries that meet its 8x8 pixels, 64 at a time: each entry's
+// coverage (the reference's quad walk, the same as the opaque pass's) and
+// depth test against the opaque depth, which is never written, set one bit of
+// each pixel's mask.  After that every pixel shades its own next entry at
+// once, in list order, until the masks are empty: the translucent shader over
+// the current colour.  A pixel's colour depends only on its own samples and
+// its quad's barycentrics, which it recomputes, so threads never wait on each
+// other.  The block holding the tile's centre quad also updates it (on screen
+// or not) and the tile luminance.
+//
+// Bound by the shading's latency and instructions.  Walking the whole list in
+// every block and shading entry by entry, with only the entry's few pixels
+// active, took 276 us on 32 spheres, half of them glass, at 1600x900 (lists of
+// up to 560 for 64x64 pixels, a few layers deep); this form takes 72.  Three
+// waves per SIMD: two (no spills) 78 us, four (44 registers spilled) 100.
+__device__ __forceinline__ void translucent_block(const RasterArgs &P, const TrArgs &Q, float4 (*rows)[TR_ROW],
+                                                  uint32_t *kept, uint32_t *sh) {
     uint32_t slot = blockIdx.x >> 4, sub = blockIdx.x & 15u;
     uint32_t s = Q.start[slot], e = min(Q.end[slot], Q.cap);
     if (e <= s) return;
@@ -3123,12 +3159,13 @@ __device__ __forceinline__ void translucent_block(const RasterArgs &P, const TrA
     int bx0 = rx0 + 16 * (int)(sub & 3u), by0 = ry0 + 16 * (int)(sub >> 2);
     bool centre_block = sub == 8u;            // holds the quad at (0, 32) of the tile
     if (!(bx0 < V.W && by0 < V.H) && !centre_block) return;
-    const int tid = threadIdx.x, lane = tid & 63, qbase = lane & ~3;
-    const int q = tid >> 2, sl = tid & 3, sx = sl & 1, sy = sl >> 1;
-    const int qpx = bx0 + 2 * (q & 7), qpy = by0 + 2 * (q >> 3);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int q = lane >> 2, sl = lane & 3, sx = sl & 1, sy = sl >> 1;
+    const int wx0 = bx0 + 8 * (wave & 1), wy0 = by0 + 8 * (wave >> 1);
+    const int qpx = wx0 + 2 * (q & 3), qpy = wy0 + 2 * (q >> 2);
     const int px = qpx + sx, py = qpy + sy;
     const bool on_screen = px < V.W && py < V.H;
-    const bool centre = centre_block && q == 0;
+    const bool centre = centre_block && tid < 4;
     const bool valid = on_screen || centre;
     size_t o = V.fb_offset + (size_t)py * (size_t)V.W + (size_t)px;
     float4 *cc = P.center_color + 4 * (size_t)slot + sl;
@@ -3143,91 +3180,86 @@ __device__ __forceinline__ void translucent_block(const RasterArgs &P, const TrA
         depth = P.out_depth[o];
     }
     for (uint32_t b0 = s; b0 < e; b0 += 256u) {
-        uint32_t nb = min(e - b0, 256u);
+        // the entries that meet the block, in order
+        uint32_t id = 0u;
+        bool meets = false;
+        if (b0 + (uint32_t)tid < e) {
+            id = Q.list[b0 + (uint32_t)tid];
+            uint4 g = P.geo[id];
+            int mnx = (int)(g.x & 0xFFFFu), mny = (int)(g.x >> 16), mxx = (int)(g.y & 0xFFFFu), mxy = (int)(g.y >> 16);
+            meets = max(mnx & ~1, bx0) < min(mxx, bx0 + 16) && max(mny & ~1, by0) < min(mxy, by0 + 16);
+        }
+        const uint64_t mm = __ballot(meets);
+        __syncthreads();                      // the previous entries are done with
+        if (lane == 0) sh[wave] = (uint32_t)__popcll(mm);
         __syncthreads();
-        if ((uint32_t)tid < nb) {
-            uint32_t id = Q.list[b0 + (uint32_t)tid];
-            TriSetup ts;
-            tri_setup(P.geo[id], P.raster + 4 * (size_t)id, rx0, ry0, ts);
+        uint32_t at = (uint32_t)__popcll(mm & ((1ull << lane) - 1ull)), nk = 0u;
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                st[(G_A + k) * 256 + tid] = __float_as_uint(ts.A[k]);
-                st[(G_B + k) * 256 + tid] = __float_as_uint(ts.B[k]);
-                st[(G_C + k) * 256 + tid] = __float_as_uint(ts.C[k]);
-                st[(G_SX + k) * 256 + tid] = __float_as_uint(ts.SX[k]);
-                st[(G_SY + k) * 256 + tid] = __float_as_uint(ts.SY[k]);
-            }
-            st[G_OOA * 256 + tid] = __float_as_uint(ts.ooa);
-            st[G_OA * 256 + tid] = __float_as_uint(ts.oa);
-            st[G_ODA * 256 + tid] = __float_as_uint(ts.oda);
-            st[G_ODB * 256 + tid] = __float_as_uint(ts.odb);
-            st[G_ZA * 256 + tid] = __float_as_uint(ts.za);
-            st[G_ZDA * 256 + tid] = __float_as_uint(ts.zda);
-            st[G_ZDB * 256 + tid] = __float_as_uint(ts.zdb);
-            st[G_ID * 256 + tid] = id;
-            st[G_ORG * 256 + tid] = (uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16);
-            st[G_LIM * 256 + tid] = (uint32_t)ts.cmxx | ((uint32_t)ts.cmxy << 16);
-            st[G_COARSE * 256 + tid] = ts.coarse ? 1u : 0u;
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) at += sh[w];
+            nk += sh[w];
+        }
+        if (meets) kept[at] = id;
+        __syncthreads();
+        if ((uint32_t)tid < nk) {
+            TriSetup ts;
+            id = kept[tid];
+            tri_setup(P.geo[id], P.raster + 4 * (size_t)id, rx0, ry0, ts);
+            tr_stage(ts, id, rows[tid]);
         }
         __syncthreads();
-        for (uint32_t k = 0; k < nb; k++) {
-#define GF(f) __uint_as_float(st[(f) * 256 + k])
-            uint32_t org = st[G_ORG * 256 + k], lim = st[G_LIM * 256 + k];
-            int ox0 = (int)(org & 0xFFFFu), oy0 = (int)(org >> 16), cmxx = (int)(lim & 0xFFFFu), cmxy = (int)(lim >> 16);
-            if (!(max(ox0, bx0) < min(cmxx, bx0 + 16) && max(oy0, by0) < min(cmxy, by0 + 16))) continue;
-            bool fm = false;
-            float b1 = 0.0f, b2 = 0.0f;
-            if (qpx >= ox0 && qpx < cmxx && qpy >= oy0 && qpy < cmxy) {
-                TriSetup ts;
-#pragma unroll
-                for (int m = 0; m < 3; m++) {
-                    ts.A[m] = GF(G_A + m);
-                    ts.B[m] = GF(G_B + m);
-                    ts.C[m] = GF(G_C + m);
-                    ts.SX[m] = GF(G_SX + m);
-                    ts.SY[m] = GF(G_SY + m);
-                }
-                bool coarse = st[G_COARSE * 256 + k] != 0u;
-                int bx = ox0, by = oy0;
-                if (coarse) {
-                    bx = ox0 + ((qpx - ox0) & ~15);
-                    by = oy0 + ((qpy - oy0) & ~15);
-                }
-                if (!(coarse && block_out(ts, bx, by))) {
-                    int i = (qpx - bx) >> 1, j = (qpy - by) >> 1;
-                    float w0 = edge_chain(ts, 0, bx, by, sx, sy, i, j);
-                    float w1 = edge_chain(ts, 1, bx, by, sx, sy, i, j);
-                    float w2 = edge_chain(ts, 2, bx, by, sx, sy, i, j);
-                    float ooa = GF(G_OOA);
-                    b1 = w1 * ooa;
-                    b2 = w2 * ooa;
-                    float wv = 1.0f / ((GF(G_OA) + b1 * GF(G_ODA)) + b2 * GF(G_ODB));
-                    float z = ((GF(G_ZA) + b1 * GF(G_ZDA)) + b2 * GF(G_ZDB)) * wv;
-                    fm = valid && w0 >= 0.0f && w1 >= 0.0f && w2 >= 0.0f && z <= depth;
-                }
+        for (uint32_t k0 = 0; k0 < nk; k0 += 64u) {
+            bool mine = false;
+            if (k0 + (uint32_t)lane < nk) {
+                const float4 *row = rows[k0 + (uint32_t)lane];
+                uint32_t org = __float_as_uint(row[5].w), lim = __float_as_uint(row[6].x);
+                mine = max((int)(org & 0xFFFFu), wx0) < min((int)(lim & 0xFFFFu), wx0 + 8) &&
+                       max((int)(org >> 16), wy0) < min((int)(lim >> 16), wy0 + 8);
             }
-#undef GF
-            if (__ballot(fm)) {
-                float qb1[4], qb2[4];
+            uint64_t todo = __ballot(mine), pass = 0ull;
+            while (todo) {
+                const int k = __ffsll((unsigned long long)todo) - 1;
+                todo &= todo - 1ull;
+                TriSetup ts;
+                tr_unstage(rows[k0 + (uint32_t)k], ts);
+                int bx, by;
+                if (!quad_origin(ts, qpx, qpy, bx, by) || (ts.coarse && block_out(ts, bx, by))) continue;
+                int i = (qpx - bx) >> 1, j = (qpy - by) >> 1;
+                float w0 = edge_chain(ts, 0, bx, by, sx, sy, i, j);
+                float w1 = edge_chain(ts, 1, bx, by, sx, sy, i, j);
+                float w2 = edge_chain(ts, 2, bx, by, sx, sy, i, j);
+                if (!(valid && w0 >= 0.0f && w1 >= 0.0f && w2 >= 0.0f)) continue;
+                float b1 = w1 * ts.ooa, b2 = w2 * ts.ooa;
+                float wv = 1.0f / ((ts.oa + b1 * ts.oda) + b2 * ts.odb);
+                float z = ((ts.za + b1 * ts.zda) + b2 * ts.zdb) * wv;
+                if (z <= depth) pass |= 1ull << k;
+            }
+            while (pass) {
+                const int k = __ffsll((unsigned long long)pass) - 1;
+                pass &= pass - 1ull;
+                TriSetup ts;
+                id = tr_unstage(rows[k0 + (uint32_t)k], ts);
+                int bx, by;
+                quad_origin(ts, qpx, qpy, bx, by);
+                int i = (qpx - bx) >> 1, j = (qpy - by) >> 1;
+                float qb1[4], qb2[4], wv[4], b1 = 0.0f, b2 = 0.0f;
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
-                    qb1[m] = __shfl(b1, qbase + m, 64);
-                    qb2[m] = __shfl(b2, qbase + m, 64);
+                    qb1[m] = edge_chain(ts, 1, bx, by, m & 1, m >> 1, i, j) * ts.ooa;
+                    qb2[m] = edge_chain(ts, 2, bx, by, m & 1, m >> 1, i, j) * ts.ooa;
+                    if (m == sl) {
+                        b1 = qb1[m];
+                        b2 = qb2[m];
+                    }
                 }
-                if (fm) {
-                    uint32_t id = st[G_ID * 256 + k];
-                    const float4 *R = P.raster + 4 * (size_t)id;
-                    CV tv[3];
-                    float4 Sh[7], Tn[3];
-                    load_tri_cv(P.src, R, tv);
-                    bool nmap = (P.geo[id].z & SR_GEO_NORMAL_MAP) != 0;
-                    tri_shade_attrs(tv, R, nmap, Sh, Tn);
-                    float wv[4];
-                    quad_w(__uint_as_float(st[G_OA * 256 + k]), __uint_as_float(st[G_ODA * 256 + k]),
-                           __uint_as_float(st[G_ODB * 256 + k]), qb1, qb2, wv);
-                    cur = shade_pixel<true>(S, V, __float_as_int(R[3].y), Sh, Tn, nmap, qb1[sl], qb2[sl], wv, sl,
-                                            cur);
-                }
+                quad_w(ts.oa, ts.oda, ts.odb, qb1, qb2, wv);
+                const float4 *R = P.raster + 4 * (size_t)id;
+                CV tv[3];
+                float4 Sh[7], Tn[3];
+                load_tri_cv(P.src, R, tv);
+                bool nmap = (P.geo[id].z & SR_GEO_NORMAL_MAP) != 0;
+                tri_shade_attrs(tv, R, nmap, Sh, Tn);
+                cur = shade_pixel<true>(S, V, __float_as_int(R[3].y), Sh, Tn, nmap, b1, b2, wv, sl, cur);
             }
         }
     }
@@ -3239,14 +3271,15 @@ __device__ __forceinline__ void translucent_block(const RasterArgs &P, const TrA
     if (centre) *cc = make_float4(cur.x, cur.y, cur.z, depth);
     // centre-quad luminance after the translucent pass (src/tilerasterizer.rs:103-106)
     float lum = (cur.x * 0.2126f + cur.y * 0.7152f) + cur.z * 0.0722f;
-    float l0 = __shfl(lum, qbase, 64), l1 = __shfl(lum, qbase + 1, 64);
-    float l2 = __shfl(lum, qbase + 2, 64), l3 = __shfl(lum, qbase + 3, 64);
+    float l0 = quad_lane<0>(lum), l1 = quad_lane<1>(lum), l2 = quad_lane<2>(lum), l3 = quad_lane<3>(lum);
     if (centre && sl == 0) P.out_lum[slot] = (((l0 + l1) + l2) + l3) * 0.25f;
 }
 
-__global__ void __launch_bounds__(256) k_translucent(RasterArgs P, TrArgs Q) {
-    __shared__ uint32_t st[G_COUNT * 256];
-    translucent_block(P, Q, st);
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_translucent(RasterArgs P, TrArgs Q) {
+    __shared__ float4 rows[256][TR_ROW];
+    __shared__ uint32_t kept[256];
+    __shared__ uint32_t sh[4];
+    translucent_block(P, Q, rows, kept, sh);
     clock_end(P.clock, CLOCK_TR_END);
 }
 

@@ -75,3 +75,40 @@ def test_translucent_sort_sizes(sr, orc, scenes, env, n, levels):
     o.render_scene(orc.OracleScene(scene), cam)
     want = o.read_frame()["rgb"]
     assert np.array_equal(rgb.view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("size", [(16, 16), (63, 65), (130, 97)])
+def test_translucent_walk_edges(sr, orc, scenes, env, size):
+    """The forward pass keeps only the entries that meet each 16x16 block
+    and masks them per pixel 64 at a time: 300 triangles from a few pixels
+    to the whole view (kept counts below and above 64 and 256), partly off
+    screen, some behind an opaque triangle, over blocks cut by the view's
+    edges.  The linear colour and the tiles' luminance are the oracle's bit
+    for bit."""
+    W, H = size
+    rng = np.random.Generator(np.random.PCG64(W))
+    scene = _glass_layers(sr, scenes, 300, 300, 11)
+    for k, prim in enumerate(scene.primitives):
+        p = prim["positions"].reshape(-1, 3, 3)
+        mid = p.mean(1, keepdims=True)
+        p[:] = mid + (p - mid) * np.exp(rng.uniform(np.log(0.2), np.log(12.0), (len(p), 1, 1))) * \
+            np.array([1.0, 1.0, 0.0], np.float32)
+    quad = np.array([[-0.5, -2, -2.3], [2, -2, -2.3], [2, 2, -2.3]], np.float32)
+    scene.primitives.append({"positions": quad, "normals": np.tile(np.float32([0, 0, 1]), (3, 1)), "texcoords": None,
+                             "tangents": None, "indices": np.arange(3, dtype=np.uint32),
+                             "material": len(scene.materials)})
+    scene.materials.append({"base_color": (0.4, 0.5, 0.6, 1.0), "metallic": 0.0, "roughness": 0.6})
+    scene.meshes.append((len(scene.primitives) - 1, 1))
+    scene.nodes.append((np.eye(4, dtype=np.float32), len(scene.meshes) - 1))
+    scene.rebuild()
+    scene.prepare(env, grid=16)
+    cam = scenes.make_camera(scenes.camera_spec((0, 0, 0), 0.0, 0.0, np.pi / 3, W, H, 20.0))
+    r = sr.Renderer(W, H)
+    r.render_scene(sr.Scene(scene), cam)
+    rgb, lum = r.read_color(), r.read_tile_luminance()
+    r.close()
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()["rgb"]
+    assert np.array_equal(rgb.view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32))
+    assert np.array_equal(lum.view(np.uint32), np.asarray(o.tile_luminance(), np.float32).view(np.uint32))
