@@ -138,7 +138,6 @@ struct DevStatus {
     uint32_t total_pairs;         // binned (triangle, tile) pairs
     uint32_t overflow_records;
     uint32_t overflow_pairs;
-    uint32_t work_counter;        // persistent-kernel queue head
     uint32_t clip_queued;         // triangles queued for clipping
     uint32_t overflow_clip;
     uint32_t clip_overflow;       // a clipped polygon outgrew its room (frame fails)
@@ -147,15 +146,22 @@ struct DevStatus {
     uint32_t seq;                 // the frame's number, set by the host in the upload
 };
 
+// A queue head of the persistent raster, in a cache line of its own.
+#define WORK_COUNTERS 64u
+struct WorkCounter {
+    uint32_t next, pad[31];
+};
+
 // Working state of the stable binning (radix passes over the bin index),
 // right after the status (every field is written in the frame before it is
 // read): each pass's element count per digit (its row scan writes them, its
-// scatter scans them into the digits' first positions) and the expansion's
-// total.
+// scatter scans them into the digits' first positions), the expansion's
+// total, and the persistent raster's queues.
 struct BinSortState {
     uint32_t digit_total[3][256];
     uint32_t chunk_total;         // pairs of all records (the expansion's size)
     uint32_t pad[3];
+    WorkCounter work[WORK_COUNTERS];    // zeroed by the frame's first kernel
 };
 
 // Stage boundaries of one frame on the GPU's constant-rate wall clock

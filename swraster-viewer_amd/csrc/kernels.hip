@@ -193,8 +193,8 @@ __device__ __forceinline__ int clip_classify(const float c[3][4]) {
     return -1;
 }
 
-// Clears the tiles' list bounds over the whole grid, in k_front (or in
-// k_frame_begin when there are no vertices); the frame's status is cleared
+// Clears the tiles' list bounds and the work counters over the whole grid, in
+// k_front (or in k_frame_begin when there are no vertices); the frame's status is cleared
 // by the upload that precedes the first kernel.
 // Stage stamps on the wall clock (StageClock): the kernel's first workgroup
 // stamps its start (workgroups are dispatched in index order).
@@ -218,6 +218,7 @@ struct FrameBegin {
     uint32_t *bin_start, *bin_end, *tr_count;
     uint32_t items, tr_slots;
     StageClock *clock;
+    WorkCounter *work;            // the persistent raster's queues (null: none)
 };
 
 __device__ __forceinline__ void frame_begin(const FrameBegin &F) {
@@ -229,6 +230,8 @@ __device__ __forceinline__ void frame_begin(const FrameBegin &F) {
     }
     if (F.clock)
         for (uint32_t k = i; k < CLOCK_ENDS * CLOCK_SPREAD; k += gridDim.x * blockDim.x) (&F.clock->end[0][0])[k] = 0ull;
+    if (F.work)
+        for (uint32_t k = i; k < WORK_COUNTERS; k += gridDim.x * blockDim.x) F.work[k].next = 0u;
     if (F.tr_count)
         for (uint32_t k = i; k < F.tr_slots; k += gridDim.x * blockDim.x) F.tr_count[k] = 0u;
 }
@@ -1873,6 +1876,7 @@ struct RasterArgs {
     DevStatus *status_out;                  // pinned host memory for the frame's status
     StageClock *clock;                      // stage stamps (or null)
     int32_t persistent;
+    WorkCounter *work;                      // the persistent raster's queues
 };
 
 __device__ __forceinline__ uint32_t depth_key(float z) {
@@ -2219,7 +2223,10 @@ __device__ __forceinline__ uint32_t xcd_item(uint32_t b) {
     return ((k / XCD_RUN) * 8u + x) * XCD_RUN + (k % XCD_RUN);
 }
 
-static inline uint32_t xcd_grid(uint32_t items) { return (items + 8u * XCD_RUN - 1) / (8u * XCD_RUN) * (8u * XCD_RUN); }
+// Positions b that xcd_item maps onto the items (and a few past the last).
+__host__ __device__ static inline uint32_t xcd_positions(uint32_t items) {
+    return (items + 8u * XCD_RUN - 1) / (8u * XCD_RUN) * (8u * XCD_RUN);
+}
 
 template <int T, int NT, bool HIZ>
 __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long long *keys, uint32_t *stage) {
@@ -2327,13 +2334,25 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
         const uint32_t item = xcd_item(blockIdx.x);
         if (item < P.total_items) raster_item<T, NT, HIZ>(P, item, keys, stage);
     } else {
-        for (;;) {
-            if (threadIdx.x == 0) next = atomicAdd(&P.status->work_counter, 1u);
+        // Every workgroup starts at its own position; the rest are drained
+        // from counters, each shared by the workgroups of one residue of the
+        // index (and so of one XCD), and the next position is asked for
+        // before the item it follows.  Atomics on one address are served
+        // one after the other, 33 ns each across the chip: with one counter
+        // for all, 64 views of 160x120 to 320x240 (11k items, 2048
+        // workgroups) took 434 us, like this 63 (one workgroup per item: 58).  Below
+        // 8 workgroups a counter there is one.
+        const uint32_t total = xcd_positions(P.total_items), nb = gridDim.x;
+        const uint32_t groups = nb >= 8u * WORK_COUNTERS ? WORK_COUNTERS : 1u, g = blockIdx.x % groups;
+        const uint32_t first = (nb - g + groups - 1u) / groups;      // the group's workgroups
+        for (uint32_t pos = blockIdx.x; pos < total;) {
+            uint32_t got = 0u;
+            if (threadIdx.x == 0) got = atomicAdd(&P.work[g].next, 1u);
+            const uint32_t item = xcd_item(pos);
+            if (item < P.total_items) raster_item<T, NT, HIZ>(P, item, keys, stage);
+            if (threadIdx.x == 0) next = g + groups * (first + got);
             __syncthreads();
-            uint32_t item = next;
-            __syncthreads();
-            if (item >= P.total_items) break;
-            raster_item<T, NT, HIZ>(P, item, keys, stage);
+            pos = next;
             __syncthreads();
         }
     }
@@ -3486,6 +3505,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     fb.tr_count = a.has_translucent ? a.tr_count : nullptr;
     fb.tr_slots = a.tr_slots;
     fb.clock = a.clock;
+    fb.work = a.persistent_blocks > 0 ? a.sort->work : nullptr;
     uint32_t tri_blocks = a.total_in > 0 ? grid_for(a.total_in, 256, GRID_CAP) : 0u;
     uint32_t vtx_blocks = a.total_xv > 0 ? grid_for(a.total_xv, 256, GRID_CAP) : 0u;
     hipEvent_t ev_none = nullptr;
@@ -3634,7 +3654,8 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     P.center_ids = (SR_GLOBAL uint32_t *)a.center_ids;
     P.center_color = (SR_GLOBAL float4 *)(a.has_translucent ? a.center_color : nullptr);
     P.persistent = a.persistent_blocks > 0;
-    uint32_t grid = P.persistent ? (uint32_t)a.persistent_blocks : xcd_grid(a.total_items);
+    P.work = a.sort->work;
+    uint32_t grid = P.persistent ? (uint32_t)a.persistent_blocks : xcd_positions(a.total_items);
     // stage events: bins done = the raster's start, the raster's end, and
     // the frame's end = the shading's end (or the translucent pass's)
     hipEvent_t e2 = a.events[2], e4 = a.events[4], e3 = a.has_translucent ? ev_none : a.events[3];
@@ -3647,12 +3668,12 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
             break;
     }
     switch (a.tile_size) {
-        case 8: SR_LAUNCH_TIMED(ev_none, e3, (k_shade<8, 64>), dim3(xcd_grid(a.total_items)), dim3(64), st, P); break;
+        case 8: SR_LAUNCH_TIMED(ev_none, e3, (k_shade<8, 64>), dim3(xcd_positions(a.total_items)), dim3(64), st, P); break;
         case 32:
-            SR_LAUNCH_TIMED(ev_none, e3, (k_shade<32, 1024>), dim3(xcd_grid(a.total_items)), dim3(1024), st, P);
+            SR_LAUNCH_TIMED(ev_none, e3, (k_shade<32, 1024>), dim3(xcd_positions(a.total_items)), dim3(1024), st, P);
             break;
         default:
-            SR_LAUNCH_TIMED(ev_none, e3, (k_shade<16, 256>), dim3(xcd_grid(a.total_items)), dim3(256), st, P);
+            SR_LAUNCH_TIMED(ev_none, e3, (k_shade<16, 256>), dim3(xcd_positions(a.total_items)), dim3(256), st, P);
             break;
     }
     if (a.has_translucent) {

@@ -112,3 +112,28 @@ def test_translucent_walk_edges(sr, orc, scenes, env, size):
     want = o.read_frame()["rgb"]
     assert np.array_equal(rgb.view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32))
     assert np.array_equal(lum.view(np.uint32), np.asarray(o.tile_luminance(), np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("blocks", [1, 3, 8, 64, 100, 4096])
+def test_persistent_raster_block_counts(sr, scenes, env, blocks):
+    """Persistent raster workgroups below, at and above the item count (one
+    workgroup for all items, counts that do not divide them, more workgroups
+    than items): every view equals the batch with one workgroup per item."""
+    scene, spec = scenes.make_c1(width=160, height=90, spheres=6, subdiv=2)
+    scene.prepare(env, grid=16)
+    gscene = sr.Scene(scene)
+    views = []
+    for k, (w, h) in enumerate(((160, 90), (1, 1), (65, 130), (96, 64))):
+        s = dict(spec)
+        s["yaw"] = 0.05 * k
+        views.append((gscene, scenes.make_camera(s, w, h), w, h, 0.0))
+    b = sr.Batch()
+    out = []
+    for persistent in (-1, blocks):
+        b.configure(persistent_blocks=persistent)
+        b.render(views)
+        out.append([(*b.read_vbuffer(i), b.read_pixels(i)) for i in range(len(views))])
+    b.close()
+    for want, got in zip(*out):
+        for x, y in zip(want, got):
+            assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
