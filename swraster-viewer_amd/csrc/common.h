@@ -38,7 +38,10 @@
 #define SR_DRAW_OPAQUE 2u
 #define SR_DRAW_TANGENTS 4u
 
-// record geo flags (rec_geo.z)
+// record geometry (rec_geo): x, y the pixel box (x | y << 16 each); z flags
+// and, from SR_GEO_VIEW_SHIFT, the view; w a depth key that no fragment goes
+// below (0: none)
+#define SR_GEO_VIEW_SHIFT 8
 #define SR_GEO_EMPTY 1u          // culled or empty bounding box: no bins
 #define SR_GEO_ALPHA 2u          // alpha-tested material
 #define SR_GEO_NORMAL_MAP 4u

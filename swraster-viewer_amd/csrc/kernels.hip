@@ -835,6 +835,38 @@ __device__ __forceinline__ bool small_tri_uncovered(const int32_t px[3], const i
     return !covered;
 }
 
+// Orderable depth bits: unsigned comparison is the depth's (-0 == +0).
+__device__ __forceinline__ uint32_t depth_key(float z) {
+    if (z == 0.0f) z = 0.0f;  // -0 == +0
+    uint32_t b = __float_as_uint(z);
+    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+
+// A depth key no fragment of the triangle goes below, or 0 (no bound), from
+// its vertices' z/w (1/w) and 1/w.  The depth ((za + b1 zda) + b2 zdb) / ((oa
+// + b1 oda) + b2 odb) is a ratio of affine functions of the barycentrics, so
+// over the triangle it lies between its values at the vertices when the
+// denominator keeps its sign.  Covered samples have b1, b2 >= 0 and b1 + b2 <=
+// 1 to within 4e-7 (the edge values and 1/area rounded once each) and are
+// evaluated to a few ulps, as are the quotients here (hardware reciprocal);
+// with the vertices' denominators within a factor 16 of each other the
+// depth's derivative in b is below 48 times the largest vertex depth, so a
+// margin of 1e-4 of that depth covers all of it with room to spare.
+__device__ __forceinline__ uint32_t tri_zmin_key(const float zow[3], const float oow[3]) {
+    float dmin = fminf(oow[0], fminf(oow[1], oow[2])), dmax = fmaxf(oow[0], fmaxf(oow[1], oow[2]));
+    if (!(dmin > 1e-30f) || !(dmax <= 16.0f * dmin)) return 0u;
+    float z0 = zow[0] * __builtin_amdgcn_rcpf(oow[0]), z1 = zow[1] * __builtin_amdgcn_rcpf(oow[1]);
+    float z2 = zow[2] * __builtin_amdgcn_rcpf(oow[2]);
+    float zabs = fmaxf(fabsf(z0), fmaxf(fabsf(z1), fabsf(z2)));
+    float lo = fminf(z0, fminf(z1, z2)) - (zabs * 1e-4f + 1e-30f);
+    if (!(z0 == z0 && z1 == z1 && z2 == z2) || !(zabs < 1e30f)) return 0u;
+    return depth_key(lo);
+}
+
+// A record's third geometry word: SR_GEO_* flags and the view.
+__device__ __forceinline__ uint32_t geo_word(uint32_t flags, int view) { return flags | ((uint32_t)view << SR_GEO_VIEW_SHIFT); }
+__device__ __forceinline__ int geo_view(uint4 g) { return (int)(g.z >> SR_GEO_VIEW_SHIFT); }
+
 // Snap, cull, bbox and setup of one (post-clip) triangle (bin_triangle,
 // src/renderer.rs:668-831).  Writes the geometry and raster records and
 // returns the bin rectangle (empty when culled, when the box is empty, or
@@ -855,7 +887,7 @@ __device__ Rect emit_triangle(const DevView &V, int view, const SnapV sv[3], uin
     int32_t px[3] = {sv[0].px, sv[1].px, sv[2].px}, py[3] = {sv[0].py, sv[1].py, sv[2].py};
     int32_t area = wsub(wmul(wsub(px[1], px[0]), wsub(py[2], py[0])), wmul(wsub(px[2], px[0]), wsub(py[1], py[0])));
     if (area > 0) {
-        O.geo[id] = make_uint4(0u, 0u, SR_GEO_EMPTY, (uint32_t)view);
+        O.geo[id] = make_uint4(0u, 0u, geo_word(SR_GEO_EMPTY, view), 0u);
         return none;
     }
     int32_t mnx = max(min(min(px[0], px[1]), px[2]), 0);
@@ -865,7 +897,7 @@ __device__ Rect emit_triangle(const DevView &V, int view, const SnapV sv[3], uin
     int32_t pmnx = mnx >> 4, pmny = mny >> 4;
     int32_t pmxx = wadd(mxx, 16) >> 4, pmxy = wadd(mxy, 16) >> 4;
     if (!(pmnx < pmxx && pmny < pmxy) || (!translucent && small_tri_uncovered(px, py, pmnx, pmny, pmxx, pmxy))) {
-        O.geo[id] = make_uint4(0u, 0u, SR_GEO_EMPTY, (uint32_t)view);
+        O.geo[id] = make_uint4(0u, 0u, geo_word(SR_GEO_EMPTY, view), 0u);
         return none;
     }
     float ooa = 1.0f / (float)wabs(area);
@@ -874,8 +906,8 @@ __device__ Rect emit_triangle(const DevView &V, int view, const SnapV sv[3], uin
     if (matflags & SR_MAT_ALPHA_TESTED) flags |= SR_GEO_ALPHA;
     if (matflags & SR_MAT_NORMAL_MAP) flags |= SR_GEO_NORMAL_MAP;
     if (translucent) flags |= SR_GEO_TRANSLUCENT;
-    O.geo[id] = make_uint4((uint32_t)pmnx | ((uint32_t)pmny << 16), (uint32_t)pmxx | ((uint32_t)pmxy << 16), flags,
-                           (uint32_t)view);
+    O.geo[id] = make_uint4((uint32_t)pmnx | ((uint32_t)pmny << 16), (uint32_t)pmxx | ((uint32_t)pmxy << 16),
+                           geo_word(flags, view), tri_zmin_key(zow, oow));
     float4 *R = O.raster + 4 * (size_t)id;
     R[0] = make_float4(__int_as_float(px[0]), __int_as_float(py[0]), __int_as_float(px[1]), __int_as_float(py[1]));
     R[1] = make_float4(__int_as_float(px[2]), __int_as_float(py[2]), ooa, oow[0]);
@@ -1196,7 +1228,7 @@ __global__ void __launch_bounds__(256) k_bin_expand(BinPass P) {
             int view = 0;
             if (id < last) {
                 uint4 g = P.geo[id];
-                view = (int)g.w;
+                view = geo_view(g);
                 if (!(g.z & (SR_GEO_EMPTY | SR_GEO_TRANSLUCENT))) {
                     int mnx = (int)(g.x & 0xFFFFu), mny = (int)(g.x >> 16), mxx = (int)(g.y & 0xFFFFu), mxy = (int)(g.y >> 16);
                     r = bin_rect(P.views[view], mnx, mny, mxx, mxy, P.T);
@@ -1879,12 +1911,6 @@ struct RasterArgs {
     WorkCounter *work;                      // the persistent raster's queues
 };
 
-__device__ __forceinline__ uint32_t depth_key(float z) {
-    if (z == 0.0f) z = 0.0f;  // -0 == +0
-    uint32_t b = __float_as_uint(z);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
 __device__ __forceinline__ bool alpha_pass(const DevScene &S, const TriSource &T, const float4 *R, float b1, float b2,
                                            float w) {
     int material = __float_as_int(R[3].y);
@@ -2171,27 +2197,6 @@ __device__ __forceinline__ void walk_quad(const DevScene &S, const RasterArgs &P
 #undef SF
 }
 
-// A depth key no fragment of the triangle goes below, or 0 (no bound).  The
-// depth ((za + b1 zda) + b2 zdb) / ((oa + b1 oda) + b2 odb) is a ratio of
-// affine functions of the barycentrics, so over the triangle it lies between
-// its values at the vertices when the denominator keeps its sign.  Covered
-// samples have b1, b2 >= 0 and b1 + b2 <= 1 to within 4e-7 (the edge values
-// and 1/area rounded once each) and are evaluated to a few ulps; with the
-// vertices' denominators within a factor 16 of each other the depth's
-// derivative in b is below 48 times the largest vertex depth, so a margin of
-// 1e-4 of that depth covers both with room to spare.
-__device__ __forceinline__ uint32_t tri_zmin_key(float za, float zda, float zdb, float oa, float oda, float odb) {
-    float d0 = oa, d1 = oa + oda, d2 = oa + odb;
-    float dmin = fminf(d0, fminf(d1, d2)), dmax = fmaxf(d0, fmaxf(d1, d2));
-    if (!(dmin > 0.0f) || !(dmax <= 16.0f * dmin)) return 0u;
-    float z0 = za / d0, z1 = (za + zda) / d1, z2 = (za + zdb) / d2;
-    float zmin = fminf(z0, fminf(z1, z2));
-    float zabs = fmaxf(fabsf(z0), fmaxf(fabsf(z1), fabsf(z2)));
-    float lo = zmin - (zabs * 1e-4f + 1e-30f);
-    if (!(lo == lo) || !(zabs < 1e30f)) return 0u;
-    return depth_key(lo);
-}
-
 __device__ __forceinline__ int find_view(const RasterArgs &P, uint32_t item) {
     int lo = 0, hi = P.num_views - 1;
     while (lo < hi) {
@@ -2205,6 +2210,104 @@ __device__ __forceinline__ int find_view(const RasterArgs &P, uint32_t item) {
 // The 2x2 quad at the origin of a tile whose origin is (64k, 64m + 32) is the
 // centre quad of its 64px reference tile (src/tilerasterizer.rs:103-106).
 __device__ __forceinline__ bool centre_tile(int tx0, int ty0) { return ((tx0 & 63) == 0) && ((ty0 & 63) == 32); }
+
+// ---------------------------------------------------------------------------
+// Workgroup sort in registers: ascending bitonic sort of the first m of
+// blockDim.x * E values, E per thread (value e of a thread is element wave *
+// 64 E + 64 e + lane); m a power of two, and all of them unless E is 1.  Exchanges at a distance below 64
+// are lane exchanges, below 64 E register exchanges; only those between
+// waves go through LDS (sh, one word per element) with barriers.
+// ---------------------------------------------------------------------------
+// Lane l's value from lane l ^ J: a DPP move where the hardware has one, else
+// a swizzle (within 32 lanes) or a permute.
+template <int J> __device__ __forceinline__ int32_t lane_xor(int32_t v) {
+    if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);          // quad_perm 1 0 3 2
+    else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);     // quad_perm 2 3 0 1
+    else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);    // row_ror 8
+    else if constexpr (J < 32) return __builtin_amdgcn_ds_swizzle(v, (J << 10) | 0x1F);       // xor within 32 lanes
+    else return __shfl_xor(v, J, 64);
+}
+
+template <int J> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) { return (uint32_t)lane_xor<J>((int32_t)v); }
+template <int J> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    const uint32_t lo = (uint32_t)lane_xor<J>((int32_t)(uint32_t)v), hi = (uint32_t)lane_xor<J>((int32_t)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+template <int J, class T, int E> __device__ __forceinline__ void sort_lanes(T (&v)[E], uint32_t i0, uint32_t k) {
+    const bool low = (threadIdx.x & J) == 0u;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        T o = lane_xor<J>(v[e]);
+        bool up = ((i0 + 64u * e) & k) == 0u;
+        if ((o < v[e]) == (low == up)) v[e] = o;
+    }
+}
+
+template <int Q, class T, int E> __device__ __forceinline__ void sort_regs(T (&v)[E], uint32_t i0, uint32_t k) {
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if ((e & Q) == 0 && e + Q < E) {
+            bool up = ((i0 + 64u * e) & k) == 0u;
+            T a = v[e], b = v[e + Q];
+            if ((b < a) == up) {
+                v[e] = b;
+                v[e + Q] = a;
+            }
+        }
+    }
+}
+
+template <class T, int E> __device__ __forceinline__ void block_sort(T (&v)[E], T *sh, uint32_t m) {
+    static_assert(E == 1 || E == 2 || E == 4 || E == 8, "values per thread");
+    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
+    for (uint32_t k = 2; k <= m; k <<= 1) {
+        for (uint32_t j = k >> 1; j >= 64u * E; j >>= 1) {
+#pragma unroll
+            for (int e = 0; e < E; e++) sh[i0 + 64u * e] = v[e];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                uint32_t i = i0 + 64u * e;
+                T o = sh[i ^ j];
+                bool low = (i & j) == 0u, up = (i & k) == 0u;
+                if ((o < v[e]) == (low == up)) v[e] = o;
+            }
+            __syncthreads();
+        }
+        if (E >= 8 && k >= 512u) sort_regs<4>(v, i0, k);
+        if (E >= 4 && k >= 256u) sort_regs<2>(v, i0, k);
+        if (E >= 2 && k >= 128u) sort_regs<1>(v, i0, k);
+        if (k >= 64u) sort_lanes<32>(v, i0, k);
+        if (k >= 32u) sort_lanes<16>(v, i0, k);
+        if (k >= 16u) sort_lanes<8>(v, i0, k);
+        if (k >= 8u) sort_lanes<4>(v, i0, k);
+        if (k >= 4u) sort_lanes<2>(v, i0, k);
+        sort_lanes<1>(v, i0, k);
+    }
+}
+
+// E groups of 64 values, one of each per lane, each sorted within its wave.
+template <int J, int E> __device__ __forceinline__ void sort_groups(uint32_t (&v)[E], uint32_t k) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool least = ((lane & J) == 0u) == ((lane & k) == 0u);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const uint32_t o = lane_xor<J>(v[e]);
+        v[e] = least ? min(v[e], o) : max(v[e], o);
+    }
+}
+template <int E> __device__ __forceinline__ void sort_wave(uint32_t (&v)[E]) {
+#pragma unroll
+    for (uint32_t k = 2; k <= 64u; k <<= 1) {
+        if (k >= 64u) sort_groups<32>(v, k);
+        if (k >= 32u) sort_groups<16>(v, k);
+        if (k >= 16u) sort_groups<8>(v, k);
+        if (k >= 8u) sort_groups<4>(v, k);
+        if (k >= 4u) sort_groups<2>(v, k);
+        sort_groups<1>(v, k);
+    }
+}
 
 // ---------------------------------------------------------------------------
 // k_raster: one workgroup per (view, tile): coverage and depth of every bin
@@ -2228,7 +2331,37 @@ __host__ __device__ static inline uint32_t xcd_positions(uint32_t items) {
     return (items + 8u * XCD_RUN - 1) / (8u * XCD_RUN) * (8u * XCD_RUN);
 }
 
-template <int T, int NT, bool HIZ>
+// ---- resolve: canonical triangle id per pixel ----
+template <int T, int NT>
+__device__ __forceinline__ void raster_resolve(const RasterArgs &P, const DevView &V, int tx0, int ty0,
+                                               const unsigned long long *keys) {
+    uint32_t rec0 = P.tri_base[V.in_tri_base];
+    bool centre = centre_tile(tx0, ty0);
+    for (int p = threadIdx.x; p < T * T; p += NT) {
+        int px = tx0 + (p % T), py = ty0 + (p / T);
+        unsigned long long key = keys[p];
+        uint32_t out = key != SR_EMPTY_KEY ? ~(uint32_t)key - rec0 : 0xFFFFFFFFu;
+        if (px < V.W && py < V.H) P.out_ids[V.fb_offset + (size_t)py * (size_t)V.W + (size_t)px] = out;
+        if (centre && px < tx0 + 2 && py < ty0 + 2) {
+            int ri = (ty0 / 64) * V.ref_tiles_x + (tx0 / 64);
+            P.center_ids[4 * (V.lum_offset + (uint32_t)ri) + (uint32_t)((py - ty0) * 2 + (px - tx0))] = out;
+        }
+    }
+}
+
+// The entries [start, end) of an item's list.  A frame whose records or list
+// entries outgrew their buffers is run again with larger ones; its lists are
+// incomplete (the binning keeps only entries that fit), so it rasterizes
+// nothing.  Every id read is also checked against the records.
+__device__ __forceinline__ void raster_list(const RasterArgs &P, uint32_t item, uint32_t nrec, uint32_t &start,
+                                            uint32_t &end) {
+    start = P.bin_start[item];
+    end = P.bin_end[item];
+    if (nrec > P.rec_cap || P.status->total_pairs > P.pair_cap) end = start;
+    if (end > P.pair_cap) end = P.pair_cap;
+}
+
+template <int T, int NT>
 __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long long *keys, uint32_t *stage) {
     constexpr int NW = NT / 64;               // waves
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2248,16 +2381,9 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
     // quad) tasks that all NT threads then walk, so one-pixel and full-tile
     // triangles, and tiles with few or many entries, keep every lane busy.
     __shared__ int wtot[NW];
-    __shared__ uint32_t zmin_s[HIZ ? NT : 1];
-    // A frame whose records or list entries outgrew their buffers is run
-    // again with larger ones; its lists are incomplete (the binning keeps
-    // only entries that fit), so it rasterizes nothing.  Every id read is
-    // also checked against the records.
-    const uint32_t nrec = P.status->total_records, npairs = P.status->total_pairs;
-    uint32_t start = P.bin_start[item];
-    uint32_t end = P.bin_end[item];
-    if (nrec > P.rec_cap || npairs > P.pair_cap) end = start;
-    if (end > P.pair_cap) end = P.pair_cap;
+    const uint32_t nrec = P.status->total_records;
+    uint32_t start, end;
+    raster_list(P, item, nrec, start, end);
     for (uint32_t c0 = start; c0 < end; c0 += (uint32_t)NT) {
         uint32_t e = c0 + (uint32_t)tid;
         int nq = 0;
@@ -2283,14 +2409,6 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
             total += wtot[w];
         }
         stage[F_INCL * NT + tid] = (uint32_t)incl;
-        // HIZ: a quad task is dropped when its entry's depth bound lies
-        // behind all four of the quad's stored depths (the entry could not
-        // win any of them; a stale read only keeps more work).
-        if constexpr (HIZ) {
-#define SFE(f) __uint_as_float(stage[(f) * NT + tid])
-            zmin_s[tid] = nq > 0 ? tri_zmin_key(SFE(F_ZA), SFE(F_ZDA), SFE(F_ZDB), SFE(F_OA), SFE(F_ODA), SFE(F_ODB)) : 0u;
-#undef SFE
-        }
         __syncthreads();
         for (int k0 = 0; k0 < total; k0 += NT) {
             int k = k0 + tid;
@@ -2301,30 +2419,15 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
                 for (int step = NT / 2; step > 0; step >>= 1)
                     if ((int)stage[F_INCL * NT + o + step - 1] <= k) o += step;
                 int before = o ? (int)stage[F_INCL * NT + o - 1] : 0;
-                uint32_t zb = 0u;
-                if constexpr (HIZ) zb = zmin_s[o];
-                walk_quad<T, NT>(S, P, stage, o, k - before, tx0, ty0, keys, zb);
+                walk_quad<T, NT>(S, P, stage, o, k - before, tx0, ty0, keys, 0u);
             }
         }
         __syncthreads();
     }
-
-    // ---- resolve: canonical triangle id per pixel ----
-    uint32_t rec0 = P.tri_base[V.in_tri_base];
-    bool centre = centre_tile(tx0, ty0);
-    for (int p = tid; p < T * T; p += NT) {
-        int px = tx0 + (p % T), py = ty0 + (p / T);
-        unsigned long long key = keys[p];
-        uint32_t out = key != SR_EMPTY_KEY ? ~(uint32_t)key - rec0 : 0xFFFFFFFFu;
-        if (px < V.W && py < V.H) P.out_ids[V.fb_offset + (size_t)py * (size_t)V.W + (size_t)px] = out;
-        if (centre && px < tx0 + 2 && py < ty0 + 2) {
-            int ri = (ty0 / 64) * V.ref_tiles_x + (tx0 / 64);
-            P.center_ids[4 * (V.lum_offset + (uint32_t)ri) + (uint32_t)((py - ty0) * 2 + (px - tx0))] = out;
-        }
-    }
+    raster_resolve<T, NT>(P, V, tx0, ty0, keys);
 }
 
-template <int T, int NT, bool HIZ = false>
+template <int T, int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : 5))) k_raster(RasterArgs P) {
     __shared__ unsigned long long keys[T * T];
     __shared__ uint32_t stage[Stage<T>::COUNT * NT];
@@ -2332,7 +2435,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
     clock_start(P.clock, CLOCK_RASTER);
     if (!P.persistent) {
         const uint32_t item = xcd_item(blockIdx.x);
-        if (item < P.total_items) raster_item<T, NT, HIZ>(P, item, keys, stage);
+        if (item < P.total_items) raster_item<T, NT>(P, item, keys, stage);
     } else {
         // Every workgroup starts at its own position; the rest are drained
         // from counters, each shared by the workgroups of one residue of the
@@ -2349,13 +2452,153 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
             uint32_t got = 0u;
             if (threadIdx.x == 0) got = atomicAdd(&P.work[g].next, 1u);
             const uint32_t item = xcd_item(pos);
-            if (item < P.total_items) raster_item<T, NT, HIZ>(P, item, keys, stage);
+            if (item < P.total_items) raster_item<T, NT>(P, item, keys, stage);
             if (threadIdx.x == 0) next = g + groups * (first + got);
             __syncthreads();
             pos = next;
             __syncthreads();
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// k_raster_near: the raster of overdrawn frames (many large triangles deep),
+// one wave per (view, 16-px tile).  The wave takes 256 bin entries at a time
+// and sorts them by depth bound (tri_zmin_key) in four groups of 64, in
+// registers.  A round sets up the 16 nearest entries left of each group, one
+// per lane, walks their quads, and then takes the largest depth stored in
+// each 8x8 quadrant of the tile.  An entry whose bound lies behind the
+// quadrants that its box meets cannot win a pixel and is not set up, and once
+// that holds for the nearest one left, the rest of the 256 are passed over; a
+// quad task is dropped likewise when its entry lies behind the quad's four
+// stored depths.  The visibility buffer does not change: the depth test's
+// minimum does not depend on the order, and what is dropped cannot win.
+//
+// Bound by VALU issue.  On 100,000 triangles about 21 deep at 3840x2160 (150
+// entries a tile) one round usually suffices: 47 entries set up and 440 quads
+// walked a tile instead of 150 and 1380.  In list order, with the quad test
+// alone and four waves a tile, the raster took 496 us at 2465 VALU
+// instructions a wave; in this order with four waves sharing a tile (one
+// setting up at a time, barriers in each round) 396 us at 1286, which is 0.69
+// of the issue rate; one wave a tile needs no barrier and takes 195 us at
+// 3420, 0.94 of it.  Frames of small triangles (the heightfield) keep
+// k_raster, whose four waves share their long lists.
+// ---------------------------------------------------------------------------
+#define NEAR_BATCH 256
+
+// Pixels, in whole quads, of tile (tx0, ty0) that the box of record g meets:
+// [x0, x1) x [y0, y1) relative to the tile, empty when x0 >= x1 or y0 >= y1.
+struct TileBox { int x0, y0, x1, y1; };
+template <int T> __device__ __forceinline__ TileBox tile_box(uint4 g, int tx0, int ty0) {
+    TileBox b;
+    b.x0 = max((int)(g.x & 0xFFFEu) - tx0, 0);
+    b.y0 = max((int)((g.x >> 16) & 0xFFFEu) - ty0, 0);
+    b.x1 = min((int)(((g.y & 0xFFFFu) + 1u) & ~1u) - tx0, T);
+    b.y1 = min((int)(((g.y >> 16) + 1u) & ~1u) - ty0, T);
+    return b;
+}
+
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = max(v, lane_xor<1>(v));
+    v = max(v, lane_xor<2>(v));
+    v = max(v, lane_xor<4>(v));
+    v = max(v, lane_xor<8>(v));
+    v = max(v, lane_xor<16>(v));
+    return max(v, lane_xor<32>(v));
+}
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_raster_near(RasterArgs P) {
+    constexpr int T = 16;
+    __shared__ unsigned long long keys[T * T];
+    __shared__ uint32_t stage[Stage<T>::COUNT * 64], zmin[64];
+    clock_start(P.clock, CLOCK_RASTER);
+    const uint32_t item = xcd_item(blockIdx.x);
+    if (item >= P.total_items) return;
+    const int lane = threadIdx.x;
+    const DevView &V = P.views[find_view(P, item)];
+    const DevScene &S = *V.scene;
+    const uint32_t tile = item - V.item_base;
+    const int tx0 = (int)(tile % (uint32_t)V.tiles_x) * T, ty0 = (int)(tile / (uint32_t)V.tiles_x) * T;
+#pragma unroll
+    for (int i = 0; i < T * T; i += 64) keys[i + lane] = SR_EMPTY_KEY;
+    __syncthreads();
+    const uint32_t nrec = P.status->total_records;
+    uint32_t start, end;
+    raster_list(P, item, nrec, start, end);
+    uint32_t zq[4] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};   // farthest depth of each quadrant
+    for (uint32_t c0 = start; c0 < end; c0 += NEAR_BATCH) {
+        uint32_t id[NEAR_BATCH / 64], key[NEAR_BATCH / 64];
+        const uint32_t far = max(max(zq[0], zq[1]), max(zq[2], zq[3]));
+#pragma unroll
+        for (int g = 0; g < NEAR_BATCH / 64; g++) {
+            const uint32_t e = c0 + (uint32_t)(64 * g + lane);
+            const uint32_t r = e < end ? P.list[e] : 0xFFFFFFFFu;
+            const uint32_t z = r < nrec ? P.geo[r].w : 0xFFFFFFFFu;
+            const bool live = r < nrec && z <= far;
+            id[g] = live ? r : 0xFFFFFFFFu;
+            // the bound loses its low bits to the lane: a bound still
+            key[g] = (live ? min(z, 0xFFFFFF7Fu) & ~63u : 0xFFFFFFC0u) | (uint32_t)lane;
+        }
+        const int groups = (int)min((end - c0 + 63u) / 64u, (uint32_t)(NEAR_BATCH / 64));
+        if (groups > 2) sort_wave(key);
+        else if (groups == 2) sort_wave(reinterpret_cast<uint32_t(&)[2]>(key));
+        else sort_wave(reinterpret_cast<uint32_t(&)[1]>(key));
+#pragma unroll
+        for (int g = 0; g < NEAR_BATCH / 64; g++) id[g] = (uint32_t)__shfl((int)id[g], (int)(key[g] & 63u), 64);
+        for (int round = 0; round < 4; round++) {
+            uint32_t nearest = 0xFFFFFFC0u;
+#pragma unroll
+            for (int g = 0; g < NEAR_BATCH / 64; g++)
+                nearest = min(nearest, (uint32_t)__builtin_amdgcn_readlane((int)key[g], 16 * round) & ~63u);
+            if (nearest > min(max(max(zq[0], zq[1]), max(zq[2], zq[3])), 0xFFFFFFBFu)) break;
+            // lanes take the groups' entries in turn, so the round's go
+            // roughly nearest first
+            uint32_t r = 0u, z = 0u;
+#pragma unroll
+            for (int g = 0; g < NEAR_BATCH / 64; g++) {
+                const uint32_t rg = (uint32_t)__shfl((int)id[g], 16 * round + (lane >> 2), 64);
+                const uint32_t zg = (uint32_t)__shfl((int)key[g], 16 * round + (lane >> 2), 64) & ~63u;
+                if ((lane & 3) == g) {
+                    r = rg;
+                    z = zg;
+                }
+            }
+            int nq = 0;
+            if (r != 0xFFFFFFFFu) {
+                const uint4 g = P.geo[r];
+                const TileBox b = tile_box<T>(g, tx0, ty0);
+                uint32_t behind = 0u;
+                if (b.x0 < 8 && b.y0 < 8) behind = max(behind, zq[0]);
+                if (b.x1 > 8 && b.y0 < 8) behind = max(behind, zq[1]);
+                if (b.x0 < 8 && b.y1 > 8) behind = max(behind, zq[2]);
+                if (b.x1 > 8 && b.y1 > 8) behind = max(behind, zq[3]);
+                if (z <= behind) {
+                    TriSetup ts;
+                    tri_setup(g, P.raster + 4 * (size_t)r, tx0, ty0, ts);
+                    nq = stage_entry<T, 64>(ts, r, g.z, tx0, ty0, stage, lane);
+                }
+            }
+            zmin[lane] = z;
+            const uint32_t incl = wave_incl_scan((uint32_t)nq);
+            stage[F_INCL * 64 + lane] = incl;
+            const int total = __builtin_amdgcn_readlane((int)incl, 63);
+            __syncthreads();
+            for (int k = lane; k < total; k += 64) {
+                // owner = number of entries whose inclusive count is <= k
+                int own = 0;
+#pragma unroll
+                for (int step = 32; step > 0; step >>= 1)
+                    if ((int)stage[F_INCL * 64 + own + step - 1] <= k) own += step;
+                const int before = own ? (int)stage[F_INCL * 64 + own - 1] : 0;
+                walk_quad<T, 64>(S, P, stage, own, k - before, tx0, ty0, keys, zmin[own]);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                zq[q] = wave_max_u32((uint32_t)(keys[(8 * (q >> 1) + (lane >> 3)) * T + 8 * (q & 1) + (lane & 7)] >> 32));
+        }
+    }
+    raster_resolve<T, 64>(P, V, tx0, ty0, keys);
 }
 
 // ---------------------------------------------------------------------------
@@ -2661,7 +2904,7 @@ __global__ void __launch_bounds__(256) k_tr_bins(const DevView *views, const uin
         int mnx = 0, mny = 0, mxx = 0, mxy = 0, bx0 = 0, by0 = 0, nx = 0, nbins = 0, tiles_x = 1, ntiles = 0;
         uint32_t first = 0u;
         if ((g.z & (SR_GEO_TRANSLUCENT | SR_GEO_EMPTY)) == SR_GEO_TRANSLUCENT) {
-            const DevView &V = views[g.w];
+            const DevView &V = views[geo_view(g)];
             mnx = (int)(g.x & 0xFFFFu); mny = (int)(g.x >> 16); mxx = (int)(g.y & 0xFFFFu); mxy = (int)(g.y >> 16);
             bx0 = mnx / SR_REF_TILE; by0 = mny / SR_REF_TILE;
             nx = max((mxx + SR_REF_TILE - 1) / SR_REF_TILE - bx0, 0);
@@ -2732,81 +2975,6 @@ __device__ __forceinline__ uint32_t z_desc_key(float z) {
     uint32_t b = __float_as_uint(z);
     uint32_t asc = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
     return ~asc;
-}
-
-// ---------------------------------------------------------------------------
-// Workgroup sort in registers: ascending bitonic sort of the first m of
-// blockDim.x * E values, E per thread (value e of a thread is element wave *
-// 64 E + 64 e + lane); m a power of two, and all of them unless E is 1.  Exchanges at a distance below 64
-// are lane exchanges, below 64 E register exchanges; only those between
-// waves go through LDS (sh, one word per element) with barriers.
-// ---------------------------------------------------------------------------
-// Lane l's value from lane l ^ J: a DPP move where the hardware has one, else
-// a swizzle (within 32 lanes) or a permute.
-template <int J> __device__ __forceinline__ int32_t lane_xor(int32_t v) {
-    if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);          // quad_perm 1 0 3 2
-    else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);     // quad_perm 2 3 0 1
-    else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);    // row_ror 8
-    else if constexpr (J < 32) return __builtin_amdgcn_ds_swizzle(v, (J << 10) | 0x1F);       // xor within 32 lanes
-    else return __shfl_xor(v, J, 64);
-}
-
-template <int J> __device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
-    const uint32_t lo = (uint32_t)lane_xor<J>((int32_t)(uint32_t)v), hi = (uint32_t)lane_xor<J>((int32_t)(v >> 32));
-    return ((unsigned long long)hi << 32) | lo;
-}
-
-template <int J, class T, int E> __device__ __forceinline__ void sort_lanes(T (&v)[E], uint32_t i0, uint32_t k) {
-    const bool low = (threadIdx.x & J) == 0u;
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        T o = lane_xor<J>(v[e]);
-        bool up = ((i0 + 64u * e) & k) == 0u;
-        if ((o < v[e]) == (low == up)) v[e] = o;
-    }
-}
-
-template <int Q, class T, int E> __device__ __forceinline__ void sort_regs(T (&v)[E], uint32_t i0, uint32_t k) {
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        if ((e & Q) == 0 && e + Q < E) {
-            bool up = ((i0 + 64u * e) & k) == 0u;
-            T a = v[e], b = v[e + Q];
-            if ((b < a) == up) {
-                v[e] = b;
-                v[e + Q] = a;
-            }
-        }
-    }
-}
-
-template <class T, int E> __device__ __forceinline__ void block_sort(T (&v)[E], T *sh, uint32_t m) {
-    static_assert(E == 1 || E == 2 || E == 4 || E == 8, "values per thread");
-    const uint32_t i0 = (threadIdx.x >> 6) * 64u * E + (threadIdx.x & 63u);
-    for (uint32_t k = 2; k <= m; k <<= 1) {
-        for (uint32_t j = k >> 1; j >= 64u * E; j >>= 1) {
-#pragma unroll
-            for (int e = 0; e < E; e++) sh[i0 + 64u * e] = v[e];
-            __syncthreads();
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                uint32_t i = i0 + 64u * e;
-                T o = sh[i ^ j];
-                bool low = (i & j) == 0u, up = (i & k) == 0u;
-                if ((o < v[e]) == (low == up)) v[e] = o;
-            }
-            __syncthreads();
-        }
-        if (E >= 8 && k >= 512u) sort_regs<4>(v, i0, k);
-        if (E >= 4 && k >= 256u) sort_regs<2>(v, i0, k);
-        if (E >= 2 && k >= 128u) sort_regs<1>(v, i0, k);
-        if (k >= 64u) sort_lanes<32>(v, i0, k);
-        if (k >= 32u) sort_lanes<16>(v, i0, k);
-        if (k >= 16u) sort_lanes<8>(v, i0, k);
-        if (k >= 8u) sort_lanes<4>(v, i0, k);
-        if (k >= 4u) sort_lanes<2>(v, i0, k);
-        sort_lanes<1>(v, i0, k);
-    }
 }
 
 // k_tr_sort: one workgroup per 64-px tile orders its list back to front as
@@ -3663,7 +3831,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
         case 8: SR_LAUNCH_TIMED(e2, e4, (k_raster<8, 64>), dim3(grid), dim3(64), st, P); break;
         case 32: SR_LAUNCH_TIMED(e2, e4, (k_raster<32, 512>), dim3(grid), dim3(512), st, P); break;
         default:
-            if (a.hiz) SR_LAUNCH_TIMED(e2, e4, (k_raster<16, 256, true>), dim3(grid), dim3(256), st, P);
+            if (a.overdraw) SR_LAUNCH_TIMED(e2, e4, k_raster_near, dim3(xcd_positions(a.total_items)), dim3(64), st, P);
             else SR_LAUNCH_TIMED(e2, e4, (k_raster<16, 256>), dim3(grid), dim3(256), st, P);
             break;
     }

@@ -189,7 +189,6 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
     a.out_lum = (float *)(base + o_lum);
     a.center_ids = (uint32_t *)(base + o_center);
     a.persistent_blocks = 0;
-    a.hiz = 0;
     if (launch_frame(a, st) != hipSuccess) return fail(SR_ERR_HIP, "launch: %s", hipGetErrorString(hipGetLastError()));
     DevStatus s;
     if (hipMemcpyAsync(&s, a.status, sizeof(s), hipMemcpyDeviceToHost, st) != hipSuccess ||

@@ -115,7 +115,7 @@ static void fill_stats(sr_renderer *r) {
     r->stats.binned_pairs = r->pipe.last_pairs;
     r->stats.tiles = r->p_items;
     r->stats.draws = (uint32_t)r->p_draws.size();
-    r->stats.depth_rejection = r->pipe.last_hiz ? 1u : 0u;
+    r->stats.depth_rejection = r->pipe.last_near ? 1u : 0u;
     r->times_pending = true;
 }
 

@@ -239,7 +239,7 @@ int Pipeline::launch_graph(const FrameArgs &a, size_t vbytes, size_t upload) {
     k.n[4] = a.total_items; k.n[5] = (uint64_t)a.tile_size; k.n[6] = (uint64_t)a.any_tangents; k.n[7] = a.rec_cap;
     k.n[8] = a.pair_cap; k.n[9] = a.clip_cap; k.n[10] = (uint64_t)a.persistent_blocks; k.n[11] = vbytes;
     k.n[12] = upload; k.n[13] = a.color_plane; k.n[14] = (uint64_t)a.has_translucent;
-    k.n[15] = ((uint64_t)a.tr_cap << 32) | a.tr_slots | ((uint64_t)a.hiz << 31);
+    k.n[15] = ((uint64_t)a.tr_cap << 32) | a.tr_slots | ((uint64_t)a.overdraw << 31);
     const void *ptrs[] = {a.views, a.draws, a.xv, a.xt, a.tri_counts, a.tri_chunks, a.tri_base, a.bin_start, a.bin_end,
                           a.scan_partials, a.list, a.rec_geo, a.rec_raster, a.clip_queue, a.clip_buf, a.status,
                           a.out_ids, a.out_depth, a.out_color, a.out_rgba, a.out_lum, a.center_ids, stage.ptr,
@@ -391,10 +391,10 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
             a.center_color = (float4 *)center_color.ptr;
         }
         a.persistent_blocks = persistent_blocks;
-        // depth rejection pays where triangles span many tiles and tiles
-        // hold many of them (high overdraw); judged from the last frame
-        a.hiz = tile_size == 16 && last_pairs > 32ull * total_items && last_pairs > 4ull * last_records;
-        last_hiz = a.hiz != 0;
+        // depth order pays where triangles span many tiles and tiles hold
+        // many of them (high overdraw); judged from the last frame
+        a.overdraw = tile_size == 16 && last_pairs > 32ull * total_items && last_pairs > 4ull * last_records;
+        last_near = a.overdraw != 0;
         if (use_graph) {
             if ((r = launch_graph(a, vbytes, upload))) return r;
         } else {

@@ -70,7 +70,7 @@ struct Pipeline {
     PinBuf stage, status_host;
     uint32_t rec_cap = 0, pair_cap = 0, clip_cap = 0, tr_cap = 0;
     uint32_t last_records = 0, last_pairs = 0;
-    bool last_hiz = false;            // the last frame's raster used depth rejection
+    bool last_near = false;           // the last frame's raster took entries nearest first (k_raster_near)
     struct GraphKey {
         uint64_t n[16];
         uint64_t p[40];

@@ -137,3 +137,45 @@ def test_persistent_raster_block_counts(sr, scenes, env, blocks):
     for want, got in zip(*out):
         for x, y in zip(want, got):
             assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+
+
+# list lengths around the groups of 64 and the batches of 256 that the
+# overdraw raster sorts; "hole" leaves part of the view uncovered, so no
+# quadrant there ever rejects, and "flat" puts all triangles at two depths
+@pytest.mark.parametrize("n", [40, 64, 65, 129, 256, 257, 520])
+@pytest.mark.parametrize("kind", ["full", "hole", "flat"])
+def test_overdraw_raster_list_lengths(sr, orc, n, kind):
+    """n large triangles over every tile of a 64x48 view (odd tile rows off
+    screen): the frame takes the overdraw raster on its second rendering and
+    both renderings have the oracle's visibility buffer."""
+    from util import attach_dummy, screen_triangle_scene
+    W, H = 64, 48
+    rng = np.random.default_rng(1000 * n + len(kind))
+    c = rng.uniform([0, 0], [W * 16, H * 16], (n, 1, 2))
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2]) + rng.uniform(-0.4, 0.4, (n, 3))
+    rad = rng.uniform(40, 90, (n, 3)) * 16
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * rad[..., None])
+    if kind == "hole":
+        tris[..., 0] = np.minimum(tris[..., 0], 40 * 16)
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    depths = rng.uniform(2.0, 90.0, (n, 1)) * rng.uniform(0.9, 1.1, (n, 3))
+    if kind == "flat":
+        depths = np.where(rng.random((n, 1)) < 0.5, 10.0, 20.0) * np.ones((n, 3))
+    scene, spec = screen_triangle_scene(sr, tris, depths, W, H)
+    attach_dummy(sr, scene)
+    import swraster_viewer_amd.scenes as sc
+    cam = sc.make_camera(spec)
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()
+    gscene = sr.Scene(scene)
+    r = sr.Renderer(W, H)
+    for k in range(2):
+        r.render_scene(gscene, cam)
+        ids, depth = r.read_vbuffer()
+        assert np.array_equal(ids, want["ids"]), f"frame {k}"
+        assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32)), f"frame {k}"
+    assert r.stats()["depth_rejection"] == 1
+    r.close()
