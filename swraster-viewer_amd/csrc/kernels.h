@@ -62,6 +62,7 @@ struct FrameArgs {
     uint32_t tr_cap;
     float4 *center_color;         // 4 (colour, depth) per 64px tile
     int32_t persistent_blocks;    // 0 = one block per item
+    int32_t direct;               // direct binning: sort_hist holds bin_matrix_entries words; no pair arrays
     int32_t overdraw;             // 16-px raster that takes overdrawn tiles' entries nearest first
     hipEvent_t events[5];         // optional stage events (the launches that carry them cost about 4 us each):
                                   // start, setup done, bins done, shade done, raster done
@@ -73,6 +74,10 @@ struct FrameArgs {
 int bin_sort_bits(uint32_t bins);
 int bin_sort_passes(uint32_t bins);
 uint32_t bin_sort_tiles(uint32_t pair_cap);
+
+// Words of the direct binning's count matrix for a frame of total_in input
+// triangles and `items` tiles, or 0 where the frame is too large for it.
+size_t bin_matrix_entries(uint32_t total_in, uint32_t items);
 
 // Launch the whole per-frame sequence on a stream.  Returns hipSuccess or the
 // first launch error.

@@ -778,6 +778,11 @@ struct SetupOut {
     uint32_t cap;
     SR_GLOBAL DevStatus *status;
     int T;
+    // direct binning (k_setup<true>): the chunks' pair counts per tile, one
+    // row of `items` per chunk, and each chunk's first record
+    SR_GLOBAL uint32_t *matrix;
+    SR_GLOBAL uint32_t *chunk_first;
+    uint32_t items, nchunks;
 };
 
 __device__ __forceinline__ int32_t top_left_bias(int32_t a, int32_t b) { return (a < 0 || (a == 0 && b > 0)) ? 0 : -1; }
@@ -1085,22 +1090,58 @@ __device__ __forceinline__ Rect emit_clipped_fan(const DevView *views, const Dev
                          SRC_CLIPPED | (f << 27) | e, 0u, O);
 }
 
+// Counts a lane's rectangle of tiles in hist (LDS adds); rectangles of more
+// than 32 tiles are shared by the wave.
+__device__ __forceinline__ void count_rect(uint32_t *hist, const RectBins &b) {
+    if (b.nb <= 32) {
+        uint32_t row = b.first;
+        for (int k = 0; k < b.nb; k += b.rw, row += (uint32_t)b.stride)
+            for (int x = 0; x < b.rw; x++) atomicAdd(&hist[row + (uint32_t)x], 1u);
+    }
+    for (uint64_t big = __ballot(b.nb > 32); big; big &= big - 1ull) {
+        const int l = __ffsll((unsigned long long)big) - 1;
+        const int nb = __builtin_amdgcn_readlane(b.nb, l), rw = __builtin_amdgcn_readlane(b.rw, l);
+        const int stride = __builtin_amdgcn_readlane(b.stride, l);
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)b.first, l);
+        for (int k = threadIdx.x & 63; k < nb; k += 64) atomicAdd(&hist[first + (uint32_t)((k / rw) * stride + k % rw)], 1u);
+    }
+}
+
 // The post-clip id of input triangle t is its chunk's first id plus the
 // fan counts before it in the chunk (a workgroup scan); it is stored for
 // the per-view offsets.  A triangle inside the frustum is set up from its
 // clip positions; one that crosses it has its fan triangles set up from
 // the polygon k_clip left in the clip buffer (ids tri_base[t] + f).
+// DIRECT (small frames, see the direct binning): `chunk` holds the chunks'
+// counts, which each workgroup adds up itself (no scan before it), and the
+// chunk's pairs are counted per tile in LDS.
+template <bool DIRECT>
 __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDraw *draws, int ndraws, uint32_t total,
                                                const float4 *xs, const uint32_t *counts, const uint32_t *chunk,
                                                const float *clip_buf, uint32_t *tri_base, SetupOut O) {
     __shared__ uint32_t sh[17];
+    extern __shared__ __align__(16) uint32_t hist[];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += stride) {
         uint32_t t = base + threadIdx.x;
         uint32_t ex, c = t < total ? counts[t] : 0u;
-        uint32_t nf = count_fans(c);
-        block_excl_scan(nf, ex, sh);
-        uint32_t id = chunk[base >> 8] + ex;
+        uint32_t nf = count_fans(c), first;
+        if constexpr (DIRECT) {
+            const uint32_t me = base >> 8;
+            uint32_t sum = 0u, none;
+            for (uint32_t k = threadIdx.x; k < me; k += 256u) sum += chunk[k];
+            for (uint32_t k = threadIdx.x; k < O.items; k += 256u) hist[k] = 0u;
+            first = block_excl_scan(sum, none, sh);
+            const uint32_t n = block_excl_scan(nf, ex, sh);
+            if (threadIdx.x == 0) {
+                O.chunk_first[me] = first;
+                if (me + 1u == O.nchunks) O.status->total_records = first + n;
+            }
+        } else {
+            first = chunk[base >> 8];
+            block_excl_scan(nf, ex, sh);
+        }
+        uint32_t id = first + ex;
         Rect r = {0, 0, 0, 0};
         int view = 0, d = 0;
         if (t < total) {
@@ -1116,7 +1157,9 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
                 if (c == 1u) r = setup_input_triangle(draws[d], d, views, t, xs, id, O);
             }
         }
-        uint32_t np = (uint32_t)rect_bins(views, view, r).nb;
+        RectBins rb = rect_bins(views, view, r);
+        uint32_t np = (uint32_t)rb.nb;
+        if constexpr (DIRECT) count_rect(hist, rb);
         int nclip = (c & SR_COUNT_CLIPPED) ? (int)nf : 0;
         int maxf = wave_max(nclip);
         for (int f = 0; f < maxf; f++) {
@@ -1124,11 +1167,21 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
             if (f < nclip)
                 rf = emit_clipped_fan(views, draws[d], clip_buf, (c & ~SR_COUNT_CLIPPED) >> 4, (uint32_t)f,
                                       id + (uint32_t)f, O);
-            np += (uint32_t)rect_bins(views, view, rf).nb;
+            rb = rect_bins(views, view, rf);
+            np += (uint32_t)rb.nb;
+            if constexpr (DIRECT) count_rect(hist, rb);
         }
-        uint32_t npx;
-        uint32_t chunk_np = block_excl_scan(np, npx, sh);
-        if (threadIdx.x == 0) O.chunk_pairs[base >> 8] = chunk_np;
+        if constexpr (DIRECT) {
+            __syncthreads();
+            SR_GLOBAL uint4 *row = reinterpret_cast<SR_GLOBAL uint4 *>(O.matrix + (size_t)(base >> 8) * O.items);
+            const uint4 *h = reinterpret_cast<const uint4 *>(hist);
+            for (uint32_t k = threadIdx.x; k < O.items / 4u; k += 256u) row[k] = h[k];
+            __syncthreads();
+        } else {
+            uint32_t npx;
+            uint32_t chunk_np = block_excl_scan(np, npx, sh);
+            if (threadIdx.x == 0) O.chunk_pairs[base >> 8] = chunk_np;
+        }
     }
 }
 
@@ -1450,6 +1503,178 @@ __global__ void __launch_bounds__(256) k_bin_bounds(BinBounds B) {
         if (b >= B.items) continue;    // (only in a frame that overflowed and runs again)
         if (i == 0u || B.key[i - 1u] != b) B.bin_start[b] = i;
         if (i + 1u == n || B.key[i + 1u] != b) B.bin_end[b] = i + 1u;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Direct binning: the same lists for small frames in two launches
+// ---------------------------------------------------------------------------
+// The radix passes take six to nine launches of a few microseconds each,
+// whatever the frame's size.  Where a matrix of (256-triangle chunk, tile)
+// counts is small, setup counts each chunk's pairs per tile in LDS and stores
+// the chunk's row; k_bin_cols turns each tile's column into the chunks'
+// offsets in the tile's list and leaves the tile's count in a last row; and
+// k_bin_place, one workgroup per chunk, scans those counts into the tiles'
+// list starts and puts the chunk's pairs at start + offset + rank, the rank
+// in record order, so the lists are the radix passes' own.  Setup also adds
+// up the chunks' record counts itself, which saves the scan before it.
+// Bound by latency: with 20,480 triangles at 1280x720 (0.3M entries) the
+// scans, expansion, passes and bounds took 44 us and this takes 15, two of
+// them in setup.  The matrix moves 4 B per entry four times and the gain over
+// the radix passes falls with it: whole frames 132 -> 102 us at 0.3M entries,
+// 188 -> 137 at 0.7M, 194 -> 171 at 2.2M, 260 -> 248 at 2.7M, so frames with
+// more than DB_MAX_ENTRIES keep the passes.
+#define DB_MAX_CHUNKS 1024u
+#define DB_MAX_ITEMS 8192u           // tile counters in LDS
+#define DB_MAX_ENTRIES (3u << 20)
+#define DB_COL_TILES 16u             // k_bin_cols: tiles and row segments of a workgroup
+#define DB_COL_SEGS 64u
+#define DB_COL_ROWS (DB_MAX_CHUNKS / DB_COL_SEGS)
+
+struct BinDirect {
+    const SR_GLOBAL DevView *views;
+    const SR_GLOBAL uint4 *geo;
+    const SR_GLOBAL uint32_t *chunk_first;
+    SR_GLOBAL uint32_t *matrix;      // nchunks rows of items, then the tiles' counts
+    SR_GLOBAL uint32_t *list, *bin_start, *bin_end;
+    SR_GLOBAL DevStatus *status;
+    uint64_t *stamp;
+    uint32_t nchunks, items, rec_cap, pair_cap;
+    int T, bits;
+};
+
+__global__ void __launch_bounds__(1024) k_bin_cols(BinDirect P) {
+    __shared__ uint32_t seg[DB_COL_SEGS][DB_COL_TILES + 1];
+    stamp_start(P.stamp);
+    const uint32_t lt = threadIdx.x % DB_COL_TILES, sg = threadIdx.x / DB_COL_TILES;
+    const uint32_t tile = blockIdx.x * DB_COL_TILES + lt;
+    const uint32_t rows = (P.nchunks + DB_COL_SEGS - 1u) / DB_COL_SEGS, r0 = sg * rows;
+    SR_GLOBAL uint32_t *col = P.matrix + tile;
+    uint32_t v[DB_COL_ROWS], sum = 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < DB_COL_ROWS; i++) {
+        v[i] = i < rows && r0 + i < P.nchunks && tile < P.items ? col[(size_t)(r0 + i) * P.items] : 0u;
+        sum += v[i];
+    }
+    seg[sg][lt] = sum;
+    __syncthreads();
+    {
+        // wave w scans tile w's segments, one per lane
+        const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+        const uint32_t x = seg[lane][w], incl = wave_incl_scan(x);
+        seg[lane][w] = incl - x;
+        if (lane == 63u && blockIdx.x * DB_COL_TILES + w < P.items)
+            P.matrix[(size_t)P.nchunks * P.items + blockIdx.x * DB_COL_TILES + w] = incl;
+    }
+    __syncthreads();
+    uint32_t run = seg[sg][lt];
+#pragma unroll
+    for (uint32_t i = 0; i < DB_COL_ROWS; i++) {
+        if (i < rows && r0 + i < P.nchunks && tile < P.items) col[(size_t)(r0 + i) * P.items] = run;
+        run += v[i];
+    }
+}
+static_assert(DB_COL_TILES * 64u == 1024u && DB_COL_SEGS == 64u, "one wave per tile of the workgroup");
+
+// A chunk's pairs are laid out flat in record order (a scan of 256 records'
+// pair counts, searched by each thread for its pairs) and taken 1024 at a
+// time, 256 consecutive ones by each wave.  Lanes of one tile are counted by
+// ballots and take their slots with one LDS add; only these adds go wave
+// after wave, which keeps the order.
+__global__ void __launch_bounds__(256) k_bin_place(BinDirect P) {
+    extern __shared__ __align__(16) uint32_t next[];        // each tile's next list entry for this chunk
+    __shared__ uint32_t sh[17];
+    __shared__ uint32_t pex[256], rfirst[256];
+    __shared__ int rrw[256], rstride[256];
+    constexpr uint32_t QUADS = DB_MAX_ITEMS / 1024u;        // most tiles of a thread, four at a time
+    const uint32_t c = blockIdx.x, tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const uint32_t quads = (P.items + 1023u) / 1024u, t0 = 4u * quads * tid;
+    const SR_GLOBAL uint32_t *totals = P.matrix + (size_t)P.nchunks * P.items;
+    const SR_GLOBAL uint32_t *row = P.matrix + (size_t)c * P.items;
+    {
+        uint4 n[QUADS];
+        uint32_t sum = 0u, run;
+#pragma unroll
+        for (uint32_t q = 0; q < QUADS; q++) {
+            n[q] = make_uint4(0u, 0u, 0u, 0u);
+            if (q < quads && t0 + 4u * q < P.items) n[q] = *reinterpret_cast<const SR_GLOBAL uint4 *>(totals + t0 + 4u * q);
+            sum += (n[q].x + n[q].y) + (n[q].z + n[q].w);
+        }
+        const uint32_t pairs = block_excl_scan(sum, run, sh);
+        if (c == 0u && tid == 0u) P.status->total_pairs = pairs;
+#pragma unroll
+        for (uint32_t q = 0; q < QUADS; q++) {
+            const uint32_t t = t0 + 4u * q;
+            if (q < quads && t < P.items) {
+                const uint4 o = *reinterpret_cast<const SR_GLOBAL uint4 *>(row + t);
+                const uint32_t s0 = run, s1 = s0 + n[q].x, s2 = s1 + n[q].y, s3 = s2 + n[q].z;
+                run = s3 + n[q].w;
+                *reinterpret_cast<uint4 *>(next + t) = make_uint4(s0 + o.x, s1 + o.y, s2 + o.z, s3 + o.w);
+                if (c == 0u) {                // the tiles' bounds
+                    *reinterpret_cast<SR_GLOBAL uint4 *>(P.bin_start + t) = make_uint4(s0, s1, s2, s3);
+                    *reinterpret_cast<SR_GLOBAL uint4 *>(P.bin_end + t) = make_uint4(s1, s2, s3, run);
+                }
+            }
+        }
+    }
+    const uint32_t total = min(P.status->total_records, P.rec_cap);
+    const uint32_t last = min(c + 1u < P.nchunks ? P.chunk_first[c + 1u] : total, total);
+    for (uint32_t r0 = P.chunk_first[c]; r0 < last; r0 += 256u) {
+        const uint32_t id = r0 + tid;
+        Rect r = {0, 0, 0, 0};
+        int view = 0;
+        if (id < last) {
+            uint4 g = P.geo[id];
+            view = geo_view(g);
+            if (!(g.z & (SR_GEO_EMPTY | SR_GEO_TRANSLUCENT))) {
+                int mnx = (int)(g.x & 0xFFFFu), mny = (int)(g.x >> 16), mxx = (int)(g.y & 0xFFFFu), mxy = (int)(g.y >> 16);
+                r = bin_rect(P.views[view], mnx, mny, mxx, mxy, P.T);
+            }
+        }
+        const RectBins b = rect_bins((const DevView *)P.views, view, r);
+        uint32_t ex;
+        const uint32_t pairs = block_excl_scan((uint32_t)b.nb, ex, sh);
+        pex[tid] = ex;
+        rfirst[tid] = b.first;
+        rrw[tid] = b.rw;
+        rstride[tid] = b.stride;
+        __syncthreads();
+        for (uint32_t p0 = 0; p0 < pairs; p0 += 1024u) {
+            uint32_t bin[4], o[4], got[4], rank[4];
+            int leader[4];
+            bool valid[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const uint32_t p = p0 + 256u * wave + 64u * s + lane;
+                valid[s] = p < pairs;
+                // the last record whose first pair is at or before p
+                o[s] = 0u;
+#pragma unroll
+                for (uint32_t step = 128; step > 0; step >>= 1)
+                    if (pex[o[s] + step] <= p) o[s] += step;
+                bin[s] = valid[s] ? bs_pair_bin(rfirst[o[s]], rrw[o[s]], rstride[o[s]], (int)(p - pex[o[s]])) : 0u;
+                const uint64_t m = bs_match(valid[s], bin[s], P.bits);
+                rank[s] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                leader[s] = valid[s] ? 63 - __clzll((long long)m) : lane;
+                got[s] = 0u;
+            }
+            const int waves = (int)min((pairs - p0 + 255u) / 256u, 4u);
+            for (int w = 0; w < waves; w++) {
+                if (wave == w) {
+#pragma unroll
+                    for (int s = 0; s < 4; s++)
+                        if (valid[s] && leader[s] == lane) got[s] = atomicAdd(&next[bin[s]], rank[s] + 1u);
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const uint32_t pos = (uint32_t)__shfl((int)got[s], leader[s], 64) + rank[s];
+                if (valid[s] && pos < P.pair_cap) P.list[pos] = r0 + o[s];      // else the frame runs again
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -3654,15 +3879,22 @@ uint32_t bin_sort_tiles(uint32_t pair_cap) {
     return std::max((uint32_t)(((uint64_t)pair_cap + te - 1) / te), 1u);
 }
 
+size_t bin_matrix_entries(uint32_t total_in, uint32_t items) {
+    const uint64_t nchunks = ((uint64_t)total_in + 255u) / 256u;
+    if (nchunks == 0 || nchunks > DB_MAX_CHUNKS || items > DB_MAX_ITEMS || nchunks * items > DB_MAX_ENTRIES) return 0;
+    return (size_t)(nchunks + 1) * items;
+}
+
 // A launch that stamps the stage-timing events from its own dispatch (start
 // when the kernel begins, stop when it ends) where the frame asks for them:
 // a separate event record between two kernels holds the queue for several
 // microseconds.
-#define SR_LAUNCH_TIMED(e0, e1, kern, grid, block, st, ...)                                      \
-    do {                                                                                        \
-        if ((e0) || (e1)) hipExtLaunchKernelGGL(kern, grid, block, 0, st, e0, e1, 0, __VA_ARGS__); \
-        else hipLaunchKernelGGL(kern, grid, block, 0, st, __VA_ARGS__);                          \
+#define SR_LAUNCH_TIMED_LDS(e0, e1, kern, grid, block, lds, st, ...)                              \
+    do {                                                                                          \
+        if ((e0) || (e1)) hipExtLaunchKernelGGL(kern, grid, block, lds, st, e0, e1, 0, __VA_ARGS__); \
+        else hipLaunchKernelGGL(kern, grid, block, lds, st, __VA_ARGS__);                          \
     } while (0)
+#define SR_LAUNCH_TIMED(e0, e1, kern, grid, block, st, ...) SR_LAUNCH_TIMED_LDS(e0, e1, kern, grid, block, 0, st, __VA_ARGS__)
 
 hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     const uint32_t GRID_CAP = 256 * 16;
@@ -3695,8 +3927,10 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     // too).  One workgroup up to SCAN_SINGLE_MAX chunks, else the
     // three-pass scan in place.
     uint32_t nchunks = (a.total_in + 255u) / 256u;
-    hipError_t e;
-    if (nchunks <= SCAN_SINGLE_MAX) {
+    hipError_t e = hipSuccess;
+    if (a.direct) {
+        // (k_setup adds the counts up)
+    } else if (nchunks <= SCAN_SINGLE_MAX) {
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, a.tri_chunks, nchunks, &a.status->total_records,
                            a.tri_base + a.total_in);
         e = hipGetLastError();
@@ -3709,8 +3943,16 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     so.cap = a.rec_cap; so.status = (SR_GLOBAL DevStatus *)a.status;
     so.T = a.tile_size;
     so.chunk_pairs = (SR_GLOBAL uint32_t *)a.chunk_pairs;
-    if (a.total_in > 0) {
-        SR_LAUNCH_TIMED(ev_none, a.events[1], k_setup, dim3(grid_for(a.total_in, 256, GRID_CAP)), dim3(256), st,
+    so.matrix = (SR_GLOBAL uint32_t *)a.sort_hist;
+    so.chunk_first = (SR_GLOBAL uint32_t *)a.chunk_pairs;
+    so.items = a.total_items;
+    so.nchunks = nchunks;
+    if (a.direct) {
+        SR_LAUNCH_TIMED_LDS(ev_none, a.events[1], k_setup<true>, dim3(nchunks), dim3(256), a.total_items * 4u, st,
+                            a.views, a.draws, a.num_draws, a.total_in, a.xv + 3 * (size_t)a.total_xv, a.tri_counts,
+                            a.tri_chunks, a.clip_buf, a.tri_base, so);
+    } else if (a.total_in > 0) {
+        SR_LAUNCH_TIMED(ev_none, a.events[1], k_setup<false>, dim3(grid_for(a.total_in, 256, GRID_CAP)), dim3(256), st,
                         a.views, a.draws, a.num_draws, a.total_in, a.xv + 3 * (size_t)a.total_xv, a.tri_counts,
                         a.tri_chunks, a.clip_buf, a.tri_base, so);
     } else if (a.events[1]) {
@@ -3723,7 +3965,28 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     const int npass = bin_sort_passes(a.total_items);
     if (npass < 1) return hipErrorInvalidValue;
     const int nbits = bin_sort_bits(a.total_items);
-    if (a.total_in > 0) {
+    if (a.direct) {
+        BinDirect bd;
+        bd.views = (const SR_GLOBAL DevView *)a.views;
+        bd.geo = (const SR_GLOBAL uint4 *)a.rec_geo;
+        bd.chunk_first = (const SR_GLOBAL uint32_t *)a.chunk_pairs;
+        bd.matrix = (SR_GLOBAL uint32_t *)a.sort_hist;
+        bd.list = (SR_GLOBAL uint32_t *)a.list;
+        bd.bin_start = (SR_GLOBAL uint32_t *)a.bin_start;
+        bd.bin_end = (SR_GLOBAL uint32_t *)a.bin_end;
+        bd.status = (SR_GLOBAL DevStatus *)a.status;
+        bd.stamp = setup_end;
+        bd.nchunks = nchunks;
+        bd.items = a.total_items;
+        bd.rec_cap = a.rec_cap;
+        bd.pair_cap = a.pair_cap;
+        bd.T = a.tile_size;
+        bd.bits = nbits;
+        hipLaunchKernelGGL(k_bin_cols, dim3((a.total_items + DB_COL_TILES - 1u) / DB_COL_TILES), dim3(1024), 0, st, bd);
+        hipLaunchKernelGGL(k_bin_place, dim3(nchunks), dim3(256), a.total_items * 4u, st, bd);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    } else if (a.total_in > 0) {
         if (nchunks <= SCAN_SINGLE_MAX) {
             ScanJobs J;
             J.job[0] = scan_job(a.chunk_pairs, nchunks, a.chunk_pairs, nullptr, &a.sort->chunk_total,

@@ -130,12 +130,27 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
     uint32_t rec_cap =
         (uint32_t)std::min<uint64_t>(std::min<uint64_t>(rec_want, rest * 4 / 5 / rec_bytes), 0xFFFFFFF0ull);
     uint32_t pair_cap = (uint32_t)std::min<uint64_t>((rest - (uint64_t)rec_cap * rec_bytes) / pair_bytes, 0xFFFFFFF0ull);
+    // a small frame's direct binning needs its count matrix instead of the
+    // pairs' arrays: taken where that holds no fewer records and entries
+    bool direct = false;
+    const uint64_t matrix = (uint64_t)bin_matrix_entries(total_in, items) * 4;
+    if (matrix > 0 && matrix + 256 < rest) {
+        const uint64_t left = rest - matrix - 256;
+        const uint64_t rc = std::min<uint64_t>(rec_want, left * 4 / 5 / rec_bytes);
+        const uint64_t pc = std::min<uint64_t>((left - rc * rec_bytes) / 4, 0xFFFFFFF0ull);
+        direct = rc >= rec_cap && pc >= pair_cap;
+        if (direct) {
+            rec_cap = (uint32_t)std::min<uint64_t>(rc, 0xFFFFFFF0ull);
+            pair_cap = (uint32_t)pc;
+        }
+    }
     uint64_t o_geo = c.take((uint64_t)rec_cap * 16);
     uint64_t o_ras = c.take((uint64_t)rec_cap * 64);
     uint64_t o_list = c.take((uint64_t)pair_cap * 4);
     uint64_t o_pairs[4] = {0, 0, 0, 0};
-    for (int k = 0; k < (sort_passes > 1 ? 4 : 3); k++) o_pairs[k] = c.take((uint64_t)pair_cap * 4);
-    uint64_t o_hist = c.take((uint64_t)bin_sort_tiles(pair_cap) * 256 * 4);
+    if (!direct)
+        for (int k = 0; k < (sort_passes > 1 ? 4 : 3); k++) o_pairs[k] = c.take((uint64_t)pair_cap * 4);
+    uint64_t o_hist = c.take(direct ? matrix : (uint64_t)bin_sort_tiles(pair_cap) * 256 * 4);
     if (c.used > cap) return fail(SR_ERR_CAPACITY, "scratch layout exceeds %llu bytes", (unsigned long long)cap);
 
     // view and draw tables and the zeroed status: one upload
@@ -169,6 +184,7 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
     a.pair_vals = (uint32_t *)(base + o_pairs[1]);
     a.pair_keys2 = (uint32_t *)(base + o_pairs[2]);
     if (sort_passes > 1) a.pair_vals2 = (uint32_t *)(base + o_pairs[3]);
+    a.direct = direct ? 1 : 0;
     a.sort_hist = (uint32_t *)(base + o_hist);
     a.chunk_pairs = (uint32_t *)(base + o_chunk_pairs);
     a.rec_geo = (uint4 *)(base + o_geo);

@@ -238,7 +238,7 @@ int Pipeline::launch_graph(const FrameArgs &a, size_t vbytes, size_t upload) {
     k.n[0] = (uint64_t)a.num_views; k.n[1] = (uint64_t)a.num_draws; k.n[2] = a.total_xv; k.n[3] = a.total_in;
     k.n[4] = a.total_items; k.n[5] = (uint64_t)a.tile_size; k.n[6] = (uint64_t)a.any_tangents; k.n[7] = a.rec_cap;
     k.n[8] = a.pair_cap; k.n[9] = a.clip_cap; k.n[10] = (uint64_t)a.persistent_blocks; k.n[11] = vbytes;
-    k.n[12] = upload; k.n[13] = a.color_plane; k.n[14] = (uint64_t)a.has_translucent;
+    k.n[12] = upload; k.n[13] = a.color_plane; k.n[14] = (uint64_t)a.has_translucent | ((uint64_t)a.direct << 1);
     k.n[15] = ((uint64_t)a.tr_cap << 32) | a.tr_slots | ((uint64_t)a.overdraw << 31);
     const void *ptrs[] = {a.views, a.draws, a.xv, a.xt, a.tri_counts, a.tri_chunks, a.tri_base, a.bin_start, a.bin_end,
                           a.scan_partials, a.list, a.rec_geo, a.rec_raster, a.clip_queue, a.clip_buf, a.status,
@@ -315,7 +315,12 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
     if (rec_cap < total_in + total_in / 8 + 1024) rec_cap = total_in + total_in / 8 + 1024;
     if (pair_cap < rec_cap * 2) pair_cap = rec_cap * 2;
     if (clip_cap < 4096) clip_cap = 4096;
+    // direct binning for small frames, unless the last frame's triangles
+    // spanned more than eight tiles each on average: one workgroup ranks a
+    // chunk's pairs, 1024 at a time, where the expansion takes up to eight
+    const size_t matrix = bin_matrix_entries(total_in, total_items);
     for (int attempt = 0; attempt < 4; attempt++) {
+        const bool direct = matrix > 0 && last_pairs <= 8ull * std::max<uint32_t>(last_records, 1u);
         // every attempt is a frame of its own number
         DevStatus init;
         memset(&init, 0, sizeof(init));
@@ -326,11 +331,15 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
         if ((r = list.ensure((size_t)pair_cap * 4))) return r;
         if ((r = clip_queue.ensure((size_t)clip_cap * 4))) return r;
         if ((r = clip_buf.ensure((size_t)clip_cap * 16 * 16 * 4))) return r;
-        if ((r = pair_keys.ensure((size_t)pair_cap * 4)) || (r = pair_vals.ensure((size_t)pair_cap * 4))) return r;
-        // (the last pass writes its bins to the key array it does not read)
-        if ((r = pair_keys2.ensure((size_t)pair_cap * 4))) return r;
-        if (sort_passes > 1 && (r = pair_vals2.ensure((size_t)pair_cap * 4))) return r;
-        if ((r = sort_hist.ensure((size_t)bin_sort_tiles(pair_cap) * 256 * 4))) return r;
+        if (direct) {
+            if ((r = sort_hist.ensure(matrix * 4))) return r;
+        } else {
+            if ((r = pair_keys.ensure((size_t)pair_cap * 4)) || (r = pair_vals.ensure((size_t)pair_cap * 4))) return r;
+            // (the last pass writes its bins to the key array it does not read)
+            if ((r = pair_keys2.ensure((size_t)pair_cap * 4))) return r;
+            if (sort_passes > 1 && (r = pair_vals2.ensure((size_t)pair_cap * 4))) return r;
+            if ((r = sort_hist.ensure((size_t)bin_sort_tiles(pair_cap) * 256 * 4))) return r;
+        }
         if (has_tr && (r = tr_list.ensure((size_t)tr_cap * 4))) return r;
         if (has_tr && (r = tr_scratch.ensure((size_t)tr_cap * 20))) return r;
         FrameArgs a;
@@ -391,6 +400,7 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
             a.center_color = (float4 *)center_color.ptr;
         }
         a.persistent_blocks = persistent_blocks;
+        a.direct = direct ? 1 : 0;
         // depth order pays where triangles span many tiles and tiles hold
         // many of them (high overdraw); judged from the last frame
         a.overdraw = tile_size == 16 && last_pairs > 32ull * total_items && last_pairs > 4ull * last_records;

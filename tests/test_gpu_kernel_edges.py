@@ -179,3 +179,63 @@ def test_overdraw_raster_list_lengths(sr, orc, n, kind):
         assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32)), f"frame {k}"
     assert r.stats()["depth_rejection"] == 1
     r.close()
+
+
+def _with_backfacing(sr, scene, n):
+    """scene plus a last primitive of n copies of one backfacing triangle in
+    every mesh-bearing node's place: they make records without bins, so the
+    tiles' lists stay the same while the frame has n more triangles."""
+    import copy
+    prims = [dict(p) for p in scene.primitives]
+    tri = np.array([[0.0, 0.0, 0.0], [0.0, 1e-3, 0.0], [1e-3, 0.0, 0.0]], np.float32)
+    prims.append({"positions": tri, "normals": np.tile(np.float32([0, 0, 1]), (3, 1)), "texcoords": None,
+                  "tangents": None, "indices": np.tile(np.arange(3, dtype=np.uint32), n), "material": 0})
+    first, count = scene.meshes[-1]
+    assert first + count == len(prims) - 1
+    meshes = list(scene.meshes[:-1]) + [(first, count + 1)]
+    out = sr.SceneData(prims, meshes, list(scene.nodes), copy.deepcopy(scene.materials), list(scene.textures))
+    return out
+
+
+# small frames by direct binning against the same frames by radix passes,
+# which 262,144 more triangles (1024 chunks) make them take: tile counts of
+# one, a few and exactly 8192, sizes that leave tiles off screen, all tile
+# sizes; "near" stands close to the terrain, so many triangles cross the
+# frustum, "big" has rectangles of more than 32 tiles
+@pytest.mark.parametrize("kind,W,H,tile", [("cluster", 16, 16, 32), ("cluster", 64, 64, 16), ("cluster", 333, 202, 8),
+                                           ("cluster", 2048, 1024, 16), ("near", 640, 360, 16), ("near", 500, 301, 32),
+                                           ("big", 640, 480, 16), ("big", 1023, 130, 8)])
+def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
+    """The tiles' lists, the visibility buffer and the pair count of a small
+    frame are those that the radix passes give."""
+    if kind == "cluster":
+        scene, spec = scenes.make_c1(width=W, height=H)
+        # one node: all spheres in world space, so the copies come last
+        prims = []
+        for (t, m) in scene.nodes:
+            p = dict(scene.primitives[m])
+            p["positions"] = (p["positions"] @ np.asarray(t, np.float32)[:3, :3].T + np.asarray(t, np.float32)[:3, 3])
+            prims.append(p)
+        scene = sr.SceneData(prims, [(0, len(prims))], [(np.eye(4, dtype=np.float32), 0)], scene.materials,
+                             scene.textures)
+    elif kind == "near":
+        scene, spec = scenes.make_c2(width=W, height=H, grid=120, tex_size=64)
+        spec["position"] = [0.0, 4.0, 10.0]
+    else:
+        scene, spec = scenes.make_c3(width=W, height=H, triangles=900, primitives=7)
+    more = _with_backfacing(sr, scene, 262144)
+    scene.prepare(env, grid=16)
+    more.attach(scene.environment, scene.voxels)
+    cam = scenes.make_camera(spec, W, H)
+    out = []
+    for data in (scene, more):
+        r = sr.Renderer(W, H, tile_size=tile)
+        gscene = sr.Scene(data)
+        r.render_scene(gscene, cam)
+        ids, depth = r.read_vbuffer()
+        out.append((ids, depth.view(np.uint32), *r.read_bins(), r.stats()["binned_pairs"]))
+        r.close()
+    assert out[0][5] == out[1][5] and out[0][5] > 0
+    for a, b in zip(out[0][:5], out[1][:5]):
+        assert np.array_equal(a, b)
+    assert np.all(np.diff(out[0][2].astype(np.int64)) >= 0) and out[0][3][-1] == out[0][5]
