@@ -64,8 +64,8 @@ struct GiScene {
 #define GI_STACK 48          // traversal stack entries; the BVH is at most 44 levels deep
 #define GI_HIT_CAP 32
 
-// Traversal stack in a private array (host).  The device keeps its stacks
-// in LDS with the same interface and capacity, so both walk identically.
+// Traversal stack in a private array (host).  The device walks a copy of the
+// tree in the same order (gi.hip).
 struct GiLocalStack {
     int32_t s[GI_STACK];
     int n = 0;
@@ -292,56 +292,60 @@ struct GiRayParams {
     float hit_bias, tmin;
 };
 
-// sky_visibility_hemisphere4 (src/gi.rs:549-570)
-template <class Stack>
-GI_HD float gi_sky_visibility(const GiScene &S, G3 origin, G3 normal, float dir_bias, float tmin, bool &over,
-                              Stack &st) {
+// Direction k of sky_visibility_hemisphere4 (src/gi.rs:549-570).
+GI_HD G3 gi_sky_dir(G3 normal, int k) {
     G3 up = fabsf(normal.z) < 0.999f ? g3(0.0f, 0.0f, 1.0f) : g3(1.0f, 0.0f, 0.0f);
     G3 tangent = gnormalize(gcross(normal, up));
     G3 bitangent = gcross(normal, tangent);
     const float dl[4][3] = {{0.0f, 0.0f, 1.0f}, {0.8660254f, 0.0f, 0.5f}, {-0.4330127f, 0.75f, 0.5f},
                             {-0.4330127f, -0.75f, 0.5f}};
+    return gnormalize(gadd(gadd(gscale(tangent, dl[k][0]), gscale(bitangent, dl[k][1])), gscale(normal, dl[k][2])));
+}
+
+// sky_visibility_hemisphere4 (src/gi.rs:549-570)
+template <class Stack>
+GI_HD float gi_sky_visibility(const GiScene &S, G3 origin, G3 normal, float dir_bias, float tmin, bool &over,
+                              Stack &st) {
     float vis = 0.0f;
     for (int k = 0; k < 4; k++) {
-        G3 dir = gnormalize(gadd(gadd(gscale(tangent, dl[k][0]), gscale(bitangent, dl[k][1])), gscale(normal, dl[k][2])));
+        G3 dir = gi_sky_dir(normal, k);
         G3 o = gadd(origin, gscale(dir, dir_bias));
         vis += gi_trace_transmittance(S, o, dir, tmin, over, st);
     }
     return vis * 0.25f;
 }
 
-// estimate_surface_bounce_radiance (src/gi.rs:450-547)
-template <class Stack>
-GI_HD G3 gi_bounce(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const GiRayParams &P, bool &over,
-                   Stack &st) {
+// estimate_surface_bounce_radiance (src/gi.rs:450-547) up to its rays: the
+// normal facing the ray, the material's albedo and emission, and the rays'
+// origin; false if the surface neither reflects nor emits.
+GI_HD bool gi_bounce_surface(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const GiRayParams &P, G3 &normal,
+                             G3 &albedo, G3 &emissive, G3 &shading_origin) {
     const GiTri &tri = S.tris[hit.tri];
     int32_t mi = (tri.material >= 0 && tri.material < S.nmat) ? tri.material : 0;
     const GiMat &M = S.mats[mi];
-    G3 normal = g3(tri.n[0], tri.n[1], tri.n[2]);
+    normal = g3(tri.n[0], tri.n[1], tri.n[2]);
     if (gdot(normal, gscale(incoming, -1.0f)) < 0.0f) normal = gscale(normal, -1.0f);
     float w = (1.0f - hit.u) - hit.v;
     float uvx = (tri.uv[0] * w + tri.uv[2] * hit.u) + tri.uv[4] * hit.v;
     float uvy = (tri.uv[1] * w + tri.uv[3] * hit.u) + tri.uv[5] * hit.v;
-    G3 emissive = g3(M.emissive[0], M.emissive[1], M.emissive[2]);
+    emissive = g3(M.emissive[0], M.emissive[1], M.emissive[2]);
     if (M.emis_tex >= 0) emissive = gmul(emissive, gi_sample_bilinear_srgb(S, M.emis_tex, M.emis_ws, M.emis_wt, uvx, uvy));
     emissive = gmax0(emissive);
-    G3 albedo = g3(M.base[0], M.base[1], M.base[2]);
+    albedo = g3(M.base[0], M.base[1], M.base[2]);
     if (M.base_tex >= 0) albedo = gmul(albedo, gi_sample_bilinear_srgb(S, M.base_tex, M.base_ws, M.base_wt, uvx, uvy));
     albedo = g3(gminf(gmaxf(albedo.x, 0.0f), 1.0f), gminf(gmaxf(albedo.y, 0.0f), 1.0f), gminf(gmaxf(albedo.z, 0.0f), 1.0f));
     albedo = gscale(albedo, 1.0f);
-    if (gdot(albedo, albedo) <= 0.0f && gdot(emissive, emissive) <= 0.0f) return g3(0.0f, 0.0f, 0.0f);
-    float dir_bias = P.hit_bias * 0.5f;
+    if (gdot(albedo, albedo) <= 0.0f && gdot(emissive, emissive) <= 0.0f) return false;
     G3 position = gadd(o, gscale(incoming, hit.t));
-    G3 shading_origin = gadd(position, gscale(normal, P.hit_bias));
-    G3 L = g3(S.light_dir[0], S.light_dir[1], S.light_dir[2]);
-    float ndl = gmaxf(gdot(normal, L), 0.0f);
+    shading_origin = gadd(position, gscale(normal, P.hit_bias));
+    return true;
+}
+
+// The rest of it: the radiance from the cosine to the sun, the sun's
+// visibility (read if the cosine is positive) and the sky's.
+GI_HD G3 gi_bounce_finish(const GiScene &S, G3 normal, G3 albedo, G3 emissive, float ndl, float vis, float sky) {
     G3 e_sun = g3(0.0f, 0.0f, 0.0f);
-    if (ndl > 0.0f) {
-        G3 so = gadd(shading_origin, gscale(L, dir_bias));
-        float vis = gi_trace_transmittance(S, so, L, P.tmin, over, st);
-        e_sun = gscale(g3(S.light_color[0], S.light_color[1], S.light_color[2]), ndl * vis);
-    }
-    float sky = gi_sky_visibility(S, shading_origin, normal, dir_bias, P.tmin, over, st);
+    if (ndl > 0.0f) e_sun = gscale(g3(S.light_color[0], S.light_color[1], S.light_color[2]), ndl * vis);
     G3 irr;
     irr.x = ((S.sh[0][0] + S.sh[1][0] * normal.y) + S.sh[2][0] * normal.z) + S.sh[3][0] * normal.x;
     irr.y = ((S.sh[0][1] + S.sh[1][1] * normal.y) + S.sh[2][1] * normal.z) + S.sh[3][1] * normal.x;
@@ -352,6 +356,23 @@ GI_HD G3 gi_bounce(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const 
     G3 bounce = g3(0.0f, 0.0f, 0.0f);
     if (gdot(e_total, e_total) > 0.0f) bounce = gmul(albedo, g3(e_total.x / PI_F, e_total.y / PI_F, e_total.z / PI_F));
     return gadd(bounce, emissive);
+}
+
+// estimate_surface_bounce_radiance (src/gi.rs:450-547)
+template <class Stack>
+GI_HD G3 gi_bounce(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const GiRayParams &P, bool &over,
+                   Stack &st) {
+    G3 normal, albedo, emissive, shading_origin;
+    if (!gi_bounce_surface(S, hit, o, incoming, P, normal, albedo, emissive, shading_origin)) return g3(0.0f, 0.0f, 0.0f);
+    float dir_bias = P.hit_bias * 0.5f;
+    G3 L = g3(S.light_dir[0], S.light_dir[1], S.light_dir[2]);
+    float ndl = gmaxf(gdot(normal, L), 0.0f), vis = 0.0f;
+    if (ndl > 0.0f) {
+        G3 so = gadd(shading_origin, gscale(L, dir_bias));
+        vis = gi_trace_transmittance(S, so, L, P.tmin, over, st);
+    }
+    float sky = gi_sky_visibility(S, shading_origin, normal, dir_bias, P.tmin, over, st);
+    return gi_bounce_finish(S, normal, albedo, emissive, ndl, vis, sky);
 }
 
 // Incident radiance along primary direction dir from the voxel centre

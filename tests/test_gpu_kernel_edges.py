@@ -239,3 +239,36 @@ def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
     for a, b in zip(out[0][:5], out[1][:5]):
         assert np.array_equal(a, b)
     assert np.all(np.diff(out[0][2].astype(np.int64)) >= 0) and out[0][3][-1] == out[0][5]
+
+
+def _gi(sr, scene, env, grid, device):
+    g = sr.sr_voxel_grid()
+    scene.environment = env
+    scene.desc.environment = sr.C.pointer(env.desc)
+    sr.check(sr.lib().sr_prepare_gi(sr.C.byref(scene.desc), grid, device, 8, sr.C.byref(g)))
+    sh4 = np.ctypeslib.as_array(g.sh4, shape=(grid ** 3 * 16,)).copy()
+    sr.lib().sr_voxel_grid_free(sr.C.byref(g))
+    return sh4.view(np.uint32)
+
+
+# a tree whose root is a leaf (up to four triangles), one inner node, a few
+# levels; grids whose active voxels leave waves of the last workgroup empty;
+# the translucent variant with rays through many layers
+@pytest.mark.parametrize("n,grid,glass", [(1, 5, False), (4, 9, False), (5, 9, False), (9, 7, True), (40, 13, False),
+                                          (40, 13, True), (700, 16, True)])
+def test_gi_tree_sizes(sr, scenes, env, n, grid, glass):
+    """The device GI bake over trees of 1 to 700 triangles equals the host
+    bake bit for bit."""
+    rng = np.random.Generator(np.random.PCG64(n))
+    pos = (rng.uniform(-2, 2, (n, 1, 3)) + rng.normal(0, 0.8, (n, 3, 3))).astype(np.float32).reshape(-1, 3)
+    half = 3 * (n // 2)
+    prims, mats = [], []
+    for k, (a, b) in enumerate(((0, half), (half, 3 * n))):
+        if a == b:
+            continue
+        prims.append({"positions": pos[a:b], "normals": np.tile(np.float32([0, 0, 1]), (b - a, 1)), "texcoords": None,
+                      "tangents": None, "indices": np.arange(b - a, dtype=np.uint32), "material": len(mats)})
+        mats.append({"base_color": (0.8, 0.5, 0.3, 1.0), "metallic": 0.0, "roughness": 0.5,
+                     "emissive": (0.2 * k, 0.1, 0.0), "is_translucent": int(glass and k == 0), "transmission": 0.6})
+    scene = sr.SceneData(prims, [(0, len(prims))], [(np.eye(4, dtype=np.float32), 0)], mats, [], name=f"gi_{n}")
+    assert np.array_equal(_gi(sr, scene, env, grid, 0), _gi(sr, scene, env, grid, -1))
