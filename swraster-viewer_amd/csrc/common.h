@@ -94,6 +94,7 @@ struct DevScene {
     int32_t vox_dims[3];
     float vox_min[3];
     float vox_size[3];            // (max - min) / dims, as src/voxelgrid.rs:154-161
+    float vox_rcp[3];             // 1 / vox_size, or 0 where a size is not within 2^+-40
     float sh_const[4][4];         // constant-SH coefficients (w of [1] = sky)
     float light_dir[3];
     float light_color[3];

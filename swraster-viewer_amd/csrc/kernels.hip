@@ -78,7 +78,31 @@ __device__ __forceinline__ uint32_t sat_index(float f, uint32_t limit) {
     uint32_t v = (uint32_t)f;
     return v < limit ? v : limit;
 }
-__device__ __forceinline__ float rsqrt_ieee(float x) { return 1.0f / sqrtf(x); }
+// Divisions and square roots with fewer instructions than the compiler's (which
+// scale their operands and fix up every special case), for operands known to
+// be in range: each gives the IEEE result.  Checked against IEEE division and
+// square root on gfx950 for every float in [2^-96, 2^96] (the reciprocal, the
+// root, and both in turn) and for 1.7e10 random pairs with exponents within
+// +-40 (the quotient: with the correctly rounded reciprocal of b, one fused
+// correction of a rcp(b) by its exact residual rounds correctly).
+__device__ __forceinline__ float rcp_in_range(float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+// a / b from y = rcp(b), correctly rounded.
+__device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
+    float q = a * y;
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+__device__ __forceinline__ float div_in_range(float a, float b) { return div_by_rcp(a, b, rcp_in_range(b)); }
+// SHORT: with the short forms where x is in range.
+template <bool SHORT = true> __device__ __forceinline__ float rsqrt_ieee(float x) {
+    if (SHORT && x >= 0x1p-96f && x <= 0x1p96f) {
+        float y = __builtin_amdgcn_rsqf(x), g = x * y;
+        return rcp_in_range(fmaf(fmaf(-g, g, x), 0.5f * y, g));
+    }
+    return 1.0f / sqrtf(x);
+}
 
 struct f3 { float x, y, z; };
 __device__ __forceinline__ f3 mk3(float x, float y, float z) { return {x, y, z}; }
@@ -88,8 +112,8 @@ __device__ __forceinline__ f3 mul3(f3 a, f3 b) { return {a.x * b.x, a.y * b.y, a
 __device__ __forceinline__ f3 muls(f3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
 __device__ __forceinline__ f3 adds(f3 a, float s) { return {a.x + s, a.y + s, a.z + s}; }
 __device__ __forceinline__ float dot3(f3 a, f3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
-__device__ __forceinline__ f3 normalize3(f3 a) {
-    float r = rsqrt_ieee(dot3(a, a));
+template <bool SHORT = true> __device__ __forceinline__ f3 normalize3(f3 a) {
+    float r = rsqrt_ieee<SHORT>(dot3(a, a));
     return {a.x * r, a.y * r, a.z * r};
 }
 __device__ __forceinline__ f3 cross3(f3 a, f3 b) {
@@ -1840,8 +1864,17 @@ __device__ __forceinline__ void cube_uv(f3 n, float &uf, float &vf, uint32_t &sl
     float v = mx ? v_x : (my ? v_y : v_z);
     float den = mx ? d_x : (my ? d_y : d_z);
     den = maxps(den, 1.0e-19f);
-    uf = 0.5f * (u / den + 1.0f);
-    vf = 0.5f * (v / den + 1.0f);
+    float qu, qv;
+    if (den <= 0x1p40f) {       // (a quotient too small for its residual adds nothing to 1)
+        float y = rcp_in_range(den);
+        qu = div_by_rcp(u, den, y);
+        qv = div_by_rcp(v, den, y);
+    } else {
+        qu = u / den;
+        qv = v / den;
+    }
+    uf = 0.5f * (qu + 1.0f);
+    vf = 0.5f * (qv + 1.0f);
     float ix = n.x >= 0.0f ? 0.0f : 1.0f;
     float iy = n.y >= 0.0f ? 2.0f : 3.0f;
     float iz = n.z >= 0.0f ? 4.0f : 5.0f;
@@ -1871,9 +1904,16 @@ __device__ __forceinline__ float tri_const(float k, float fx, float fy, float fz
 }
 
 __device__ __forceinline__ void voxel_lookup(const DevScene &S, f3 p, f3 rgb[4], float &w0, float &w1) {
-    float vx = (p.x - S.vox_min[0]) / S.vox_size[0];
-    float vy = (p.y - S.vox_min[1]) / S.vox_size[1];
-    float vz = (p.z - S.vox_min[2]) / S.vox_size[2];
+    float vx = p.x - S.vox_min[0], vy = p.y - S.vox_min[1], vz = p.z - S.vox_min[2];
+    if (S.vox_rcp[0] > 0.0f) {
+        vx = div_by_rcp(vx, S.vox_size[0], S.vox_rcp[0]);
+        vy = div_by_rcp(vy, S.vox_size[1], S.vox_rcp[1]);
+        vz = div_by_rcp(vz, S.vox_size[2], S.vox_rcp[2]);
+    } else {
+        vx = vx / S.vox_size[0];
+        vy = vy / S.vox_size[1];
+        vz = vz / S.vox_size[2];
+    }
     float x0f = floorf(vx), y0f = floorf(vy), z0f = floorf(vz);
     uint32_t W = (uint32_t)S.vox_dims[0], H = (uint32_t)S.vox_dims[1], D = (uint32_t)S.vox_dims[2];
     uint32_t x0 = sat_index(x0f, W - 1), y0 = sat_index(y0f, H - 1), z0 = sat_index(z0f, D - 1);
@@ -1927,7 +1967,10 @@ __device__ __forceinline__ void voxel_lookup(const DevScene &S, f3 p, f3 rgb[4],
 // ---------------------------------------------------------------------------
 // PBR shading of one pixel (pbr_shader, src/shader.rs:110-309)
 // b1[4], b2[4]: the quad's four barycentric pairs; lane: this pixel's lane.
-// TR: the translucent form, which blends over cur (src/shader.rs:66-76).
+// TR: the translucent form, which blends over cur (src/shader.rs:66-76); it
+// keeps the compiler's roots and BRDF divisions, since the short forms' branches
+// cost k_translucent 7 more spilled registers (72 -> 77 us) where they take 5%
+// off k_shade.
 // ---------------------------------------------------------------------------
 // The quad's four w = 1 / interpolated 1/w of this pixel's triangle at each
 // lane's barycentrics (src/shader.rs:123-130: du_dv takes all four lanes'
@@ -1949,33 +1992,33 @@ __device__ __forceinline__ f3 shade_pixel(const DevScene &S, const DevView &V, i
     f3 na = mk3(s0.x, s0.y, s0.z), nda = mk3(s0.w, s1.x, s1.y), ndb = mk3(s1.z, s1.w, s2.x);
     f3 pa = mk3(s2.y, s2.z, s2.w), pda = mk3(s3.x, s3.y, s3.z), pdb = mk3(s3.w, s4.x, s4.y);
     f3 in_n = mk3((na.x + B1 * nda.x) + B2 * ndb.x, (na.y + B1 * nda.y) + B2 * ndb.y, (na.z + B1 * nda.z) + B2 * ndb.z);
-    in_n = normalize3(in_n);
+    in_n = normalize3<!TR>(in_n);
     f3 pos = mk3(((pa.x + B1 * pda.x) + B2 * pdb.x) * w, ((pa.y + B1 * pda.y) + B2 * pdb.y) * w,
                  ((pa.z + B1 * pda.z) + B2 * pdb.z) * w);
     float uvx = ((s4.z + B1 * s4.w) + B2 * s5.x) * w;
     float uvy = ((s5.y + B1 * s5.z) + B2 * s5.w) * w;
     float dd[4] = {s6.x * wv[0], s6.y * wv[1], s6.z * wv[2], s6.w * wv[3]};
-    f3 nw = normalize3(in_n);
+    f3 nw = normalize3<!TR>(in_n);
     if ((M.flags & SR_MAT_NORMAL_MAP) && nmap) {
         float4 t0 = Tn[0], t1 = Tn[1], t2 = Tn[2];
         f3 ta = mk3(t0.x, t0.y, t0.z), tda = mk3(t0.w, t1.x, t1.y), tdb = mk3(t1.z, t1.w, t2.x);
         f3 in_t = mk3((ta.x + B1 * tda.x) + B2 * tdb.x, (ta.y + B1 * tda.y) + B2 * tdb.y, (ta.z + B1 * tda.z) + B2 * tdb.z);
-        in_t = normalize3(in_t);
+        in_t = normalize3<!TR>(in_t);
         float tsign = (t2.y + B1 * t2.z) + B2 * t2.w;
-        f3 tw = normalize3(sub3(in_t, muls(in_n, dot3(in_n, in_t))));
+        f3 tw = normalize3<!TR>(sub3(in_t, muls(in_n, dot3(in_n, in_t))));
         float hand = tsign >= 0.0f ? 1.0f : -1.0f;
         f3 bw = muls(cross3(in_n, tw), hand);
         f3 tsn = unpack_rgb(texel_nearest(S, M.normal_tex, uvx, uvy, dd));
         tsn = mk3(tsn.x * 2.0f - 1.0f, tsn.y * 2.0f - 1.0f, tsn.z * 2.0f - 1.0f);
         nw = add3(add3(muls(tw, tsn.x), muls(bw, tsn.y)), muls(in_n, tsn.z));
-        nw = normalize3(nw);
+        nw = normalize3<!TR>(nw);
     }
     f3 L = mk3(S.light_dir[0], S.light_dir[1], S.light_dir[2]);
     f3 LC = mk3(S.light_color[0], S.light_color[1], S.light_color[2]);
     f3 vdir = sub3(mk3(V.cam_pos[0], V.cam_pos[1], V.cam_pos[2]), pos);
-    f3 vn = normalize3(vdir);
+    f3 vn = normalize3<!TR>(vdir);
     float ndl = maxps(dot3(nw, L), 0.0f);
-    f3 hv = normalize3(add3(L, vn));
+    f3 hv = normalize3<!TR>(add3(L, vn));
     float ndh = maxps(dot3(nw, hv), 0.0f);
     float ndv = maxps(dot3(nw, vn), 1.0e-4f);
     float vdh = maxps(dot3(vn, hv), 0.0f);
@@ -2019,13 +2062,20 @@ __device__ __forceinline__ f3 shade_pixel(const DevScene &S, const DevView &V, i
     float alpha2 = alpha * alpha;
     float ndh2 = ndh * ndh;
     float dden = ndh2 * (alpha2 - 1.0f) + 1.0f;
-    float brdf_d = alpha2 / (PI * (dden * dden) + EPS);
     float k = rough + 1.0f;
     k = (k * k) * 0.125f;
-    float gv = ndv / ((ndv * (1.0f - k) + k) + EPS);
-    float gl = ndl / ((ndl * (1.0f - k) + k) + EPS);
-    float brdf_g = gv * gl;
-    float sdg = (brdf_d * brdf_g) / ((4.0f * ndl) * ndv + EPS);
+    float den_d = PI * (dden * dden) + EPS, den_v = (ndv * (1.0f - k) + k) + EPS, den_l = (ndl * (1.0f - k) + k) + EPS;
+    float den_s = (4.0f * ndl) * ndv + EPS;
+    float sdg;
+    // roughness is at least 0.045 and N.V at least 1e-4, and all cosines are
+    // about 1 at most, so only N.L can take an operand out of range
+    if (!TR && (ndl == 0.0f || ndl >= 0x1p-40f) && fmaxf(fmaxf(ndl, ndv), ndh2) <= 2.0f) {
+        float brdf_g = div_in_range(ndv, den_v) * div_in_range(ndl, den_l);
+        sdg = div_in_range(div_in_range(alpha2, den_d) * brdf_g, den_s);
+    } else {
+        float brdf_g = (ndv / den_v) * (ndl / den_l);
+        sdg = ((alpha2 / den_d) * brdf_g) / den_s;
+    }
     float om = 1.0f - metal;
     f3 kdd = mk3((1.0f - bf.x) * om, (1.0f - bf.y) * om, (1.0f - bf.z) * om);
     const float INV_PI = 1.0f / 3.14159265358979323846f;
@@ -2157,7 +2207,9 @@ enum {
 // equal 32 A and 32 B exactly unless 32 a wraps (|a| >= 2^26), which the
 // entry's STEP_WRAP flag marks and walk_quad then recomputes.
 #define STEP_WRAP 4u
-// F_FLAGS: coarse 1, alpha 2, STEP_WRAP; from bit 3 and 28 the first quad's
+// The entry's 1/w at its covered samples is in range for rcp_in_range.
+#define W_IN_RANGE 0x80u
+// F_FLAGS: coarse 1, alpha 2, STEP_WRAP, W_IN_RANGE; from bit 3 and 28 the first quad's
 // column and row in the tile; from bit 8 the rejected blocks, from 20 and 24
 // the first block.  After F_ROWS: inclusive quad counts per quad row (bytes up
 // to 16-px tiles, whose entries have at most 64 quads, else u16 pairs), then
@@ -2172,6 +2224,16 @@ template <int T> struct Stage {
     static constexpr int LO = CUM + (BYTES ? NR / 4 : NR / 2);
     static constexpr int COUNT = LO + (NR + 7) / 8;
 };
+
+// Whether the interpolated 1/w, (oa + b1 oda) + b2 odb, stays within 2^+-60
+// (or little beyond) at covered samples: b1, b2 >= 0 and b1 + b2 <= 1 to
+// within 4e-7 keep it between the vertices' values, which differ by a factor
+// of 2^16 at most, to a few percent of the smallest.
+__device__ __forceinline__ bool w_in_range(float oa, float oda, float odb) {
+    float d1 = oa + oda, d2 = oa + odb;
+    float lo = fminf(oa, fminf(d1, d2)), hi = fmaxf(oa, fmaxf(d1, d2));
+    return oa == oa && d1 == d1 && d2 == d2 && lo >= 0x1p-60f && hi <= 0x1p60f && hi <= 65536.0f * lo;
+}
 
 // f32 corner test of the 16px block at (bx, by) (src/tilerasterizer.rs:258-291)
 __device__ __forceinline__ bool block_out(const TriSetup &ts, int bx, int by) {
@@ -2238,7 +2300,8 @@ __device__ __forceinline__ int stage_entry(const TriSetup &ts, uint32_t id, uint
     st[F_ORG * SW + lane] = (uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16);
 
     // rejected 16px blocks among the (at most 3x3) that meet the tile
-    uint32_t flags = (ts.coarse ? 1u : 0u) | ((gflags & SR_GEO_ALPHA) ? 2u : 0u) | (wrap ? STEP_WRAP : 0u);
+    uint32_t flags = (ts.coarse ? 1u : 0u) | ((gflags & SR_GEO_ALPHA) ? 2u : 0u) | (wrap ? STEP_WRAP : 0u) |
+                     (w_in_range(ts.oa, ts.oda, ts.odb) ? W_IN_RANGE : 0u);
     if (nqx > 0 && nqy > 0) flags |= ((uint32_t)(qx0 - tx0) >> 1 << 3) | ((uint32_t)(qy0 - ty0) >> 1 << 28);
     if (ts.coarse && nqx > 0 && nqy > 0) {
         int kx0 = (qx0 - ts.ox0) >> 4, kx1 = (qx0 + 2 * (nqx - 1) - ts.ox0) >> 4;
@@ -2424,7 +2487,8 @@ __device__ __forceinline__ void walk_quad(const DevScene &S, const RasterArgs &P
     for (int s = 0; s < 4; s++) {
         if (!(w[0][s] >= 0.0f && w[1][s] >= 0.0f && w[2][s] >= 0.0f)) continue;
         float b1 = w[1][s] * ooa, b2 = w[2][s] * ooa;
-        float wv = 1.0f / ((oa + b1 * oda) + b2 * odb);
+        float den = (oa + b1 * oda) + b2 * odb;
+        float wv = (flags & W_IN_RANGE) ? rcp_in_range(den) : 1.0f / den;
         float z = ((za + b1 * zda) + b2 * zdb) * wv;
         if (z != z) continue;
         if (alpha && !alpha_pass(S, P.src, P.raster + 4 * (size_t)id, b1, b2, wv)) continue;
@@ -2872,7 +2936,7 @@ __device__ __forceinline__ uint32_t tt_hash(uint32_t id, int hs) { return (id * 
 
 // Row layout: [0] A1 B1 C1 SX1, [1] SY1 A2 B2 C2, [2] SX2 SY2 ooa oa,
 // [3] oda odb za zda, [4] zdb origin(ox0 | oy0 << 16) flags(coarse 1,
-// normal map 2) material, [5..11] shading interpolators Sh[0..6],
+// normal map 2, w_in_range 4) material, [5..11] shading interpolators Sh[0..6],
 // [12..14] tangent frame Tn[0..2] (normal-mapped triangles only).
 __device__ __forceinline__ void tt_fill(const RasterArgs &P, uint32_t id, int tx0, int ty0, float4 *row) {
     const float4 *R = P.raster + 4 * (size_t)id;
@@ -2886,7 +2950,9 @@ __device__ __forceinline__ void tt_fill(const RasterArgs &P, uint32_t id, int tx
         row[2] = make_float4(ts.SX[2], ts.SY[2], ts.ooa, ts.oa);
         row[3] = make_float4(ts.oda, ts.odb, ts.za, ts.zda);
         row[4] = make_float4(ts.zdb, __uint_as_float((uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16)),
-                             __uint_as_float((ts.coarse ? 1u : 0u) | (nmap ? 2u : 0u)), R[3].y);
+                             __uint_as_float((ts.coarse ? 1u : 0u) | (nmap ? 2u : 0u) |
+                                             (w_in_range(ts.oa, ts.oda, ts.odb) ? 4u : 0u)),
+                             R[3].y);
     }
     CV tv[3];
     float4 Sh[7], Tn[3];
@@ -2973,7 +3039,7 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
     if (has) {
         float A1, B1, C1, SX1, SY1, A2, B2, C2, SX2, SY2, ooa, za, zda, zdb;
         int ox0, oy0;
-        bool coarse;
+        bool coarse, in_range;
         if (table) {
             float4 r0 = rw[0], r1 = rw[1], r2 = rw[2], r3 = rw[3], r4 = rw[4];
             A1 = r0.x; B1 = r0.y; C1 = r0.z; SX1 = r0.w;
@@ -2985,6 +3051,7 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
             ox0 = (int)(org & 0xFFFFu);
             oy0 = (int)(org >> 16);
             coarse = (__float_as_uint(r4.z) & 1u) != 0u;
+            in_range = (__float_as_uint(r4.z) & 4u) != 0u;
         } else {
             TriSetup ts;
             tri_setup(P.geo[id], P.raster + 4 * (size_t)id, tx0, ty0, ts);
@@ -2992,6 +3059,7 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
             A2 = ts.A[2]; B2 = ts.B[2]; C2 = ts.C[2]; SX2 = ts.SX[2]; SY2 = ts.SY[2];
             ooa = ts.ooa; oa = ts.oa; oda = ts.oda; odb = ts.odb; za = ts.za; zda = ts.zda; zdb = ts.zdb;
             ox0 = ts.ox0; oy0 = ts.oy0; coarse = ts.coarse;
+            in_range = w_in_range(oa, oda, odb);
         }
         // the walk origin of the pixel's quad (quad_origin; the quad is walked)
         int bx = ox0, by = oy0;
@@ -3004,7 +3072,8 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
         float w2 = edge_chain_v(A2, B2, C2, SX2, SY2, bx, by, sx, sy, i, j);
         b1 = w1 * ooa;
         b2 = w2 * ooa;
-        w = 1.0f / ((oa + b1 * oda) + b2 * odb);
+        float den = (oa + b1 * oda) + b2 * odb;
+        w = in_range ? rcp_in_range(den) : 1.0f / den;
         z = ((za + b1 * zda) + b2 * zdb) * w;
     }
     // every lane of the wave is active here (one thread per pixel).  When

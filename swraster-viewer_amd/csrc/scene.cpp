@@ -328,6 +328,11 @@ SR_API int sr_scene_create(const sr_scene_desc *d, int32_t device, sr_scene **ou
         float ws = vg.world_max[k] - vg.world_min[k];
         ds.vox_size[k] = ws / (float)vg.dims[k];
     }
+    // reciprocals that the shading divides by (rounded once), where every size
+    // is well inside the floats' range
+    bool in_range = true;
+    for (int k = 0; k < 3; k++) in_range = in_range && ds.vox_size[k] >= 0x1p-40f && ds.vox_size[k] <= 0x1p40f;
+    for (int k = 0; k < 3; k++) ds.vox_rcp[k] = in_range ? 1.0f / ds.vox_size[k] : 0.0f;
     for (int c = 0; c < 4; c++) {
         for (int k = 0; k < 3; k++) ds.sh_const[c][k] = env.irradiance_sh[c][k] * vg.sh_scale;
         ds.sh_const[c][3] = 0.0f;
