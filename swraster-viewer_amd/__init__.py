@@ -441,6 +441,26 @@ class VoxelGrid:
         self.wmax = np.array(wmax, np.float32)
 
 
+class _LibraryGrid:
+    """A voxel grid that the library allocated; its arrays share the memory,
+    which is freed with the last of them (64 B per voxel of a GI grid are not
+    copied and paged in again)."""
+
+    def __init__(self, grid):
+        self.grid = grid
+
+    def array(self, pointer, count):
+        buf = (C.c_float * count).from_address(C.addressof(pointer.contents))
+        buf.owner = self
+        return np.frombuffer(buf, np.float32)
+
+    def __del__(self):
+        try:
+            lib().sr_voxel_grid_free(C.byref(self.grid))
+        except Exception:
+            pass
+
+
 # ---------------------------------------------------------------------------
 # Scene description (host arrays) and the HBM-resident scene
 # ---------------------------------------------------------------------------
@@ -653,14 +673,13 @@ class SceneData:
             check(lib().sr_prepare_gi(C.byref(self.desc), grid, -1 if device is None else int(device),
                                       threads, C.byref(g)))
             n = g.dims[0] * g.dims[1] * g.dims[2]
-            light = np.ctypeslib.as_array(g.light_intensity, shape=(n,)).copy()
-            sh4 = np.ctypeslib.as_array(g.sh4, shape=(n * 16,)).copy()
+            owner = _LibraryGrid(g)
+            light, sh4 = owner.array(g.light_intensity, n), owner.array(g.sh4, n * 16)
             dims, wmin, wmax = list(g.dims), list(g.world_min), list(g.world_max)
             if gi_cache and lib().sr_gi_cache_save(os.fsencode(gi_cache), C.byref(g)) != 0:
                 # as the reference (src/main.rs:258-262): report and go on
                 print(f"Failed to write GI cache {gi_cache}: {lib().sr_last_error().decode(errors='replace')}",
                       file=sys.stderr)
-            lib().sr_voxel_grid_free(C.byref(g))
             if path:
                 os.makedirs(CACHE_DIR, exist_ok=True)
                 np.savez(path, dims=dims, wmin=wmin, wmax=wmax, light=light, sh4=sh4)

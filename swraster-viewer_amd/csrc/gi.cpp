@@ -238,14 +238,13 @@ void gi_initial(const GiHost &h, const std::vector<float> &light, std::vector<fl
 }
 
 int gi_bake_host(const GiHost &h, const std::vector<uint8_t> &active, const std::vector<float> &light, int threads,
-                 std::vector<float> &out) {
+                 float *out) {
     int G = h.frame.grid;
     size_t nvox = (size_t)G * G * G;
     std::vector<float> coeffs;
     gi_initial(h, light, coeffs);
-    out.resize(nvox * 16);
     if (std::find(active.begin(), active.end(), (uint8_t)1) == active.end()) {
-        out = coeffs;       // nothing active: the scene SH, not blurred (src/gi.rs:338-341)
+        std::copy(coeffs.begin(), coeffs.end(), out);       // nothing active: the scene SH, not blurred (src/gi.rs:338-341)
         return SR_OK;
     }
     GiScene S = gi_scene_view(h);
@@ -310,9 +309,7 @@ SR_API int sr_prepare_gi(const sr_scene_desc *scene, int32_t grid, int32_t devic
     if (rc) return rc;
     GiHost h;
     if ((rc = gi_prepare(scene, grid, h))) return rc;
-    std::vector<float> sh4;
-    rc = device >= 0 ? gi_bake_device(h, active, light, device, sh4) : gi_bake_host(h, active, light, threads, sh4);
-    if (rc) return rc;
+    // the bake writes the grid where the caller gets it (64 B per voxel)
     size_t nvox = (size_t)grid * grid * grid;
     float *lp = (float *)malloc(nvox * 4);
     float *sp = (float *)malloc(nvox * 64);
@@ -321,8 +318,13 @@ SR_API int sr_prepare_gi(const sr_scene_desc *scene, int32_t grid, int32_t devic
         free(sp);
         return fail(SR_ERR_OUT_OF_MEMORY, "GI grid");
     }
+    rc = device >= 0 ? gi_bake_device(h, active, light, device, sp) : gi_bake_host(h, active, light, threads, sp);
+    if (rc) {
+        free(lp);
+        free(sp);
+        return rc;
+    }
     memcpy(lp, light.data(), nvox * 4);
-    memcpy(sp, sh4.data(), nvox * 64);
     out->dims[0] = out->dims[1] = out->dims[2] = grid;
     memcpy(out->world_min, h.frame.wmin, 12);
     memcpy(out->world_max, h.frame.wmax, 12);

@@ -398,7 +398,7 @@ inline uint32_t blocks(size_t n) { return (uint32_t)std::min<size_t>(std::max<si
     } while (0)
 
 int gi_bake_device(const GiHost &h, const std::vector<uint8_t> &active, const std::vector<float> &light, int device,
-                   std::vector<float> &out) {
+                   float *out) {
     const int grid = h.frame.grid;
     const size_t nvox = (size_t)grid * grid * grid;
     if (active.size() != nvox || light.size() != nvox) return fail(SR_ERR_INVALID_ARGUMENT, "GI grid size mismatch");
@@ -485,9 +485,8 @@ int gi_bake_device(const GiHost &h, const std::vector<uint8_t> &active, const st
     G.P = h.params;
     hipLaunchKernelGGL(k_gi_init, dim3(blocks(nvox)), dim3(256), 0, nullptr, G, nvox);
     GI_TRY(hipGetLastError());
-    out.resize(nvox * 16);
     if (list.empty()) {     // nothing active: the scene SH, not blurred (src/gi.rs:338-341)
-        GI_TRY(hipMemcpy(out.data(), G.coeffs, nvox * 64, hipMemcpyDeviceToHost));
+        GI_TRY(hipMemcpy(out, G.coeffs, nvox * 64, hipMemcpyDeviceToHost));
         return SR_OK;
     }
     bool translucent = false;
@@ -505,7 +504,7 @@ int gi_bake_device(const GiHost &h, const std::vector<uint8_t> &active, const st
     uint32_t over = 0;
     GI_TRY(hipMemcpy(&over, G.over, 4, hipMemcpyDeviceToHost));
     if (over) return fail(SR_ERR_CAPACITY, "a GI ray met more than %d translucent surfaces", GI_HIT_CAP);
-    GI_TRY(hipMemcpy(out.data(), blurred, nvox * 64, hipMemcpyDeviceToHost));
+    GI_TRY(hipMemcpy(out, blurred, nvox * 64, hipMemcpyDeviceToHost));
     return SR_OK;
 }
 

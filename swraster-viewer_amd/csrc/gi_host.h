@@ -30,10 +30,11 @@ struct GiHost {
 int gi_prepare(const sr_scene_desc *d, int grid, GiHost &h);
 GiScene gi_scene_view(const GiHost &h);
 void gi_initial(const GiHost &h, const std::vector<float> &light, std::vector<float> &sh4);
+// out: 16 floats per voxel.
 int gi_bake_host(const GiHost &h, const std::vector<uint8_t> &active, const std::vector<float> &light, int threads,
-                 std::vector<float> &out);
+                 float *out);
 // The same bake on a HIP device (gi.hip); identical results.
 int gi_bake_device(const GiHost &h, const std::vector<uint8_t> &active, const std::vector<float> &light, int device,
-                   std::vector<float> &out);
+                   float *out);
 
 }  // namespace sr
