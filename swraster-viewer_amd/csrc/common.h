@@ -37,6 +37,7 @@
 #define SR_DRAW_CLIP 1u
 #define SR_DRAW_OPAQUE 2u
 #define SR_DRAW_TANGENTS 4u
+#define SR_DRAW_ALPHA 8u         // alpha-tested material
 
 // record geometry (rec_geo): x, y the pixel box (x | y << 16 each); z flags
 // and, from SR_GEO_VIEW_SHIFT, the view; w a depth key that no fragment goes

@@ -18,6 +18,7 @@ struct FrameArgs {
     uint32_t total_items;         // (view, tile) items == bins
     int32_t tile_size;            // 8, 16 or 32
     int32_t any_tangents;
+    int32_t any_alpha;            // some draw's material is alpha tested
     // transient buffers
     float4 *xv;                   // total_xv clip positions, 2 * total_xv attribute float4, then
                                   // total_xv snaps (px, py, 1/w, z/w)

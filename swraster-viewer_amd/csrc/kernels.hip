@@ -40,6 +40,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "kernels.h"
 #include "swraster.h"
 
@@ -1836,18 +1838,38 @@ __device__ __forceinline__ uint32_t compute_mip(const DevTexture &T, const float
     return mip < T.max_mip ? mip : T.max_mip;
 }
 
-__device__ __forceinline__ uint32_t texel_nearest(const DevScene &S, const DevTexRef &ref, float u, float v,
-                                                  const float dd[4]) {
+// The mip level that a texture is sampled from, given the UV derivatives.
+struct TexLevel {
+    const SR_GLOBAL uint32_t *texels;
+    float wf, hf;
+    uint32_t bw;                  // 4x4-texel blocks per row
+    int wrap_s, wrap_t;
+};
+__device__ __forceinline__ TexLevel texel_level(const DevScene &S, const DevTexRef &ref, const float dd[4]) {
     const DevTexture &T = S.textures[ref.tex];
     uint32_t mip = compute_mip(T, dd);
-    float wf = (float)T.mip_w[mip], hf = (float)T.mip_h[mip];
-    uint32_t x = sat_u32(apply_wrap(floorf(u * wf), wf, ref.wrap_s));
-    uint32_t y = sat_u32(apply_wrap(floorf(v * hf), hf, ref.wrap_t));
+    TexLevel L;
+    L.texels = S.texels + T.base + T.mip_off[mip];
+    L.wf = (float)T.mip_w[mip];
+    L.hf = (float)T.mip_h[mip];
+    L.bw = (T.mip_w[mip] + 3u) >> 2;
+    L.wrap_s = ref.wrap_s;
+    L.wrap_t = ref.wrap_t;
+    return L;
+}
+
+__device__ __forceinline__ uint32_t texel_at(const TexLevel &L, float u, float v) {
+    uint32_t x = sat_u32(apply_wrap(floorf(u * L.wf), L.wf, L.wrap_s));
+    uint32_t y = sat_u32(apply_wrap(floorf(v * L.hf), L.hf, L.wrap_t));
     // levels are stored in 4x4-texel blocks, row-major over the level
     // padded to multiples of 4
-    uint32_t bw = (T.mip_w[mip] + 3u) >> 2;
-    uint32_t idx = T.mip_off[mip] + ((((y >> 2) * bw) + (x >> 2)) << 4) + ((y & 3u) << 2) + (x & 3u);
-    return S.texels[T.base + idx];
+    uint32_t idx = ((((y >> 2) * L.bw) + (x >> 2)) << 4) + ((y & 3u) << 2) + (x & 3u);
+    return L.texels[idx];
+}
+
+__device__ __forceinline__ uint32_t texel_nearest(const DevScene &S, const DevTexRef &ref, float u, float v,
+                                                  const float dd[4]) {
+    return texel_at(texel_level(S, ref, dd), u, v);
 }
 
 __device__ __forceinline__ void cube_uv(f3 n, float &uf, float &vf, uint32_t &slice) {
@@ -2180,20 +2202,28 @@ struct RasterArgs {
     WorkCounter *work;                      // the persistent raster's queues
 };
 
-__device__ __forceinline__ bool alpha_pass(const DevScene &S, const TriSource &T, const float4 *R, float b1, float b2,
-                                           float w) {
-    int material = __float_as_int(R[3].y);
-    const DevMaterial &M = S.materials[material];
+// What the alpha test of one triangle's samples needs: its UV interpolators,
+// texture level (the derivatives are the triangle's) and cutoff.
+struct AlphaTest {
+    float u0, ua, ub, v0, va, vb, cutoff;
+    TexLevel level;
+};
+__device__ __forceinline__ void alpha_setup(const DevScene &S, const TriSource &T, const float4 *R, AlphaTest &A) {
+    const DevMaterial &M = S.materials[__float_as_int(R[3].y)];
     CV tv[3];
     float4 Sh[7], Tn[3];
     load_tri_cv(T, R, tv);
     tri_shade_attrs(tv, R, false, Sh, Tn);
-    float4 s4 = Sh[4], s5 = Sh[5], s6 = Sh[6];
-    float u = ((s4.z + b1 * s4.w) + b2 * s5.x) * w;
-    float v = ((s5.y + b1 * s5.z) + b2 * s5.w) * w;
-    float dd[4] = {s6.x, s6.y, s6.z, s6.w};
-    float a = unpack_a(texel_nearest(S, M.base_tex, u, v, dd));
-    return a >= M.alpha_cutoff;
+    A.u0 = Sh[4].z; A.ua = Sh[4].w; A.ub = Sh[5].x;
+    A.v0 = Sh[5].y; A.va = Sh[5].z; A.vb = Sh[5].w;
+    A.cutoff = M.alpha_cutoff;
+    const float dd[4] = {Sh[6].x, Sh[6].y, Sh[6].z, Sh[6].w};
+    A.level = texel_level(S, M.base_tex, dd);
+}
+__device__ __forceinline__ bool alpha_pass(const AlphaTest &A, float b1, float b2, float w) {
+    float u = ((A.u0 + b1 * A.ua) + b2 * A.ub) * w;
+    float v = ((A.v0 + b1 * A.va) + b2 * A.vb) * w;
+    return unpack_a(texel_at(A.level, u, v)) >= A.cutoff;
 }
 
 // Per-wave staging of one batch of 64 bin entries (structure of arrays, one
@@ -2391,7 +2421,7 @@ __device__ __forceinline__ int stage_entry(const TriSetup &ts, uint32_t id, uint
 // reference's block choice and rejection, then the four samples' edge
 // chains (src/tilerasterizer.rs:220-381); covered samples with a non-NaN
 // depth enter the 64-bit minimum.
-template <int T, int SW>
+template <int T, int SW, bool ALPHA>
 __device__ __forceinline__ void walk_quad(const DevScene &S, const RasterArgs &P, const uint32_t *st, int o, int local,
                                           int tx0, int ty0, unsigned long long *keys, uint32_t zbound) {
     using SG = Stage<T>;
@@ -2479,19 +2509,26 @@ __device__ __forceinline__ void walk_quad(const DevScene &S, const RasterArgs &P
         }
     }
     uint32_t id = st[F_ID * SW + o];
-    bool alpha = (flags & 2u) != 0;
+    bool covered[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) covered[s] = w[0][s] >= 0.0f && w[1][s] >= 0.0f && w[2][s] >= 0.0f;
+    // an alpha-tested entry's setup, once for the quad's samples
+    const bool alpha = ALPHA && (flags & 2u) != 0;
+    AlphaTest at;
+    if (ALPHA && alpha && (covered[0] || covered[1] || covered[2] || covered[3]))
+        alpha_setup(S, P.src, P.raster + 4 * (size_t)id, at);
     float ooa = SF(F_OOA), oa = SF(F_OA), oda = SF(F_ODA), odb = SF(F_ODB);
     float za = SF(F_ZA), zda = SF(F_ZDA), zdb = SF(F_ZDB);
     unsigned long long *kq = keys + (qpy - ty0) * T + (qpx - tx0);
 #pragma unroll
     for (int s = 0; s < 4; s++) {
-        if (!(w[0][s] >= 0.0f && w[1][s] >= 0.0f && w[2][s] >= 0.0f)) continue;
+        if (!covered[s]) continue;
         float b1 = w[1][s] * ooa, b2 = w[2][s] * ooa;
         float den = (oa + b1 * oda) + b2 * odb;
         float wv = (flags & W_IN_RANGE) ? rcp_in_range(den) : 1.0f / den;
         float z = ((za + b1 * zda) + b2 * zdb) * wv;
         if (z != z) continue;
-        if (alpha && !alpha_pass(S, P.src, P.raster + 4 * (size_t)id, b1, b2, wv)) continue;
+        if (ALPHA && alpha && !alpha_pass(at, b1, b2, wv)) continue;
         unsigned long long key = ((unsigned long long)depth_key(z) << 32) | (unsigned long long)(~id);
         atomicMin(&kq[(s >> 1) * T + (s & 1)], key);
     }
@@ -2662,7 +2699,7 @@ __device__ __forceinline__ void raster_list(const RasterArgs &P, uint32_t item, 
     if (end > P.pair_cap) end = P.pair_cap;
 }
 
-template <int T, int NT>
+template <int T, int NT, bool ALPHA>
 __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long long *keys, uint32_t *stage) {
     constexpr int NW = NT / 64;               // waves
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2715,7 +2752,7 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
                 for (int step = NT / 2; step > 0; step >>= 1)
                     if ((int)stage[F_INCL * NT + o + step - 1] <= k) o += step;
                 int before = o ? (int)stage[F_INCL * NT + o - 1] : 0;
-                walk_quad<T, NT>(S, P, stage, o, k - before, tx0, ty0, keys, 0u);
+                walk_quad<T, NT, ALPHA>(S, P, stage, o, k - before, tx0, ty0, keys, 0u);
             }
         }
         __syncthreads();
@@ -2723,15 +2760,17 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
     raster_resolve<T, NT>(P, V, tx0, ty0, keys);
 }
 
-template <int T, int NT>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : 6))) k_raster(RasterArgs P) {
+// ALPHA: some of the frame's materials are alpha tested (the test's setup and
+// fetch would cost every other frame registers).
+template <int T, int NT, bool ALPHA>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : (ALPHA ? 5 : 6)))) k_raster(RasterArgs P) {
     __shared__ unsigned long long keys[T * T];
     __shared__ uint32_t stage[Stage<T>::COUNT * NT];
     __shared__ uint32_t next;
     clock_start(P.clock, CLOCK_RASTER);
     if (!P.persistent) {
         const uint32_t item = xcd_item(blockIdx.x);
-        if (item < P.total_items) raster_item<T, NT>(P, item, keys, stage);
+        if (item < P.total_items) raster_item<T, NT, ALPHA>(P, item, keys, stage);
     } else {
         // Every workgroup starts at its own position; the rest are drained
         // from counters, each shared by the workgroups of one residue of the
@@ -2748,7 +2787,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
             uint32_t got = 0u;
             if (threadIdx.x == 0) got = atomicAdd(&P.work[g].next, 1u);
             const uint32_t item = xcd_item(pos);
-            if (item < P.total_items) raster_item<T, NT>(P, item, keys, stage);
+            if (item < P.total_items) raster_item<T, NT, ALPHA>(P, item, keys, stage);
             if (threadIdx.x == 0) next = g + groups * (first + got);
             __syncthreads();
             pos = next;
@@ -2803,6 +2842,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return max(v, lane_xor<32>(v));
 }
 
+template <bool ALPHA>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_raster_near(RasterArgs P) {
     constexpr int T = 16;
     __shared__ unsigned long long keys[T * T];
@@ -2886,7 +2926,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                 for (int step = 32; step > 0; step >>= 1)
                     if ((int)stage[F_INCL * 64 + own + step - 1] <= k) own += step;
                 const int before = own ? (int)stage[F_INCL * 64 + own - 1] : 0;
-                walk_quad<T, 64>(S, P, stage, own, k - before, tx0, ty0, keys, zmin[own]);
+                walk_quad<T, 64, ALPHA>(S, P, stage, own, k - before, tx0, ty0, keys, zmin[own]);
             }
             __syncthreads();
 #pragma unroll
@@ -4162,14 +4202,20 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     // stage events: bins done = the raster's start, the raster's end, and
     // the frame's end = the shading's end (or the translucent pass's)
     hipEvent_t e2 = a.events[2], e4 = a.events[4], e3 = a.has_translucent ? ev_none : a.events[3];
-    switch (a.tile_size) {
-        case 8: SR_LAUNCH_TIMED(e2, e4, (k_raster<8, 64>), dim3(grid), dim3(64), st, P); break;
-        case 32: SR_LAUNCH_TIMED(e2, e4, (k_raster<32, 512>), dim3(grid), dim3(512), st, P); break;
-        default:
-            if (a.overdraw) SR_LAUNCH_TIMED(e2, e4, k_raster_near, dim3(xcd_positions(a.total_items)), dim3(64), st, P);
-            else SR_LAUNCH_TIMED(e2, e4, (k_raster<16, 256>), dim3(grid), dim3(256), st, P);
-            break;
-    }
+    auto raster = [&](auto alpha) {
+        constexpr bool ALPHA = decltype(alpha)::value;
+        switch (a.tile_size) {
+            case 8: SR_LAUNCH_TIMED(e2, e4, (k_raster<8, 64, ALPHA>), dim3(grid), dim3(64), st, P); break;
+            case 32: SR_LAUNCH_TIMED(e2, e4, (k_raster<32, 512, ALPHA>), dim3(grid), dim3(512), st, P); break;
+            default:
+                if (a.overdraw)
+                    SR_LAUNCH_TIMED(e2, e4, k_raster_near<ALPHA>, dim3(xcd_positions(a.total_items)), dim3(64), st, P);
+                else SR_LAUNCH_TIMED(e2, e4, (k_raster<16, 256, ALPHA>), dim3(grid), dim3(256), st, P);
+                break;
+        }
+    };
+    if (a.any_alpha) raster(std::true_type());
+    else raster(std::false_type());
     switch (a.tile_size) {
         case 8: SR_LAUNCH_TIMED(ev_none, e3, (k_shade<8, 64>), dim3(xcd_positions(a.total_items)), dim3(64), st, P); break;
         case 32:

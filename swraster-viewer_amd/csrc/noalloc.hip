@@ -171,6 +171,8 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
     a.total_items = items;
     a.tile_size = T;
     a.any_tangents = 0;
+    for (const DevDraw &d : draws)
+        if (d.flags & SR_DRAW_ALPHA) a.any_alpha = 1;
     a.xv = (float4 *)(base + o_xv);
     a.xt = nullptr;
     a.tri_counts = (uint32_t *)(base + o_counts);

@@ -176,7 +176,7 @@ int build_draws(const sr_scene *scene, const sr_camera &cam, int view, uint32_t 
                 d.view = view;
                 d.material = p.material;
                 d.flags = (ft == FT_INTERSECTING ? SR_DRAW_CLIP : 0u) | (pass == 0 ? SR_DRAW_OPAQUE : 0u) |
-                          (p.tangents ? SR_DRAW_TANGENTS : 0u);
+                          (p.tangents ? SR_DRAW_TANGENTS : 0u) | (p.alpha ? SR_DRAW_ALPHA : 0u);
                 in_tri += p.num_tri;
                 xv += p.num_vtx;
                 if (p.num_tri == 0) continue;
@@ -236,7 +236,7 @@ int Pipeline::launch_graph(const FrameArgs &a, size_t vbytes, size_t upload) {
     GraphKey k;
     memset(&k, 0, sizeof(k));
     k.n[0] = (uint64_t)a.num_views; k.n[1] = (uint64_t)a.num_draws; k.n[2] = a.total_xv; k.n[3] = a.total_in;
-    k.n[4] = a.total_items; k.n[5] = (uint64_t)a.tile_size; k.n[6] = (uint64_t)a.any_tangents; k.n[7] = a.rec_cap;
+    k.n[4] = a.total_items; k.n[5] = (uint64_t)a.tile_size; k.n[6] = (uint64_t)a.any_tangents | ((uint64_t)a.any_alpha << 1); k.n[7] = a.rec_cap;
     k.n[8] = a.pair_cap; k.n[9] = a.clip_cap; k.n[10] = (uint64_t)a.persistent_blocks; k.n[11] = vbytes;
     k.n[12] = upload; k.n[13] = a.color_plane; k.n[14] = (uint64_t)a.has_translucent | ((uint64_t)a.direct << 1);
     k.n[15] = ((uint64_t)a.tr_cap << 32) | a.tr_slots | ((uint64_t)a.overdraw << 31);
@@ -301,8 +301,11 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
     for (const DevView &v : hv)
         lum_slots = std::max<size_t>(lum_slots, (size_t)v.lum_offset + (size_t)v.ref_tiles_x * v.ref_tiles_y);
     if ((r = center.ensure(lum_slots * 16))) return r;
-    bool has_tr = false;
-    for (const DevDraw &d : hd) has_tr = has_tr || !(d.flags & SR_DRAW_OPAQUE);
+    bool has_tr = false, any_alpha = false;
+    for (const DevDraw &d : hd) {
+        has_tr = has_tr || !(d.flags & SR_DRAW_OPAQUE);
+        any_alpha = any_alpha || (d.flags & SR_DRAW_ALPHA);
+    }
     if (has_tr) {
         if ((r = tr_count.ensure(lum_slots * 4))) return r;
         if ((r = tr_start.ensure(lum_slots * 4))) return r;
@@ -353,6 +356,7 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
         a.total_items = total_items;
         a.tile_size = tile_size;
         a.any_tangents = any_tangents ? 1 : 0;
+        a.any_alpha = any_alpha ? 1 : 0;
         a.xv = (float4 *)xv.ptr;
         a.xt = any_tangents ? (float4 *)xt.ptr : nullptr;
         a.tri_counts = (uint32_t *)tri_counts.ptr;

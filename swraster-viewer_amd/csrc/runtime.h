@@ -40,6 +40,7 @@ struct HostPrim {
     uint32_t vtx_base, num_vtx, idx_base, num_tri;
     int32_t material;
     bool tangents;
+    bool alpha;                   // alpha-tested material
     Sphere bs;
 };
 struct HostMesh {

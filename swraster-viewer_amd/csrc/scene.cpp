@@ -192,6 +192,7 @@ SR_API int sr_scene_create(const sr_scene_desc *d, int32_t device, sr_scene **ou
         h.num_tri = p.num_indices / 3;
         h.material = p.material;
         h.tangents = mat_normal[p.material];
+        h.alpha = (mats[p.material].flags & SR_MAT_ALPHA_TESTED) != 0;
         h.bs = bounding_sphere(p.positions, p.num_vertices);
         for (uint32_t v = 0; v < p.num_vertices; v++) {
             px[vb + v] = p.positions[3 * v];
