@@ -10,16 +10,23 @@
 //   k_scan_*        device-wide exclusive scan (post-clip ids, chunk pairs)
 //   k_setup         clipping with attributes, snap, cull, bbox, setup records,
 //                   pair counts per chunk   src/renderer.rs:668-846
+//   k_bin_cols, k_bin_place
+//                   stable binning of small frames: the bins' offsets from
+//                   k_setup's (chunk, bin) counts, then the lists themselves
 //   k_bin_expand    stable binning: the records' pairs in record order
 //   k_bin_hist, k_bin_rowscan, k_bin_scatter, k_bin_bounds
 //                   stable binning: radix passes over the bin index, then
 //                   each tile's list bounds src/bumpqueue.rs:96-112
-//   k_raster_shade  one workgroup per screen tile: coverage with the
-//                   reference's exact f32 edge-evaluation chains into a 64-bit
-//                   (depth, id) LDS buffer, then visibility-buffer PBR
-//                   shading, skybox and centre luminance
-//                                           src/tilerasterizer.rs:72-543,
-//                                           src/shader.rs:102-329
+//   k_raster, k_raster_near
+//                   per screen tile: coverage with the reference's exact f32
+//                   edge-evaluation chains into a 64-bit (depth, id) LDS
+//                   buffer                  src/tilerasterizer.rs:72-543
+//   k_shade         visibility-buffer PBR shading, skybox and centre
+//                   luminance               src/shader.rs:102-329
+//   k_tr_bins, k_tr_sort, k_translucent
+//                   translucent triangles: 64-px lists, back-to-front order,
+//                   forward blend           src/tilerasterizer.rs:72-543
+//   k_exposure      the exposure step from the tiles' luminance
 //   k_blit          exposure, tonemap, quantize, pack
 //                                           src/renderer.rs:293-355
 //
@@ -2203,7 +2210,9 @@ struct RasterArgs {
 };
 
 // What the alpha test of one triangle's samples needs: its UV interpolators,
-// texture level (the derivatives are the triangle's) and cutoff.
+// texture level (the derivatives are the triangle's) and cutoff.  Set up once
+// for a quad's covered samples (per sample it refetched the three vertices:
+// raster of a cut-out heightfield at 1366x769 56.6 -> 40.5 us).
 struct AlphaTest {
     float u0, ua, ub, v0, va, vb, cutoff;
     TexLevel level;
@@ -2760,8 +2769,10 @@ __device__ void raster_item(const RasterArgs &P, uint32_t item, unsigned long lo
     raster_resolve<T, NT>(P, V, tx0, ty0, keys);
 }
 
-// ALPHA: some of the frame's materials are alpha tested (the test's setup and
-// fetch would cost every other frame registers).
+// ALPHA: some of the frame's materials are alpha tested.  Frames without one
+// take the variant without the test, whose code costs registers: 74 VGPRs and
+// spilled scalars at 16-px tiles against 64 (64 views: 8.29 -> 8.21 ms), 248 B
+// of scratch a thread at 32-px tiles against none.
 template <int T, int NT, bool ALPHA>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : (ALPHA ? 5 : 6)))) k_raster(RasterArgs P) {
     __shared__ unsigned long long keys[T * T];
@@ -2815,8 +2826,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
 // alone and four waves a tile, the raster took 496 us at 2465 VALU
 // instructions a wave; in this order with four waves sharing a tile (one
 // setting up at a time, barriers in each round) 396 us at 1286, which is 0.69
-// of the issue rate; one wave a tile needs no barrier and takes 195 us at
-// 3420, 0.94 of it.  Frames of small triangles (the heightfield) keep
+// of the issue rate; one wave a tile needs no barrier and took 195 us at
+// 3420, 0.94 of it (182 with shorter scans and without the alpha test).  Frames of small triangles (the heightfield) keep
 // k_raster, whose four waves share their long lists.
 // ---------------------------------------------------------------------------
 #define NEAR_BATCH 256

@@ -181,6 +181,53 @@ def test_overdraw_raster_list_lengths(sr, orc, n, kind):
     r.close()
 
 
+# the raster variants with the alpha test: each tile size, and the overdraw
+# raster (tile 16, a list of 300); "far" minifies the texture to its last levels
+@pytest.mark.parametrize("n,tile,far", [(24, 8, False), (24, 16, True), (24, 32, False), (300, 16, False),
+                                        (300, 16, True), (300, 32, True)])
+def test_alpha_raster_variants(sr, orc, n, tile, far):
+    """n large triangles over a 64x48 view, two in three cut out by their
+    texture's alpha, the rest opaque: both renderings have the oracle's
+    visibility buffer, the second of 300 at 16-px tiles by the overdraw raster."""
+    from util import attach_dummy, screen_triangle_scene
+    import swraster_viewer_amd.scenes as sc
+    W, H = 64, 48
+    rng = np.random.default_rng(n + tile)
+    c = rng.uniform([0, 0], [W * 16, H * 16], (n, 1, 2))
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2]) + rng.uniform(-0.4, 0.4, (n, 3))
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * (rng.uniform(40, 90, (n, 3)) * 16)[..., None])
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    scene, spec = screen_triangle_scene(sr, tris, rng.uniform(2.0, 90.0, (n, 1)) * rng.uniform(0.9, 1.1, (n, 3)), W, H)
+    p, mat = scene.primitives[0], scene.materials[0]
+    uv = (rng.uniform(-2, 2, (3 * n, 2)) * (40.0 if far else 1.0)).astype(np.float32)
+    tex = (32, 32, sr.SR_TEX_SRGB, sr.pack_rgba(rng.integers(0, 256, (32 * 32, 4), dtype=np.uint8)).ravel())
+    prims, mats = [], []
+    for k, part in enumerate(np.array_split(np.arange(3 * n).reshape(n, 3), 3)):
+        part = part.reshape(-1)
+        prims.append({"positions": p["positions"][part], "normals": p["normals"][part], "texcoords": uv[part],
+                      "tangents": None, "indices": np.arange(len(part), dtype=np.uint32), "material": k})
+        mats.append(dict(mat, **({} if k == 1 else {
+            "alpha_mode": sr.SR_ALPHA_MASK, "alpha_cutoff": 0.3 + 0.2 * k,
+            "base_color_tex": (0, sr.SR_WRAP_REPEAT, sr.SR_WRAP_MIRRORED_REPEAT)})))
+    scene = sr.SceneData(prims, [(0, 3)], list(scene.nodes), mats, [tex], name="cut")
+    attach_dummy(sr, scene)
+    cam = sc.make_camera(spec)
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()
+    r = sr.Renderer(W, H, tile_size=tile)
+    gscene = sr.Scene(scene)
+    for k in range(2):
+        r.render_scene(gscene, cam)
+        ids, depth = r.read_vbuffer()
+        assert np.array_equal(ids, want["ids"]), f"frame {k}"
+        assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32)), f"frame {k}"
+    assert n < 300 or r.stats()["depth_rejection"] == int(tile == 16)
+    r.close()
+
+
 def _with_backfacing(sr, scene, n):
     """scene plus a last primitive of n copies of one backfacing triangle in
     every mesh-bearing node's place: they make records without bins, so the
