@@ -2212,7 +2212,7 @@ struct RasterArgs {
 // What the alpha test of one triangle's samples needs: its UV interpolators,
 // texture level (the derivatives are the triangle's) and cutoff.  Set up once
 // for a quad's covered samples (per sample it refetched the three vertices:
-// raster of a cut-out heightfield at 1366x769 56.6 -> 40.5 us).
+// raster of 24 cut-out spheres at 1367x771 56.6 -> 40.5 us).
 struct AlphaTest {
     float u0, ua, ub, v0, va, vb, cutoff;
     TexLevel level;
