@@ -41,7 +41,7 @@
 
 // record geometry (rec_geo): x, y the pixel box (x | y << 16 each); z flags
 // and, from SR_GEO_VIEW_SHIFT, the view; w a depth key that no fragment goes
-// below (0: none)
+// below (0: none), where the frame's raster uses it
 #define SR_GEO_VIEW_SHIFT 8
 #define SR_GEO_EMPTY 1u          // culled or empty bounding box: no bins
 #define SR_GEO_ALPHA 2u          // alpha-tested material

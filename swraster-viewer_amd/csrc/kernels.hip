@@ -51,6 +51,7 @@
 
 #include "kernels.h"
 #include "swraster.h"
+#include "tri_bound.h"
 
 namespace sr {
 
@@ -805,6 +806,7 @@ struct SetupOut {
     uint32_t cap;
     SR_GLOBAL DevStatus *status;
     int T;
+    int bounds;                           // the raster reads the records' depth bounds
     // direct binning (k_setup<true>): the chunks' pair counts per tile, one
     // row of `items` per chunk, and each chunk's first record
     SR_GLOBAL uint32_t *matrix;
@@ -874,27 +876,6 @@ __device__ __forceinline__ uint32_t depth_key(float z) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-// A depth key no fragment of the triangle goes below, or 0 (no bound), from
-// its vertices' z/w (1/w) and 1/w.  The depth ((za + b1 zda) + b2 zdb) / ((oa
-// + b1 oda) + b2 odb) is a ratio of affine functions of the barycentrics, so
-// over the triangle it lies between its values at the vertices when the
-// denominator keeps its sign.  Covered samples have b1, b2 >= 0 and b1 + b2 <=
-// 1 to within 4e-7 (the edge values and 1/area rounded once each) and are
-// evaluated to a few ulps, as are the quotients here (hardware reciprocal);
-// with the vertices' denominators within a factor 16 of each other the
-// depth's derivative in b is below 48 times the largest vertex depth, so a
-// margin of 1e-4 of that depth covers all of it with room to spare.
-__device__ __forceinline__ uint32_t tri_zmin_key(const float zow[3], const float oow[3]) {
-    float dmin = fminf(oow[0], fminf(oow[1], oow[2])), dmax = fmaxf(oow[0], fmaxf(oow[1], oow[2]));
-    if (!(dmin > 1e-30f) || !(dmax <= 16.0f * dmin)) return 0u;
-    float z0 = zow[0] * __builtin_amdgcn_rcpf(oow[0]), z1 = zow[1] * __builtin_amdgcn_rcpf(oow[1]);
-    float z2 = zow[2] * __builtin_amdgcn_rcpf(oow[2]);
-    float zabs = fmaxf(fabsf(z0), fmaxf(fabsf(z1), fabsf(z2)));
-    float lo = fminf(z0, fminf(z1, z2)) - (zabs * 1e-4f + 1e-30f);
-    if (!(z0 == z0 && z1 == z1 && z2 == z2) || !(zabs < 1e30f)) return 0u;
-    return depth_key(lo);
-}
-
 // A record's third geometry word: SR_GEO_* flags and the view.
 __device__ __forceinline__ uint32_t geo_word(uint32_t flags, int view) { return flags | ((uint32_t)view << SR_GEO_VIEW_SHIFT); }
 __device__ __forceinline__ int geo_view(uint4 g) { return (int)(g.z >> SR_GEO_VIEW_SHIFT); }
@@ -938,8 +919,11 @@ __device__ Rect emit_triangle(const DevView &V, int view, const SnapV sv[3], uin
     if (matflags & SR_MAT_ALPHA_TESTED) flags |= SR_GEO_ALPHA;
     if (matflags & SR_MAT_NORMAL_MAP) flags |= SR_GEO_NORMAL_MAP;
     if (translucent) flags |= SR_GEO_TRANSLUCENT;
+    uint32_t zkey = 0u;
+    float zmin;
+    if (O.bounds && tri_zmin(px, py, ooa, zow, oow, zmin)) zkey = depth_key(zmin);
     O.geo[id] = make_uint4((uint32_t)pmnx | ((uint32_t)pmny << 16), (uint32_t)pmxx | ((uint32_t)pmxy << 16),
-                           geo_word(flags, view), tri_zmin_key(zow, oow));
+                           geo_word(flags, view), zkey);
     float4 *R = O.raster + 4 * (size_t)id;
     R[0] = make_float4(__int_as_float(px[0]), __int_as_float(py[0]), __int_as_float(px[1]), __int_as_float(py[1]));
     R[1] = make_float4(__int_as_float(px[2]), __int_as_float(py[2]), ooa, oow[0]);
@@ -2810,7 +2794,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
 // ---------------------------------------------------------------------------
 // k_raster_near: the raster of overdrawn frames (many large triangles deep),
 // one wave per (view, 16-px tile).  The wave takes 256 bin entries at a time
-// and sorts them by depth bound (tri_zmin_key) in four groups of 64, in
+// and sorts them by depth bound (tri_zmin) in four groups of 64, in
 // registers.  A round sets up the 16 nearest entries left of each group, one
 // per lane, walks their quads, and then takes the largest depth stored in
 // each 8x8 quadrant of the tile.  An entry whose bound lies behind the
@@ -4069,6 +4053,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     so.geo = (SR_GLOBAL uint4 *)a.rec_geo; so.raster = (SR_GLOBAL float4 *)a.rec_raster;
     so.cap = a.rec_cap; so.status = (SR_GLOBAL DevStatus *)a.status;
     so.T = a.tile_size;
+    so.bounds = a.overdraw;
     so.chunk_pairs = (SR_GLOBAL uint32_t *)a.chunk_pairs;
     so.matrix = (SR_GLOBAL uint32_t *)a.sort_hist;
     so.chunk_first = (SR_GLOBAL uint32_t *)a.chunk_pairs;

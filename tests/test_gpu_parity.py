@@ -296,6 +296,35 @@ def test_depth_rejection_tilted_overdraw(sr, orc, scenes, seed):
         assert np.array_equal(ids, o["ids"]) and np.array_equal(bits(depth), bits(o["depth"]))
 
 
+@pytest.mark.parametrize("W,H,radius", [(5120, 2880, 1200), (7680, 4320, 2000)])
+def test_depth_rejection_wrapping_edges(sr, orc, scenes, W, H, radius):
+    """300 large triangles in frames above 2^31 / 256 pixels, where the i32
+    constants of long edges wrap and the reference draws such triangles far
+    outside their vertices' depths: the depth-rejecting raster draws them
+    too."""
+    from util import attach_dummy, screen_triangle_scene
+    rng = np.random.default_rng(radius)
+    n = 300
+    c = rng.uniform([0, 0], [W * 16, H * 16], (n, 1, 2))
+    ang = rng.uniform(0, 2 * np.pi, (n, 3))
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * radius * 16)
+    tris = np.clip(tris, 0, [W * 16 - 1, H * 16 - 1])
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    depths = rng.uniform(2.0, 90.0, (n, 1)) * rng.uniform(0.5, 1.0, (n, 3))
+    scene, cam = screen_triangle_scene(sr, tris, depths, W, H)
+    attach_dummy(sr, scene)
+    gscene = sr.Scene(scene)
+    camera = scenes.make_camera(cam)
+    (i1, d1, h1), (i2, d2, h2) = _two_frames(sr, gscene, camera, W, H)
+    assert h2 == 1, "the overdraw did not select the depth-rejecting raster"
+    o = render_oracle(orc, scene, camera, W, H, threads=16)
+    for k, (ids, depth) in enumerate(((i1, d1), (i2, d2))):
+        assert np.array_equal(ids, o["ids"]), f"frame {k}: {int((ids != o['ids']).sum())} pixels"
+        assert np.array_equal(bits(depth), bits(o["depth"])), f"frame {k}"
+
+
 @pytest.mark.parametrize("W,H,seed", [(256, 144, 7), (130, 66, 8)])
 def test_tiny_triangles_parity(sr, orc, scenes, W, H, seed):
     """Dense sub-pixel to 4-px triangles (most of them cover no pixel centre,
