@@ -99,6 +99,13 @@ __device__ __forceinline__ float rcp_in_range(float b) {
     float y = __builtin_amdgcn_rcpf(b);
     return fmaf(fmaf(-b, y, 1.0f), y, y);
 }
+// 1 / b for any b.  (The 1/w that a sample interpolates is between its
+// vertices' only inside the triangle; covered samples of a triangle whose
+// integer edge constants wrap lie anywhere, and it can be zero there.)
+__device__ __forceinline__ float rcp_ieee(float b) {
+    if (b >= 0x1p-96f && b <= 0x1p96f) return rcp_in_range(b);
+    return 1.0f / b;
+}
 // a / b from y = rcp(b), correctly rounded.
 __device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
     float q = a * y;
@@ -2230,9 +2237,7 @@ enum {
 // equal 32 A and 32 B exactly unless 32 a wraps (|a| >= 2^26), which the
 // entry's STEP_WRAP flag marks and walk_quad then recomputes.
 #define STEP_WRAP 4u
-// The entry's 1/w at its covered samples is in range for rcp_in_range.
-#define W_IN_RANGE 0x80u
-// F_FLAGS: coarse 1, alpha 2, STEP_WRAP, W_IN_RANGE; from bit 3 and 28 the first quad's
+// F_FLAGS: coarse 1, alpha 2, STEP_WRAP; from bit 3 and 28 the first quad's
 // column and row in the tile; from bit 8 the rejected blocks, from 20 and 24
 // the first block.  After F_ROWS: inclusive quad counts per quad row (bytes up
 // to 16-px tiles, whose entries have at most 64 quads, else u16 pairs), then
@@ -2247,16 +2252,6 @@ template <int T> struct Stage {
     static constexpr int LO = CUM + (BYTES ? NR / 4 : NR / 2);
     static constexpr int COUNT = LO + (NR + 7) / 8;
 };
-
-// Whether the interpolated 1/w, (oa + b1 oda) + b2 odb, stays within 2^+-60
-// (or little beyond) at covered samples: b1, b2 >= 0 and b1 + b2 <= 1 to
-// within 4e-7 keep it between the vertices' values, which differ by a factor
-// of 2^16 at most, to a few percent of the smallest.
-__device__ __forceinline__ bool w_in_range(float oa, float oda, float odb) {
-    float d1 = oa + oda, d2 = oa + odb;
-    float lo = fminf(oa, fminf(d1, d2)), hi = fmaxf(oa, fmaxf(d1, d2));
-    return oa == oa && d1 == d1 && d2 == d2 && lo >= 0x1p-60f && hi <= 0x1p60f && hi <= 65536.0f * lo;
-}
 
 // f32 corner test of the 16px block at (bx, by) (src/tilerasterizer.rs:258-291)
 __device__ __forceinline__ bool block_out(const TriSetup &ts, int bx, int by) {
@@ -2323,8 +2318,7 @@ __device__ __forceinline__ int stage_entry(const TriSetup &ts, uint32_t id, uint
     st[F_ORG * SW + lane] = (uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16);
 
     // rejected 16px blocks among the (at most 3x3) that meet the tile
-    uint32_t flags = (ts.coarse ? 1u : 0u) | ((gflags & SR_GEO_ALPHA) ? 2u : 0u) | (wrap ? STEP_WRAP : 0u) |
-                     (w_in_range(ts.oa, ts.oda, ts.odb) ? W_IN_RANGE : 0u);
+    uint32_t flags = (ts.coarse ? 1u : 0u) | ((gflags & SR_GEO_ALPHA) ? 2u : 0u) | (wrap ? STEP_WRAP : 0u);
     if (nqx > 0 && nqy > 0) flags |= ((uint32_t)(qx0 - tx0) >> 1 << 3) | ((uint32_t)(qy0 - ty0) >> 1 << 28);
     if (ts.coarse && nqx > 0 && nqy > 0) {
         int kx0 = (qx0 - ts.ox0) >> 4, kx1 = (qx0 + 2 * (nqx - 1) - ts.ox0) >> 4;
@@ -2517,8 +2511,7 @@ __device__ __forceinline__ void walk_quad(const DevScene &S, const RasterArgs &P
     for (int s = 0; s < 4; s++) {
         if (!covered[s]) continue;
         float b1 = w[1][s] * ooa, b2 = w[2][s] * ooa;
-        float den = (oa + b1 * oda) + b2 * odb;
-        float wv = (flags & W_IN_RANGE) ? rcp_in_range(den) : 1.0f / den;
+        float wv = rcp_ieee((oa + b1 * oda) + b2 * odb);
         float z = ((za + b1 * zda) + b2 * zdb) * wv;
         if (z != z) continue;
         if (ALPHA && alpha && !alpha_pass(at, b1, b2, wv)) continue;
@@ -2971,7 +2964,7 @@ __device__ __forceinline__ uint32_t tt_hash(uint32_t id, int hs) { return (id * 
 
 // Row layout: [0] A1 B1 C1 SX1, [1] SY1 A2 B2 C2, [2] SX2 SY2 ooa oa,
 // [3] oda odb za zda, [4] zdb origin(ox0 | oy0 << 16) flags(coarse 1,
-// normal map 2, w_in_range 4) material, [5..11] shading interpolators Sh[0..6],
+// normal map 2) material, [5..11] shading interpolators Sh[0..6],
 // [12..14] tangent frame Tn[0..2] (normal-mapped triangles only).
 __device__ __forceinline__ void tt_fill(const RasterArgs &P, uint32_t id, int tx0, int ty0, float4 *row) {
     const float4 *R = P.raster + 4 * (size_t)id;
@@ -2985,9 +2978,7 @@ __device__ __forceinline__ void tt_fill(const RasterArgs &P, uint32_t id, int tx
         row[2] = make_float4(ts.SX[2], ts.SY[2], ts.ooa, ts.oa);
         row[3] = make_float4(ts.oda, ts.odb, ts.za, ts.zda);
         row[4] = make_float4(ts.zdb, __uint_as_float((uint32_t)ts.ox0 | ((uint32_t)ts.oy0 << 16)),
-                             __uint_as_float((ts.coarse ? 1u : 0u) | (nmap ? 2u : 0u) |
-                                             (w_in_range(ts.oa, ts.oda, ts.odb) ? 4u : 0u)),
-                             R[3].y);
+                             __uint_as_float((ts.coarse ? 1u : 0u) | (nmap ? 2u : 0u)), R[3].y);
     }
     CV tv[3];
     float4 Sh[7], Tn[3];
@@ -3074,7 +3065,7 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
     if (has) {
         float A1, B1, C1, SX1, SY1, A2, B2, C2, SX2, SY2, ooa, za, zda, zdb;
         int ox0, oy0;
-        bool coarse, in_range;
+        bool coarse;
         if (table) {
             float4 r0 = rw[0], r1 = rw[1], r2 = rw[2], r3 = rw[3], r4 = rw[4];
             A1 = r0.x; B1 = r0.y; C1 = r0.z; SX1 = r0.w;
@@ -3086,7 +3077,6 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
             ox0 = (int)(org & 0xFFFFu);
             oy0 = (int)(org >> 16);
             coarse = (__float_as_uint(r4.z) & 1u) != 0u;
-            in_range = (__float_as_uint(r4.z) & 4u) != 0u;
         } else {
             TriSetup ts;
             tri_setup(P.geo[id], P.raster + 4 * (size_t)id, tx0, ty0, ts);
@@ -3094,7 +3084,6 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
             A2 = ts.A[2]; B2 = ts.B[2]; C2 = ts.C[2]; SX2 = ts.SX[2]; SY2 = ts.SY[2];
             ooa = ts.ooa; oa = ts.oa; oda = ts.oda; odb = ts.odb; za = ts.za; zda = ts.zda; zdb = ts.zdb;
             ox0 = ts.ox0; oy0 = ts.oy0; coarse = ts.coarse;
-            in_range = w_in_range(oa, oda, odb);
         }
         // the walk origin of the pixel's quad (quad_origin; the quad is walked)
         int bx = ox0, by = oy0;
@@ -3107,8 +3096,7 @@ __device__ void shade_item(const RasterArgs &P, uint32_t item) {
         float w2 = edge_chain_v(A2, B2, C2, SX2, SY2, bx, by, sx, sy, i, j);
         b1 = w1 * ooa;
         b2 = w2 * ooa;
-        float den = (oa + b1 * oda) + b2 * odb;
-        w = in_range ? rcp_in_range(den) : 1.0f / den;
+        w = rcp_ieee((oa + b1 * oda) + b2 * odb);
         z = ((za + b1 * zda) + b2 * zdb) * w;
     }
     // every lane of the wave is active here (one thread per pixel).  When

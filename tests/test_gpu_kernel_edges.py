@@ -319,3 +319,32 @@ def test_gi_tree_sizes(sr, scenes, env, n, grid, glass):
                      "emissive": (0.2 * k, 0.1, 0.0), "is_translucent": int(glass and k == 0), "transmission": 0.6})
     scene = sr.SceneData(prims, [(0, len(prims))], [(np.eye(4, dtype=np.float32), 0)], mats, [], name=f"gi_{n}")
     assert np.array_equal(_gi(sr, scene, env, grid, 0), _gi(sr, scene, env, grid, -1))
+
+
+# (depth of vertex 0, of the other two, pixel): a covered sample of the
+# triangle at which the interpolated 1/w is exactly zero
+@pytest.mark.parametrize("w0,w1,px,py", [(21.636152, 67.772125, 4963, 1629), (15.870249, 80.99527, 5004, 1632),
+                                         (5.1477737, 84.73842, 4949, 1749)])
+def test_zero_denominator_sample(sr, orc, scenes, w0, w1, px, py):
+    """A triangle whose integer edge constants wrap covers samples far outside
+    itself, one of them where the interpolated 1/w is zero: w and the depth
+    are infinite there, as IEEE division gives them, and the pixel is the
+    triangle's, in the raster and in the shading."""
+    from util import attach_dummy, screen_triangle_scene
+    W, H = 5120, 2880
+    tri = np.array([[[81888, 28748], [81888, 24724], [65594, 46048]]])
+    scene, spec = screen_triangle_scene(sr, tri, np.float32([[w0, w1, w1]]), W, H)
+    attach_dummy(sr, scene)
+    cam = scenes.make_camera(spec)
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam, threads=16)
+    want = o.read_frame()
+    assert want["ids"][py, px] == 0 and np.isinf(want["depth"][py, px])
+    r = sr.Renderer(W, H)
+    r.render_scene(sr.Scene(scene), cam)
+    ids, depth = r.read_vbuffer()
+    rgb = r.read_color()
+    r.close()
+    assert np.array_equal(ids, want["ids"]), (ids[py, px], int((ids != want["ids"]).sum()))
+    assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32))
+    assert np.array_equal(rgb, want["rgb"], equal_nan=True)
