@@ -484,6 +484,10 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
  * front end. */
 SR_API int sr_renderer_read_bins(sr_renderer *renderer, uint32_t *start, uint32_t *end, uint32_t *list,
                                  uint64_t list_len, uint32_t *items);
+/* Parity hook: *direct is 1 if the last frame's lists were made by the direct
+ * binning (small frames without large triangles), 0 if by the radix passes;
+ * both make the same lists. */
+SR_API int sr_renderer_direct_binning(sr_renderer *renderer, int32_t *direct);
 /* Device pointers of the last frame's visibility buffer and colour (for
  * in-HBM consumers); valid until the next render call. */
 SR_API int sr_renderer_device_buffers(sr_renderer *renderer, void **tri_id, void **depth,

@@ -229,6 +229,7 @@ _SIGS = {
     "sr_server_read_pixels": (C.c_int, [_P, C.c_uint64, C.POINTER(C.c_uint32)]),
     "sr_server_read_vbuffer": (C.c_int, [_P, C.c_uint64, C.POINTER(C.c_uint32), C.POINTER(C.c_float)]),
     "sr_server_release": (C.c_int, [_P, C.c_uint64]),
+    "sr_renderer_direct_binning": (C.c_int, [_P, C.POINTER(C.c_int32)]),
     "sr_renderer_read_bins": (C.c_int, [_P, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32),
                                         C.c_uint64, C.POINTER(C.c_uint32)]),
     "sr_server_drain": (C.c_int, [_P]),
@@ -800,6 +801,12 @@ class Renderer:
         out = np.empty(n.value, np.float32)
         check(lib().sr_renderer_read_tile_luminance(self.handle, _fptr(out), C.byref(n)))
         return out
+
+    def direct_binning(self):
+        """Whether the last frame's lists were made by the direct binning."""
+        n = C.c_int32()
+        check(lib().sr_renderer_direct_binning(self.handle, C.byref(n)))
+        return bool(n.value)
 
     def read_bins(self):
         """The last frame's per-tile lists: (start, end, list) arrays."""

@@ -819,6 +819,7 @@ struct SetupOut {
     SR_GLOBAL uint32_t *matrix;
     SR_GLOBAL uint32_t *chunk_first;
     uint32_t items, nchunks;
+    int large_rects;                      // the status's large_rects is asked for
 };
 
 __device__ __forceinline__ int32_t top_left_bias(int32_t a, int32_t b) { return (a < 0 || (a == 0 && b > 0)) ? 0 : -1; }
@@ -1125,6 +1126,20 @@ __device__ __forceinline__ void count_rect(uint32_t *hist, const RectBins &b) {
     }
 }
 
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(v), 63);
+}
+
+// Most (triangle, tile) pairs of 64 consecutive input triangles that the direct
+// binning takes: their lanes count them in LDS, and k_bin_place's workgroup
+// ranks its four waves' pairs 1024 at a time, one batch after the other, where
+// the radix passes use the whole chip.  Setup and binning of 200 to 20,000
+// triangles of one size, direct against radix, meet at 16 to 24 pairs a
+// triangle at 640x360 and 1280x720 (57 us both for 5000 of 11, 66 both for
+// 17, 116 against 76 for 44) and at 12 at 1920x1080; 64 triangles over a
+// whole 1080p frame took 5943 us without a limit and 877 by the passes.
+#define DB_MAX_WAVE_PAIRS 768u
+
 // The post-clip id of input triangle t is its chunk's first id plus the
 // fan counts before it in the chunk (a workgroup scan); it is stored for
 // the per-view offsets.  A triangle inside the frustum is set up from its
@@ -1132,7 +1147,7 @@ __device__ __forceinline__ void count_rect(uint32_t *hist, const RectBins &b) {
 // the polygon k_clip left in the clip buffer (ids tri_base[t] + f).
 // DIRECT (small frames, see the direct binning): `chunk` holds the chunks'
 // counts, which each workgroup adds up itself (no scan before it), and the
-// chunk's pairs are counted per tile in LDS.
+// chunk's pairs are counted per tile in LDS, up to DB_MAX_WAVE_PAIRS a wave.
 template <bool DIRECT>
 __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDraw *draws, int ndraws, uint32_t total,
                                                const float4 *xs, const uint32_t *counts, const uint32_t *chunk,
@@ -1176,8 +1191,11 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
             }
         }
         RectBins rb = rect_bins(views, view, r);
-        uint32_t np = (uint32_t)rb.nb;
-        if constexpr (DIRECT) count_rect(hist, rb);
+        uint32_t np = (uint32_t)rb.nb, wave_pairs = 0u;
+        if constexpr (DIRECT) {
+            wave_pairs = wave_sum(np);
+            if (wave_pairs <= DB_MAX_WAVE_PAIRS) count_rect(hist, rb);
+        }
         int nclip = (c & SR_COUNT_CLIPPED) ? (int)nf : 0;
         int maxf = __ballot(nclip > 0) ? wave_max(nclip) : 0;
         for (int f = 0; f < maxf; f++) {
@@ -1187,9 +1205,13 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
                                       id + (uint32_t)f, O);
             rb = rect_bins(views, view, rf);
             np += (uint32_t)rb.nb;
-            if constexpr (DIRECT) count_rect(hist, rb);
+            if constexpr (DIRECT) {
+                wave_pairs += wave_sum((uint32_t)rb.nb);
+                if (wave_pairs <= DB_MAX_WAVE_PAIRS) count_rect(hist, rb);
+            }
         }
         if constexpr (DIRECT) {
+            if (wave_pairs > DB_MAX_WAVE_PAIRS && (threadIdx.x & 63) == 0) O.status->large_rects = 1u;
             __syncthreads();
             SR_GLOBAL uint4 *row = reinterpret_cast<SR_GLOBAL uint4 *>(O.matrix + (size_t)(base >> 8) * O.items);
             const uint4 *h = reinterpret_cast<const uint4 *>(hist);
@@ -1199,6 +1221,11 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
             uint32_t npx;
             uint32_t chunk_np = block_excl_scan(np, npx, sh);
             if (threadIdx.x == 0) O.chunk_pairs[base >> 8] = chunk_np;
+            if (O.large_rects) {
+                wave_pairs = (uint32_t)__builtin_amdgcn_readlane((int)(npx + np), 63) -
+                             (uint32_t)__builtin_amdgcn_readlane((int)npx, 0);
+                if (wave_pairs > DB_MAX_WAVE_PAIRS && (threadIdx.x & 63) == 0) O.status->large_rects = 1u;
+            }
         }
     }
 }
@@ -1541,7 +1568,9 @@ __global__ void __launch_bounds__(256) k_bin_bounds(BinBounds B) {
 // them in setup.  The matrix moves 4 B per entry four times and the gain over
 // the radix passes falls with it: whole frames 132 -> 102 us at 0.3M entries,
 // 188 -> 137 at 0.7M, 194 -> 171 at 2.2M, 260 -> 248 at 2.7M, so frames with
-// more than DB_MAX_ENTRIES keep the passes.
+// more than DB_MAX_ENTRIES keep the passes.  So do those with large triangles
+// (DB_MAX_WAVE_PAIRS): setup finds them and says so in the status, the lists
+// then stay empty, and the host runs the frame again by the passes.
 #define DB_MAX_CHUNKS 1024u
 #define DB_MAX_ITEMS 8192u           // tile counters in LDS
 #define DB_MAX_ENTRIES (3u << 20)
@@ -1610,6 +1639,10 @@ __global__ void __launch_bounds__(256) k_bin_place(BinDirect P) {
     const uint32_t quads = (P.items + 1023u) / 1024u, t0 = 4u * quads * tid;
     const SR_GLOBAL uint32_t *totals = P.matrix + (size_t)P.nchunks * P.items;
     const SR_GLOBAL uint32_t *row = P.matrix + (size_t)c * P.items;
+    // large_rects: the counts are incomplete and the frame runs again, without
+    // direct binning; until then the tiles' bounds stay empty
+    const uint32_t total = min(P.status->total_records, P.rec_cap);
+    const bool again = P.status->large_rects != 0u;
     {
         uint4 n[QUADS];
         uint32_t sum = 0u, run;
@@ -1620,6 +1653,7 @@ __global__ void __launch_bounds__(256) k_bin_place(BinDirect P) {
             sum += (n[q].x + n[q].y) + (n[q].z + n[q].w);
         }
         const uint32_t pairs = block_excl_scan(sum, run, sh);
+        if (again) return;
         if (c == 0u && tid == 0u) P.status->total_pairs = pairs;
 #pragma unroll
         for (uint32_t q = 0; q < QUADS; q++) {
@@ -1636,7 +1670,6 @@ __global__ void __launch_bounds__(256) k_bin_place(BinDirect P) {
             }
         }
     }
-    const uint32_t total = min(P.status->total_records, P.rec_cap);
     const uint32_t last = min(c + 1u < P.nchunks ? P.chunk_first[c + 1u] : total, total);
     for (uint32_t r0 = P.chunk_first[c]; r0 < last; r0 += 256u) {
         const uint32_t id = r0 + tid;
@@ -4047,6 +4080,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     so.chunk_first = (SR_GLOBAL uint32_t *)a.chunk_pairs;
     so.items = a.total_items;
     so.nchunks = nchunks;
+    so.large_rects = a.direct || bin_matrix_entries(a.total_in, a.total_items) > 0;
     if (a.direct) {
         SR_LAUNCH_TIMED_LDS(ev_none, a.events[1], k_setup<true>, dim3(nchunks), dim3(256), a.total_items * 4u, st,
                             a.views, a.draws, a.num_draws, a.total_in, a.xv + 3 * (size_t)a.total_xv, a.tri_counts,

@@ -68,8 +68,9 @@ struct Carve {
 
 extern "C" {
 
-SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camera, int32_t width, int32_t height,
-                                   float exposure, uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream) {
+// The frame; *again is set if it must be rendered without direct binning.
+static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t width, int32_t height, float exposure,
+                        uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream, bool allow_direct, bool *again) {
     if (!scene || !camera || !tri_id || !depth || !rgba) return fail(SR_ERR_INVALID_ARGUMENT, "null argument");
     if (width <= 0 || height <= 0 || width > 32000 || height > 32000)
         return fail(SR_ERR_INVALID_ARGUMENT, "frame size must be in 1..32000");
@@ -131,10 +132,12 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
         (uint32_t)std::min<uint64_t>(std::min<uint64_t>(rec_want, rest * 4 / 5 / rec_bytes), 0xFFFFFFF0ull);
     uint32_t pair_cap = (uint32_t)std::min<uint64_t>((rest - (uint64_t)rec_cap * rec_bytes) / pair_bytes, 0xFFFFFFF0ull);
     // a small frame's direct binning needs its count matrix instead of the
-    // pairs' arrays: taken where that holds no fewer records and entries
+    // pairs' arrays: taken where that holds no fewer records and entries, and
+    // the scene's last frame had no triangles too large for it (if this one
+    // has, it runs again by the radix passes)
     bool direct = false;
     const uint64_t matrix = (uint64_t)bin_matrix_entries(total_in, items) * 4;
-    if (matrix > 0 && matrix + 256 < rest) {
+    if (matrix > 0 && matrix + 256 < rest && allow_direct) {
         const uint64_t left = rest - matrix - 256;
         const uint64_t rc = std::min<uint64_t>(rec_want, left * 4 / 5 / rec_bytes);
         const uint64_t pc = std::min<uint64_t>((left - rc * rec_bytes) / 4, 0xFFFFFFF0ull);
@@ -214,6 +217,11 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
         return fail(SR_ERR_HIP, "frame: %s", hipGetErrorString(hipGetLastError()));
     if (s.clip_overflow)
         return fail(SR_ERR_UNSUPPORTED, "a frustum-clipped polygon exceeded 16 vertices (degenerate rounding)");
+    scene->noalloc_large.store(s.large_rects != 0, std::memory_order_relaxed);
+    if (direct && s.large_rects) {
+        *again = true;
+        return SR_OK;
+    }
     if (s.overflow_records || s.overflow_pairs || s.overflow_clip || s.total_records > rec_cap ||
         s.total_pairs > pair_cap || s.clip_queued > clip_cap)
         return fail(SR_ERR_CAPACITY,
@@ -221,6 +229,16 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
                     "and %u",
                     s.total_records, s.total_pairs, s.clip_queued, rec_cap, pair_cap, clip_cap);
     return SR_OK;
+}
+
+SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camera, int32_t width, int32_t height,
+                                   float exposure, uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream) {
+    bool again = false;
+    const bool direct = scene && !scene->noalloc_large.load(std::memory_order_relaxed);
+    int rc = render_frame(scene, camera, width, height, exposure, tri_id, depth, rgba, stream, direct, &again);
+    if (!rc && again)
+        rc = render_frame(scene, camera, width, height, exposure, tri_id, depth, rgba, stream, false, &again);
+    return rc;
 }
 
 }  // extern "C"

@@ -479,6 +479,14 @@ SR_API int sr_renderer_set_stage_timing(sr_renderer *r, int32_t mode) {
     return SR_OK;
 }
 
+SR_API int sr_renderer_direct_binning(sr_renderer *r, int32_t *direct) {
+    if (!r || !direct) return fail(SR_ERR_INVALID_ARGUMENT, "null argument");
+    if (int rc = finish(r)) return rc;
+    if (!r->has_frame) return fail(SR_ERR_INVALID_ARGUMENT, "no frame rendered yet");
+    *direct = r->pipe.last_direct ? 1 : 0;
+    return SR_OK;
+}
+
 SR_API int sr_renderer_read_bins(sr_renderer *r, uint32_t *start, uint32_t *end, uint32_t *list, uint64_t list_len,
                                  uint32_t *items) {
     if (!r) return fail(SR_ERR_INVALID_ARGUMENT, "null renderer");

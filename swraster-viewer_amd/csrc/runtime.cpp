@@ -318,12 +318,13 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
     if (rec_cap < total_in + total_in / 8 + 1024) rec_cap = total_in + total_in / 8 + 1024;
     if (pair_cap < rec_cap * 2) pair_cap = rec_cap * 2;
     if (clip_cap < 4096) clip_cap = 4096;
-    // direct binning for small frames, unless the last frame's triangles
-    // spanned more than eight tiles each on average: one workgroup ranks a
-    // chunk's pairs, 1024 at a time, where the expansion takes up to eight
+    // direct binning for small frames without large triangles: setup finds
+    // those (DB_MAX_WAVE_PAIRS), the frame then runs again by the radix passes,
+    // and so do the next ones until setup finds none
     const size_t matrix = bin_matrix_entries(total_in, total_items);
-    for (int attempt = 0; attempt < 4; attempt++) {
-        const bool direct = matrix > 0 && last_pairs <= 8ull * std::max<uint32_t>(last_records, 1u);
+    for (int attempt = 0; attempt < 5; attempt++) {
+        const bool direct = matrix > 0 && !last_large;
+        last_direct = direct;
         // every attempt is a frame of its own number
         DevStatus init;
         memset(&init, 0, sizeof(init));
@@ -437,12 +438,13 @@ int Pipeline::settle(bool has_tr, bool &again) {
     const DevStatus &s = frame_status();
     last_records = s.total_records;
     last_pairs = s.total_pairs;
+    last_large = s.large_rects != 0;
     again = false;
     if (s.clip_overflow)
         return fail(SR_ERR_UNSUPPORTED, "a frustum-clipped polygon exceeded 16 vertices (degenerate rounding)");
     bool tr_ok = !has_tr || (!s.overflow_tr && s.total_tr_pairs <= tr_cap);
     if (!s.overflow_records && !s.overflow_pairs && !s.overflow_clip && s.total_records <= rec_cap &&
-        s.total_pairs <= pair_cap && tr_ok)
+        s.total_pairs <= pair_cap && tr_ok && !(last_direct && last_large))
         return SR_OK;
     again = true;
     if (!tr_ok) tr_cap = s.total_tr_pairs + s.total_tr_pairs / 8 + 4096;

@@ -71,6 +71,7 @@ struct Pipeline {
     PinBuf stage, status_host;
     uint32_t rec_cap = 0, pair_cap = 0, clip_cap = 0, tr_cap = 0;
     uint32_t last_records = 0, last_pairs = 0;
+    bool last_direct = false, last_large = false;     // direct binning used; rectangles too large for it
     bool last_near = false;           // the last frame's raster took entries nearest first (k_raster_near)
     struct GraphKey {
         uint64_t n[16];
@@ -108,6 +109,7 @@ struct sr_scene {
     bool any_tangents = false;
     bool any_translucent = false;     // a node draws a translucent primitive
     std::atomic<int> pending_frames{0};   // renderer frames queued and not yet checked
+    mutable std::atomic<bool> noalloc_large{false};   // its last no-allocation frame had large_rects
     uint64_t triangles = 0, vertices = 0, device_bytes = 0;
 };
 

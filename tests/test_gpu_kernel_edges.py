@@ -288,6 +288,42 @@ def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
     assert np.all(np.diff(out[0][2].astype(np.int64)) >= 0) and out[0][3][-1] == out[0][5]
 
 
+def _mixed(sr, scenes, W, H, n, radius, huge=0):
+    from util import attach_dummy, mixed_triangle_scene
+    scene, spec = mixed_triangle_scene(sr, W, H, n, radius, huge)
+    attach_dummy(sr, scene)
+    return scene, scenes.make_camera(spec, W, H)
+
+
+def test_large_triangles_leave_direct_binning(sr, scenes):
+    """A frame with three screen-filling triangles among small ones is binned
+    by the radix passes: a renderer's first frame, a frame after small ones,
+    and as long as the last one had such triangles; frames without them go
+    back to the direct binning.  All have the frame that radix passes give."""
+    W, H = 640, 360
+    small, cam = _mixed(sr, scenes, W, H, 3000, 40)
+    large, _ = _mixed(sr, scenes, W, H, 3000, 40, huge=3)
+    want = {}
+    for name, data in (("small", small), ("large", large)):
+        more = _with_backfacing(sr, data, 262144)
+        more.attach(data.environment, data.voxels)
+        r = sr.Renderer(W, H)
+        r.render_scene(sr.Scene(more), cam)
+        assert not r.direct_binning()
+        want[name] = (*r.read_vbuffer(), *r.read_bins())
+        r.close()
+    gpu = {"small": sr.Scene(small), "large": sr.Scene(large)}
+    r = sr.Renderer(W, H)
+    for k, (name, direct) in enumerate((("large", False), ("large", False), ("small", False), ("small", True),
+                                        ("large", False), ("small", False), ("small", True))):
+        r.render_scene(gpu[name], cam)
+        got = (*r.read_vbuffer(), *r.read_bins())
+        assert r.direct_binning() == direct, (k, name)
+        for x, y in zip(got, want[name]):
+            assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), (k, name)
+    r.close()
+
+
 def _gi(sr, scene, env, grid, device):
     g = sr.sr_voxel_grid()
     scene.environment = env

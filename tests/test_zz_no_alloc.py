@@ -97,6 +97,23 @@ def test_noalloc_heightfield_1080p(sr, scenes, env):
     check_same(sr, got, plain(sr, g, cam, 1920, 1080), "c2 1920x1080")
 
 
+def test_noalloc_large_triangles(sr, scenes):
+    """Screen-filling triangles among small ones, which the direct binning
+    leaves to the radix passes (the scene's first call finds that out, the
+    second knows), then the same scene without them in view."""
+    from util import attach_dummy, mixed_triangle_scene
+    W, H = 640, 360
+    scene, spec = mixed_triangle_scene(sr, W, H, 3000, 40, huge=3)
+    attach_dummy(sr, scene)
+    g = sr.Scene(scene)
+    away = dict(spec, yaw=spec["yaw"] + np.pi / 2)
+    for name, sp in (("large, first", spec), ("large, second", spec), ("away", away), ("large again", spec)):
+        cam = scenes.make_camera(sp, W, H)
+        rc, msg, got = noalloc(sr, g, cam, W, H)
+        assert rc == 0, msg
+        check_same(sr, got, plain(sr, g, cam, W, H), name)
+
+
 def test_noalloc_rejects_what_does_not_fit(sr, scenes, env):
     """A 2M-triangle heightfield needs more than the scratch array holds: the
     call fails with SR_ERR_CAPACITY before launching anything; a translucent

@@ -110,3 +110,21 @@ def dark_environment(sr, sky=(128, 160, 200)):
     spec = np.full(3 * 6 * 16, black, np.uint32)
     lut = np.full(64, sr.pack_rgba(np.array([[200, 40, 0, 255]], np.uint8))[0], np.uint32)
     return sr.Environment(cube, spec, 3, lut, np.zeros((4, 3), np.float32))
+
+
+def mixed_triangle_scene(sr, W, H, n, radius, huge=0, seed=3):
+    """n triangles of about 5 px radius over the view, one in 70 of them of
+    the given radius, and `huge` more over the whole view after the first
+    hundred, at random depths."""
+    rng = np.random.default_rng(seed)
+    rad = np.where(np.arange(n) % 70 == 35, radius, 6.0) * rng.uniform(0.7, 1.0, n)
+    rad = np.insert(rad, 100, np.full(huge, 2.0 * W))
+    n += huge
+    c = rng.uniform([0, 0], [W * 16, H * 16], (n, 1, 2))
+    c[100:100 + huge] = [W * 8, H * 8]
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2])
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * (rad * 16)[:, None, None])
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    return screen_triangle_scene(sr, tris, rng.uniform(2.0, 90.0, n), W, H)
