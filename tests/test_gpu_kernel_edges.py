@@ -248,13 +248,15 @@ def _with_backfacing(sr, scene, n):
 # which 262,144 more triangles (1024 chunks) make them take: tile counts of
 # one, a few and exactly 8192, sizes that leave tiles off screen, all tile
 # sizes; "near" stands close to the terrain, so many triangles cross the
-# frustum, "big" has rectangles of more than 32 tiles
+# frustum, "mixed" has rectangles of more than 32 tiles among small ones and
+# more pairs than a first frame has room for (it runs again, direct still)
 @pytest.mark.parametrize("kind,W,H,tile", [("cluster", 16, 16, 32), ("cluster", 64, 64, 16), ("cluster", 333, 202, 8),
                                            ("cluster", 2048, 1024, 16), ("near", 640, 360, 16), ("near", 500, 301, 32),
-                                           ("big", 640, 480, 16), ("big", 1023, 130, 8)])
+                                           ("mixed", 640, 480, 16), ("mixed", 1023, 130, 8)])
 def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
     """The tiles' lists, the visibility buffer and the pair count of a small
-    frame are those that the radix passes give."""
+    frame are those that the radix passes give, and so are the views of a
+    batch of three."""
     if kind == "cluster":
         scene, spec = scenes.make_c1(width=W, height=H)
         # one node: all spheres in world space, so the copies come last
@@ -269,7 +271,8 @@ def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
         scene, spec = scenes.make_c2(width=W, height=H, grid=120, tex_size=64)
         spec["position"] = [0.0, 4.0, 10.0]
     else:
-        scene, spec = scenes.make_c3(width=W, height=H, triangles=900, primitives=7)
+        from util import mixed_triangle_scene
+        scene, spec = mixed_triangle_scene(sr, W, H, 12000, 4 * tile)
     more = _with_backfacing(sr, scene, 262144)
     scene.prepare(env, grid=16)
     more.attach(scene.environment, scene.voxels)
@@ -281,7 +284,17 @@ def test_direct_binning_equals_radix(sr, scenes, env, kind, W, H, tile):
         r.render_scene(gscene, cam)
         ids, depth = r.read_vbuffer()
         out.append((ids, depth.view(np.uint32), *r.read_bins(), r.stats()["binned_pairs"]))
+        assert r.direct_binning() == (data is scene)
         r.close()
+        if data is scene:
+            b = sr.Batch(tile_size=tile)
+            b.render([(gscene, cam, W, H, 0.0), (gscene, cam, 50, 70, 0.0), (gscene, cam, W, H, 0.0)])
+            views = [b.read_vbuffer(k) for k in (0, 2)]
+            b.close()
+    if kind == "mixed":
+        assert out[0][5] > 2 * (12000 + 12000 // 8 + 1024)       # the first frame's room
+    for ids, depth in views:
+        assert np.array_equal(ids, out[1][0]) and np.array_equal(depth.view(np.uint32), out[1][1])
     assert out[0][5] == out[1][5] and out[0][5] > 0
     for a, b in zip(out[0][:5], out[1][:5]):
         assert np.array_equal(a, b)
