@@ -2837,8 +2837,11 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
 // instructions a wave; in this order with four waves sharing a tile (one
 // setting up at a time, barriers in each round) 396 us at 1286, which is 0.69
 // of the issue rate; one wave a tile needs no barrier and took 195 us at
-// 3420, 0.94 of it (182 with shorter scans and without the alpha test).  Frames of small triangles (the heightfield) keep
-// k_raster, whose four waves share their long lists.
+// 3420, 0.94 of it (182 with shorter scans and without the alpha test).
+// Pixels off the screen must not hold quadrants open: with the last row of
+// tiles half below a 640x360 view, 92,727 triangles (5841 entries a tile) took
+// 740 us, and the frame 1141 (without 478).  Frames of small triangles (the
+// heightfield) keep k_raster, whose four waves share their long lists.
 // ---------------------------------------------------------------------------
 #define NEAR_BATCH 256
 
@@ -2876,8 +2879,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     const DevScene &S = *V.scene;
     const uint32_t tile = item - V.item_base;
     const int tx0 = (int)(tile % (uint32_t)V.tiles_x) * T, ty0 = (int)(tile / (uint32_t)V.tiles_x) * T;
+    // pixels off the screen that nobody reads (all but the centre quad's) are
+    // in front of everything from the start, so they hold no quadrant open
 #pragma unroll
-    for (int i = 0; i < T * T; i += 64) keys[i + lane] = SR_EMPTY_KEY;
+    for (int i = 0; i < T * T; i += 64) {
+        const int p = i + lane, px = tx0 + p % T, py = ty0 + p / T;
+        const bool read = (px < V.W && py < V.H) || (centre_tile(tx0, ty0) && px < tx0 + 2 && py < ty0 + 2);
+        keys[p] = read ? SR_EMPTY_KEY : 0ull;
+    }
     __syncthreads();
     const uint32_t nrec = P.status->total_records;
     uint32_t start, end;

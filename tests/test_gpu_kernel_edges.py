@@ -181,6 +181,43 @@ def test_overdraw_raster_list_lengths(sr, orc, n, kind):
     r.close()
 
 
+# sizes that leave part of a tile, whole quadrants or whole tiles off the
+# screen, the centre quad of a 64-px tile among them (32 rows: just off it)
+@pytest.mark.parametrize("size", [(64, 32), (70, 40), (33, 97), (47, 34), (640, 360)])
+def test_overdraw_raster_screen_edges(sr, orc, size):
+    """Large triangles reaching past the right and bottom edge: both
+    renderings (the second by the overdraw raster) have the oracle's
+    visibility buffer and tile luminance."""
+    from util import attach_dummy, screen_triangle_scene
+    import swraster_viewer_amd.scenes as sc
+    W, H = size
+    n = 300 + W * H // 80
+    rng = np.random.default_rng(W + H)
+    c = rng.uniform([0, 0], [(W + 20) * 16, (H + 20) * 16], (n, 1, 2))
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2]) + rng.uniform(-0.4, 0.4, (n, 3))
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * (rng.uniform(40, 90, (n, 3)) * 16)[..., None])
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    scene, spec = screen_triangle_scene(sr, tris, rng.uniform(2.0, 90.0, (n, 1)) * rng.uniform(0.9, 1.1, (n, 3)), W, H)
+    attach_dummy(sr, scene)
+    cam = sc.make_camera(spec)
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()
+    gscene = sr.Scene(scene)
+    r = sr.Renderer(W, H)
+    for k in range(2):
+        r.render_scene(gscene, cam)
+        ids, depth = r.read_vbuffer()
+        assert np.array_equal(ids, want["ids"]), f"frame {k}"
+        assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32)), f"frame {k}"
+        assert np.array_equal(r.read_tile_luminance().view(np.uint32),
+                              np.asarray(o.tile_luminance(), np.float32).view(np.uint32)), f"frame {k}"
+    assert r.stats()["depth_rejection"] == 1
+    r.close()
+
+
 # the raster variants with the alpha test: each tile size, and the overdraw
 # raster (tile 16, a list of 300); "far" minifies the texture to its last levels
 @pytest.mark.parametrize("n,tile,far", [(24, 8, False), (24, 16, True), (24, 32, False), (300, 16, False),
