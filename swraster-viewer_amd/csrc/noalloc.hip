@@ -18,6 +18,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -100,7 +101,8 @@ static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t 
     const int sort_passes = bin_sort_passes(items);
     if (sort_passes < 1) return fail(SR_ERR_CAPACITY, "%u screen tiles; at most 2^24", items);
     Carve c;
-    uint64_t o_views = c.take(upload + sizeof(BinSortState));
+    // (no room for the persistent raster's queues, which this frame has not)
+    uint64_t o_views = c.take(upload + offsetof(BinSortState, work));
     uint64_t o_xv = c.take((uint64_t)std::max<uint32_t>(total_xv, 1) * 64);
     uint64_t o_counts = c.take(((uint64_t)total_in + 1) * 4);
     uint64_t o_chunks = c.take(((uint64_t)total_in / 256 + 2) * 4);

@@ -114,6 +114,23 @@ def test_noalloc_large_triangles(sr, scenes):
         check_same(sr, got, plain(sr, g, cam, W, H), name)
 
 
+def test_noalloc_scratch_room(sr, scenes):
+    """The scratch of a 1080p frame of 1000 triangles, which are clipped into
+    more records than it holds, has room for 7,917,183 list entries of the
+    radix passes: none of it goes to state that the frame has not (the queues
+    of a persistent raster)."""
+    import re
+    from util import attach_dummy, screen_triangle_scene
+    W, H, n = 1920, 1080, 1000
+    tri = np.array([[[-16000, -16000], [-16000, 64000], [64000, -16000]]])
+    scene, spec = screen_triangle_scene(sr, np.tile(tri, (n, 1, 1)), np.linspace(2, 90, n), W, H)
+    attach_dummy(sr, scene)
+    rc, msg, _ = noalloc(sr, sr.Scene(scene), scenes.make_camera(spec), W, H)
+    assert rc == SR_ERR_CAPACITY
+    records, entries, clipped = map(int, re.search(r"scratch holds (\d+), (\d+) and (\d+)", msg).groups())
+    assert records == n + n // 8 + 1024 and entries >= 7917183, msg
+
+
 def test_noalloc_rejects_what_does_not_fit(sr, scenes, env):
     """A 2M-triangle heightfield needs more than the scratch array holds: the
     call fails with SR_ERR_CAPACITY before launching anything; a translucent
