@@ -64,7 +64,8 @@ struct FrameArgs {
     float4 *center_color;         // 4 (colour, depth) per 64px tile
     int32_t persistent_blocks;    // 0 = one block per item
     int32_t direct;               // direct binning: sort_hist holds bin_matrix_entries words; no pair arrays.
-                                  // The frame runs again without it if its status says large_rects
+                                  // 1: leaves the lists empty if the status says large_rects, and the frame
+                                  // runs again without it; 2: makes them however large the triangles
     int32_t overdraw;             // 16-px raster that takes overdrawn tiles' entries nearest first
     hipEvent_t events[5];         // optional stage events (the launches that carry them cost about 4 us each):
                                   // start, setup done, bins done, shade done, raster done

@@ -820,6 +820,7 @@ struct SetupOut {
     SR_GLOBAL uint32_t *chunk_first;
     uint32_t items, nchunks;
     int large_rects;                      // the status's large_rects is asked for
+    uint32_t max_wave_pairs;              // k_setup<true> counts no more
 };
 
 __device__ __forceinline__ int32_t top_left_bias(int32_t a, int32_t b) { return (a < 0 || (a == 0 && b > 0)) ? 0 : -1; }
@@ -1147,7 +1148,7 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 // the polygon k_clip left in the clip buffer (ids tri_base[t] + f).
 // DIRECT (small frames, see the direct binning): `chunk` holds the chunks'
 // counts, which each workgroup adds up itself (no scan before it), and the
-// chunk's pairs are counted per tile in LDS, up to DB_MAX_WAVE_PAIRS a wave.
+// chunk's pairs are counted per tile in LDS, up to max_wave_pairs a wave.
 template <bool DIRECT>
 __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDraw *draws, int ndraws, uint32_t total,
                                                const float4 *xs, const uint32_t *counts, const uint32_t *chunk,
@@ -1194,7 +1195,7 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
         uint32_t np = (uint32_t)rb.nb, wave_pairs = 0u;
         if constexpr (DIRECT) {
             wave_pairs = wave_sum(np);
-            if (wave_pairs <= DB_MAX_WAVE_PAIRS) count_rect(hist, rb);
+            if (wave_pairs <= O.max_wave_pairs) count_rect(hist, rb);
         }
         int nclip = (c & SR_COUNT_CLIPPED) ? (int)nf : 0;
         int maxf = __ballot(nclip > 0) ? wave_max(nclip) : 0;
@@ -1207,7 +1208,7 @@ __global__ void __launch_bounds__(256) k_setup(const DevView *views, const DevDr
             np += (uint32_t)rb.nb;
             if constexpr (DIRECT) {
                 wave_pairs += wave_sum((uint32_t)rb.nb);
-                if (wave_pairs <= DB_MAX_WAVE_PAIRS) count_rect(hist, rb);
+                if (wave_pairs <= O.max_wave_pairs) count_rect(hist, rb);
             }
         }
         if constexpr (DIRECT) {
@@ -1587,7 +1588,7 @@ struct BinDirect {
     SR_GLOBAL DevStatus *status;
     uint64_t *stamp;
     uint32_t nchunks, items, rec_cap, pair_cap;
-    int T, bits;
+    int T, bits, any_size;
 };
 
 __global__ void __launch_bounds__(1024) k_bin_cols(BinDirect P) {
@@ -1642,7 +1643,7 @@ __global__ void __launch_bounds__(256) k_bin_place(BinDirect P) {
     // large_rects: the counts are incomplete and the frame runs again, without
     // direct binning; until then the tiles' bounds stay empty
     const uint32_t total = min(P.status->total_records, P.rec_cap);
-    const bool again = P.status->large_rects != 0u;
+    const bool again = P.status->large_rects != 0u && !P.any_size;
     {
         uint4 n[QUADS];
         uint32_t sum = 0u, run;
@@ -4089,6 +4090,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
     so.chunk_first = (SR_GLOBAL uint32_t *)a.chunk_pairs;
     so.items = a.total_items;
     so.nchunks = nchunks;
+    so.max_wave_pairs = a.direct == 2 ? 0xFFFFFFFFu : DB_MAX_WAVE_PAIRS;
     so.large_rects = a.direct || bin_matrix_entries(a.total_in, a.total_items) > 0;
     if (a.direct) {
         SR_LAUNCH_TIMED_LDS(ev_none, a.events[1], k_setup<true>, dim3(nchunks), dim3(256), a.total_items * 4u, st,
@@ -4125,6 +4127,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
         bd.pair_cap = a.pair_cap;
         bd.T = a.tile_size;
         bd.bits = nbits;
+        bd.any_size = a.direct == 2;
         hipLaunchKernelGGL(k_bin_cols, dim3((a.total_items + DB_COL_TILES - 1u) / DB_COL_TILES), dim3(1024), 0, st, bd);
         hipLaunchKernelGGL(k_bin_place, dim3(nchunks), dim3(256), a.total_items * 4u, st, bd);
         e = hipGetLastError();

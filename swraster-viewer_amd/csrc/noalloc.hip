@@ -55,6 +55,11 @@ int scratch_ptr(int dev, uint8_t **out) {
     return SR_OK;
 }
 
+// How a frame is binned: directly, to be run again if its triangles are too
+// large for that; by the radix passes; directly whatever the triangles (their
+// lists take 4 B an entry instead of 17 or 21, so it holds more of them).
+enum { BIN_DIRECT, BIN_RADIX, BIN_ANY_SIZE };
+
 // Consecutive 256-byte aligned pieces of the scratch array.
 struct Carve {
     uint64_t used = 0;
@@ -69,9 +74,11 @@ struct Carve {
 
 extern "C" {
 
-// The frame; *again is set if it must be rendered without direct binning.
+// The frame, binned as asked (or by the radix passes, where its sizes leave no
+// choice).  *again: it must be rendered again, binned so; else -1.
 static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t width, int32_t height, float exposure,
-                        uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream, bool allow_direct, bool *again) {
+                        uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream, int binning, int *again) {
+    *again = -1;
     if (!scene || !camera || !tri_id || !depth || !rgba) return fail(SR_ERR_INVALID_ARGUMENT, "null argument");
     if (width <= 0 || height <= 0 || width > 32000 || height > 32000)
         return fail(SR_ERR_INVALID_ARGUMENT, "frame size must be in 1..32000");
@@ -134,20 +141,20 @@ static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t 
         (uint32_t)std::min<uint64_t>(std::min<uint64_t>(rec_want, rest * 4 / 5 / rec_bytes), 0xFFFFFFF0ull);
     uint32_t pair_cap = (uint32_t)std::min<uint64_t>((rest - (uint64_t)rec_cap * rec_bytes) / pair_bytes, 0xFFFFFFF0ull);
     // a small frame's direct binning needs its count matrix instead of the
-    // pairs' arrays: taken where that holds no fewer records and entries, and
-    // the scene's last frame had no triangles too large for it (if this one
-    // has, it runs again by the radix passes)
-    bool direct = false;
+    // pairs' arrays: possible where that holds no fewer records and entries
     const uint64_t matrix = (uint64_t)bin_matrix_entries(total_in, items) * 4;
-    if (matrix > 0 && matrix + 256 < rest && allow_direct) {
+    const uint32_t radix_pairs = pair_cap;
+    uint64_t direct_records = 0, direct_pairs = 0;
+    if (matrix > 0 && matrix + 256 < rest) {
         const uint64_t left = rest - matrix - 256;
-        const uint64_t rc = std::min<uint64_t>(rec_want, left * 4 / 5 / rec_bytes);
-        const uint64_t pc = std::min<uint64_t>((left - rc * rec_bytes) / 4, 0xFFFFFFF0ull);
-        direct = rc >= rec_cap && pc >= pair_cap;
-        if (direct) {
-            rec_cap = (uint32_t)std::min<uint64_t>(rc, 0xFFFFFFF0ull);
-            pair_cap = (uint32_t)pc;
-        }
+        direct_records = std::min<uint64_t>(std::min<uint64_t>(rec_want, left * 4 / 5 / rec_bytes), 0xFFFFFFF0ull);
+        direct_pairs = std::min<uint64_t>((left - direct_records * rec_bytes) / 4, 0xFFFFFFF0ull);
+    }
+    const bool can_direct = direct_records >= rec_cap && direct_pairs >= pair_cap;
+    const bool direct = can_direct && binning != BIN_RADIX;
+    if (direct) {
+        rec_cap = (uint32_t)direct_records;
+        pair_cap = (uint32_t)direct_pairs;
     }
     uint64_t o_geo = c.take((uint64_t)rec_cap * 16);
     uint64_t o_ras = c.take((uint64_t)rec_cap * 64);
@@ -191,7 +198,7 @@ static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t 
     a.pair_vals = (uint32_t *)(base + o_pairs[1]);
     a.pair_keys2 = (uint32_t *)(base + o_pairs[2]);
     if (sort_passes > 1) a.pair_vals2 = (uint32_t *)(base + o_pairs[3]);
-    a.direct = direct ? 1 : 0;
+    a.direct = !direct ? 0 : binning == BIN_DIRECT ? 1 : 2;
     a.sort_hist = (uint32_t *)(base + o_hist);
     a.chunk_pairs = (uint32_t *)(base + o_chunk_pairs);
     a.rec_geo = (uint4 *)(base + o_geo);
@@ -219,11 +226,21 @@ static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t 
         return fail(SR_ERR_HIP, "frame: %s", hipGetErrorString(hipGetLastError()));
     if (s.clip_overflow)
         return fail(SR_ERR_UNSUPPORTED, "a frustum-clipped polygon exceeded 16 vertices (degenerate rounding)");
-    scene->noalloc_large.store(s.large_rects != 0, std::memory_order_relaxed);
-    if (direct && s.large_rects) {
-        *again = true;
-        return SR_OK;
+    // the scene's next frame: direct binning if this one had no triangles too
+    // large for it, else the radix passes if they hold the lists
+    const bool large = s.large_rects != 0;
+    if (direct && binning == BIN_DIRECT) {
+        if (large) *again = BIN_RADIX;
+    } else if (!direct && can_direct && !s.overflow_records && !s.overflow_clip && s.total_records <= rec_cap &&
+               s.clip_queued <= clip_cap && s.total_pairs > radix_pairs && s.total_pairs <= direct_pairs) {
+        *again = BIN_ANY_SIZE;
     }
+    int next = BIN_DIRECT;
+    if (large)
+        next = *again == BIN_ANY_SIZE || (direct && binning == BIN_ANY_SIZE && s.total_pairs > radix_pairs) ? BIN_ANY_SIZE
+                                                                                                       : BIN_RADIX;
+    scene->noalloc_binning.store(next, std::memory_order_relaxed);
+    if (*again >= 0) return SR_OK;
     if (s.overflow_records || s.overflow_pairs || s.overflow_clip || s.total_records > rec_cap ||
         s.total_pairs > pair_cap || s.clip_queued > clip_cap)
         return fail(SR_ERR_CAPACITY,
@@ -235,11 +252,10 @@ static int render_frame(const sr_scene *scene, const sr_camera *camera, int32_t 
 
 SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camera, int32_t width, int32_t height,
                                    float exposure, uint32_t *tri_id, float *depth, uint32_t *rgba, void *stream) {
-    bool again = false;
-    const bool direct = scene && !scene->noalloc_large.load(std::memory_order_relaxed);
-    int rc = render_frame(scene, camera, width, height, exposure, tri_id, depth, rgba, stream, direct, &again);
-    if (!rc && again)
-        rc = render_frame(scene, camera, width, height, exposure, tri_id, depth, rgba, stream, false, &again);
+    int again = scene ? scene->noalloc_binning.load(std::memory_order_relaxed) : BIN_DIRECT, rc = SR_OK;
+    do {
+        rc = render_frame(scene, camera, width, height, exposure, tri_id, depth, rgba, stream, again, &again);
+    } while (!rc && again >= 0);
     return rc;
 }
 

@@ -109,7 +109,7 @@ struct sr_scene {
     bool any_tangents = false;
     bool any_translucent = false;     // a node draws a translucent primitive
     std::atomic<int> pending_frames{0};   // renderer frames queued and not yet checked
-    mutable std::atomic<bool> noalloc_large{false};   // its last no-allocation frame had large_rects
+    mutable std::atomic<int> noalloc_binning{0};      // how its next no-allocation frame is binned (noalloc.hip)
     uint64_t triangles = 0, vertices = 0, device_bytes = 0;
 };
 

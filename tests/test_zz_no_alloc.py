@@ -114,6 +114,23 @@ def test_noalloc_large_triangles(sr, scenes):
         check_same(sr, got, plain(sr, g, cam, W, H), name)
 
 
+def test_noalloc_lists_that_only_direct_binning_holds(sr, scenes):
+    """1000 screen-filling triangles at 1080p have 8.2 million list entries,
+    more than the scratch has room for with the radix passes' arrays: the
+    direct binning takes them, however large its triangles are."""
+    from util import attach_dummy, screen_triangle_scene
+    W, H, n = 1920, 1080, 1000
+    tri = np.array([[[16, 16], [16, H * 16 - 16], [W * 16 - 16, 16]]])
+    scene, spec = screen_triangle_scene(sr, np.tile(tri, (n, 1, 1)), np.linspace(90, 2, n), W, H)
+    attach_dummy(sr, scene)
+    g, cam = sr.Scene(scene), scenes.make_camera(spec, W, H)
+    want = plain(sr, g, cam, W, H)
+    for k in range(2):
+        rc, msg, got = noalloc(sr, g, cam, W, H)
+        assert rc == 0, msg
+        check_same(sr, got, want, f"call {k}")
+
+
 def test_noalloc_scratch_room(sr, scenes):
     """The scratch of a 1080p frame of 1000 triangles, which are clipped into
     more records than it holds, has room for 7,917,183 list entries of the
