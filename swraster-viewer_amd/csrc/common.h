@@ -148,6 +148,7 @@ struct DevStatus {
     uint32_t clip_overflow;       // a clipped polygon outgrew its room (frame fails)
     uint32_t total_tr_pairs;      // (translucent triangle, 64-px tile) pairs
     uint32_t overflow_tr;
+    uint32_t long_tr_list;        // a tile's translucent list is longer than LDS holds
     uint32_t large_rects;         // 64 consecutive triangles have more pairs than the direct binning takes
     uint32_t seq;                 // the frame's number, set by the host in the upload
 };

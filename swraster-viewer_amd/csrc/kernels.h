@@ -59,7 +59,8 @@ struct FrameArgs {
     uint32_t *tr_start;           // tr_slots
     uint32_t *tr_end;             // tr_slots (cursor, then end)
     uint32_t *tr_list;            // tr_cap record ids
-    unsigned long long *tr_scratch;  // tr_cap x 20 B: sort room for lists longer than LDS holds
+    unsigned long long *tr_scratch;  // tr_cap x 20 B: sort room for lists longer than LDS holds (null: none;
+                                  // the frame runs again with it if its status says long_tr_list)
     uint32_t tr_cap;
     float4 *center_color;         // 4 (colour, depth) per 64px tile
     int32_t persistent_blocks;    // 0 = one block per item

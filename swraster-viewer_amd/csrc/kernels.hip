@@ -3627,7 +3627,7 @@ __device__ __forceinline__ void tr_order(V v, int n, uint32_t *out, C *ties, R c
 // then cap counts.
 __global__ void __launch_bounds__(TR_SORT_NT) k_tr_sort(const uint32_t *tr_start, const uint32_t *tr_end,
                                                         uint32_t *list, uint32_t cap, unsigned long long *scratch,
-                                                        const float4 *raster, TriSource src) {
+                                                        const float4 *raster, TriSource src, DevStatus *status) {
     __shared__ unsigned long long sk[TR_SORT_MAX];
     __shared__ uint16_t ties[TR_SORT_MAX];
     __shared__ uint32_t ranges[TR_SORT_MAX];
@@ -3637,6 +3637,10 @@ __global__ void __launch_bounds__(TR_SORT_NT) k_tr_sort(const uint32_t *tr_start
     uint32_t s = tr_start[slot], e = min(tr_end[slot], cap);
     if (e <= s + 1) return;
     const int n = (int)(e - s);
+    if (tr_end[slot] - s > TR_SORT_MAX) {
+        if (threadIdx.x == 0) status->long_tr_list = 1u;
+        if (!scratch) return;
+    }
     auto key_of = [&](int i) {
         uint32_t id = list[s + i];
         return ((unsigned long long)z_desc_key(tri_avg_z(src, raster + 4 * (size_t)id)) << 32) | id;
@@ -4210,7 +4214,7 @@ hipError_t launch_frame(const FrameArgs &a, hipStream_t st) {
         hipLaunchKernelGGL(k_tr_bins, dim3(g), dim3(256), 0, st, a.views, a.rec_geo, a.rec_cap, a.tr_end, a.tr_list,
                            a.tr_cap, slot_bits, a.status);
         hipLaunchKernelGGL(k_tr_sort, dim3(a.tr_slots), dim3(TR_SORT_NT), 0, st, a.tr_start, a.tr_end, a.tr_list, a.tr_cap,
-                           a.tr_scratch, a.rec_raster, src);
+                           a.tr_scratch, a.rec_raster, src, a.status);
     }
     RasterArgs P;
     P.views = (const SR_GLOBAL DevView *)a.views; P.num_views = a.num_views; P.total_items = a.total_items;

@@ -345,7 +345,7 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
             if ((r = sort_hist.ensure((size_t)bin_sort_tiles(pair_cap) * 256 * 4))) return r;
         }
         if (has_tr && (r = tr_list.ensure((size_t)tr_cap * 4))) return r;
-        if (has_tr && (r = tr_scratch.ensure((size_t)tr_cap * 20))) return r;
+        if (has_tr && tr_room && (r = tr_scratch.ensure((size_t)tr_cap * 20))) return r;
         FrameArgs a;
         memset(&a, 0, sizeof(a));
         a.views = (const DevView *)views.ptr;
@@ -400,7 +400,7 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
             a.tr_start = (uint32_t *)tr_start.ptr;
             a.tr_end = (uint32_t *)tr_end.ptr;
             a.tr_list = (uint32_t *)tr_list.ptr;
-            a.tr_scratch = (unsigned long long *)tr_scratch.ptr;
+            a.tr_scratch = tr_room ? (unsigned long long *)tr_scratch.ptr : nullptr;
             a.tr_cap = tr_cap;
             a.center_color = (float4 *)center_color.ptr;
         }
@@ -446,12 +446,13 @@ int Pipeline::settle(bool has_tr, bool &again) {
     again = false;
     if (s.clip_overflow)
         return fail(SR_ERR_UNSUPPORTED, "a frustum-clipped polygon exceeded 16 vertices (degenerate rounding)");
-    bool tr_ok = !has_tr || (!s.overflow_tr && s.total_tr_pairs <= tr_cap);
+    bool tr_ok = !has_tr || (!s.overflow_tr && s.total_tr_pairs <= tr_cap && (tr_room || !s.long_tr_list));
     if (!s.overflow_records && !s.overflow_pairs && !s.overflow_clip && s.total_records <= rec_cap &&
         s.total_pairs <= pair_cap && tr_ok && !(last_direct && last_large))
         return SR_OK;
     again = true;
-    if (!tr_ok) tr_cap = s.total_tr_pairs + s.total_tr_pairs / 8 + 4096;
+    if (has_tr && s.long_tr_list) tr_room = true;
+    if (has_tr && (s.overflow_tr || s.total_tr_pairs > tr_cap)) tr_cap = s.total_tr_pairs + s.total_tr_pairs / 8 + 4096;
     if (s.overflow_clip || s.clip_queued > clip_cap) clip_cap = s.clip_queued + s.clip_queued / 4 + 1024;
     if (clip_cap > (1u << 27))      // clip-queue slots are 27-bit fields of the counts and record tags
         return fail(SR_ERR_CAPACITY, "more than 2^27 triangles cross the frustum");

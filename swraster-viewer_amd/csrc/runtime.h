@@ -71,6 +71,7 @@ struct Pipeline {
     PinBuf stage, status_host;
     uint32_t rec_cap = 0, pair_cap = 0, clip_cap = 0, tr_cap = 0;
     uint32_t last_records = 0, last_pairs = 0;
+    bool tr_room = false;             // tr_scratch is there: a frame had a list too long to sort in LDS
     bool last_direct = false, last_large = false;     // direct binning used; rectangles too large for it
     bool last_near = false;           // the last frame's raster took entries nearest first (k_raster_near)
     struct GraphKey {

@@ -77,6 +77,32 @@ def test_translucent_sort_sizes(sr, orc, scenes, env, n, levels):
     assert np.array_equal(rgb.view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32))
 
 
+def test_translucent_long_list_later(sr, orc, scenes, env):
+    """The room to sort a list of more than 4096 is taken when a frame first
+    has one: after a frame of 7000 triangles in two tiles, whose lists fit,
+    one of 5000 in one tile outgrows no other buffer and has the oracle's
+    colour, and so has the next of each."""
+    W, H = 128, 64
+    cam = scenes.make_camera(scenes.camera_spec((0, 0, 0), 0.0, 0.0, np.pi / 3, W, H, 20.0))
+    pairs = []
+    for n, sides in ((7000, (-1.15, 1.15)), (5000, (1.15, 1.15))):
+        scene = _glass_layers(sr, scenes, n, n, n)
+        for prim in scene.primitives:
+            p = prim["positions"].reshape(-1, 3, 3)
+            p[::2, :, 0] += np.float32(sides[0])
+            p[1::2, :, 0] += np.float32(sides[1])
+        scene.rebuild()
+        scene.prepare(env, grid=16)
+        o = orc.OracleRenderer(W, H)
+        o.render_scene(orc.OracleScene(scene), cam)
+        pairs.append((sr.Scene(scene), np.ascontiguousarray(o.read_frame()["rgb"], np.float32)))
+    r = sr.Renderer(W, H)
+    for k in (0, 1, 0, 1):
+        r.render_scene(pairs[k][0], cam)
+        assert np.array_equal(r.read_color().view(np.uint32), pairs[k][1].view(np.uint32)), k
+    r.close()
+
+
 @pytest.mark.parametrize("size", [(16, 16), (63, 65), (130, 97)])
 def test_translucent_walk_edges(sr, orc, scenes, env, size):
     """The forward pass keeps only the entries that meet each 16x16 block
