@@ -484,6 +484,11 @@ SR_API int sr_render_frame_noalloc(const sr_scene *scene, const sr_camera *camer
  * front end. */
 SR_API int sr_renderer_read_bins(sr_renderer *renderer, uint32_t *start, uint32_t *end, uint32_t *list,
                                  uint64_t list_len, uint32_t *items);
+/* Parity hook: compares the shading's and raster's short divisions and roots
+ * on `device` with IEEE division and square root.  mismatches: of the
+ * reciprocal and of 1 / sqrt, over every float in [2^-96, 2^96], and of the
+ * quotient, over `pairs` pairs drawn from `seed` with exponents within +-40. */
+SR_API int sr_check_short_forms(int32_t device, uint64_t seed, uint64_t pairs, uint64_t mismatches[3]);
 /* Parity hook: *direct is 1 if the last frame's lists were made by the direct
  * binning (small frames without large triangles), 0 if by the radix passes;
  * both make the same lists. */

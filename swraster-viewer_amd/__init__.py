@@ -229,6 +229,7 @@ _SIGS = {
     "sr_server_read_pixels": (C.c_int, [_P, C.c_uint64, C.POINTER(C.c_uint32)]),
     "sr_server_read_vbuffer": (C.c_int, [_P, C.c_uint64, C.POINTER(C.c_uint32), C.POINTER(C.c_float)]),
     "sr_server_release": (C.c_int, [_P, C.c_uint64]),
+    "sr_check_short_forms": (C.c_int, [C.c_int32, C.c_uint64, C.c_uint64, C.POINTER(C.c_uint64)]),
     "sr_renderer_direct_binning": (C.c_int, [_P, C.POINTER(C.c_int32)]),
     "sr_renderer_read_bins": (C.c_int, [_P, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32),
                                         C.c_uint64, C.POINTER(C.c_uint32)]),

@@ -50,6 +50,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "short_div.h"
 #include "swraster.h"
 #include "tri_bound.h"
 
@@ -88,39 +89,6 @@ __device__ __forceinline__ uint32_t sat_index(float f, uint32_t limit) {
     uint32_t v = (uint32_t)f;
     return v < limit ? v : limit;
 }
-// Divisions and square roots with fewer instructions than the compiler's (which
-// scale their operands and fix up every special case), for operands known to
-// be in range: each gives the IEEE result.  Checked against IEEE division and
-// square root on gfx950 for every float in [2^-96, 2^96] (the reciprocal, the
-// root, and both in turn) and for 1.7e10 random pairs with exponents within
-// +-40 (the quotient: with the correctly rounded reciprocal of b, one fused
-// correction of a rcp(b) by its exact residual rounds correctly).
-__device__ __forceinline__ float rcp_in_range(float b) {
-    float y = __builtin_amdgcn_rcpf(b);
-    return fmaf(fmaf(-b, y, 1.0f), y, y);
-}
-// 1 / b for any b.  (The 1/w that a sample interpolates is between its
-// vertices' only inside the triangle; covered samples of a triangle whose
-// integer edge constants wrap lie anywhere, and it can be zero there.)
-__device__ __forceinline__ float rcp_ieee(float b) {
-    if (b >= 0x1p-96f && b <= 0x1p96f) return rcp_in_range(b);
-    return 1.0f / b;
-}
-// a / b from y = rcp(b), correctly rounded.
-__device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
-    float q = a * y;
-    return fmaf(fmaf(-b, q, a), y, q);
-}
-__device__ __forceinline__ float div_in_range(float a, float b) { return div_by_rcp(a, b, rcp_in_range(b)); }
-// SHORT: with the short forms where x is in range.
-template <bool SHORT = true> __device__ __forceinline__ float rsqrt_ieee(float x) {
-    if (SHORT && x >= 0x1p-96f && x <= 0x1p96f) {
-        float y = __builtin_amdgcn_rsqf(x), g = x * y;
-        return rcp_in_range(fmaf(fmaf(-g, g, x), 0.5f * y, g));
-    }
-    return 1.0f / sqrtf(x);
-}
-
 struct f3 { float x, y, z; };
 __device__ __forceinline__ f3 mk3(float x, float y, float z) { return {x, y, z}; }
 __device__ __forceinline__ f3 add3(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }

@@ -460,3 +460,12 @@ def test_zero_denominator_sample(sr, orc, scenes, w0, w1, px, py):
     assert np.array_equal(ids, want["ids"]), (ids[py, px], int((ids != want["ids"]).sum()))
     assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32))
     assert np.array_equal(rgb, want["rgb"], equal_nan=True)
+
+
+def test_short_divisions_and_roots_are_ieee(sr):
+    """The reciprocal and 1 / sqrt in their short forms for every float in
+    [2^-96, 2^96], the quotient for 4e9 random pairs with exponents within
+    +-40: all equal IEEE division and square root bit for bit."""
+    bad = (sr.C.c_uint64 * 3)()
+    sr.check(sr.lib().sr_check_short_forms(0, 20240229, 4 * 10 ** 9, bad))
+    assert list(bad) == [0, 0, 0]
