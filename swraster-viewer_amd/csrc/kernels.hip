@@ -1927,7 +1927,9 @@ __device__ __forceinline__ float tri_const(float k, float fx, float fy, float fz
 
 __device__ __forceinline__ void voxel_lookup(const DevScene &S, f3 p, f3 rgb[4], float &w0, float &w1) {
     float vx = p.x - S.vox_min[0], vy = p.y - S.vox_min[1], vz = p.z - S.vox_min[2];
-    if (S.vox_rcp[0] > 0.0f) {
+    // (the quotients' residuals need the offsets within 2^+-80)
+    const float far = fmaxf(fmaxf(fabsf(vx), fabsf(vy)), fabsf(vz)), near = fminf(fminf(fabsf(vx), fabsf(vy)), fabsf(vz));
+    if (S.vox_rcp[0] > 0.0f && far <= 0x1p80f && near >= 0x1p-80f) {
         vx = div_by_rcp(vx, S.vox_size[0], S.vox_rcp[0]);
         vy = div_by_rcp(vy, S.vox_size[1], S.vox_rcp[1]);
         vz = div_by_rcp(vz, S.vox_size[2], S.vox_rcp[2]);

@@ -26,10 +26,10 @@ __device__ __forceinline__ float rcp_ieee(float b) {
     if (b >= 0x1p-96f && b <= 0x1p96f) return rcp_in_range(b);
     return 1.0f / b;
 }
-// a / b from y = rcp(b), for a (or a zero) and b within 2^+-40: with the
-// correctly rounded reciprocal of b, one fused correction of a y by its exact
-// residual rounds correctly.  That holds as long as neither the quotient nor
-// the residual leaves the floats' range.
+// a / b from y = rcp(b), correctly rounded: with the correctly rounded
+// reciprocal of b, one fused correction of a y by its exact residual.  That
+// holds while neither the quotient nor the residual leaves the floats' range:
+// for b within 2^+-40, while a is a zero or within 2^+-80.
 __device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
     float q = a * y;
     return fmaf(fmaf(-b, q, a), y, q);

@@ -469,3 +469,39 @@ def test_short_divisions_and_roots_are_ieee(sr):
     bad = (sr.C.c_uint64 * 3)()
     sr.check(sr.lib().sr_check_short_forms(0, 20240229, 4 * 10 ** 9, bad))
     assert list(bad) == [0, 0, 0]
+
+
+# heights of the floor over the grid's corner, down to where the quotient by
+# the voxel's size is denormal
+@pytest.mark.parametrize("y", [1e-30, 3e-34, 1.3e-36, 2e-38])
+def test_voxel_lookup_tiny_offsets(sr, orc, scenes, y):
+    """A floor a hair above the voxel grid's corner, dark below and lit above:
+    the light is the height over the voxel's size, in sizes that are no power
+    of two, and it is the oracle's to the bit however small."""
+    from util import dark_environment
+    W, H = 96, 64
+    rng = np.random.default_rng(5)
+    n = 40
+    p = np.zeros((n * n, 3), np.float32)
+    g = np.linspace(-2, 2, n)
+    p[:, 0], p[:, 2] = np.tile(g, n), np.repeat(g, n)
+    p[:, 1] = (y * rng.uniform(0.2, 1.0, n * n)).astype(np.float32)
+    i = (np.arange(n - 1)[:, None] * n + np.arange(n - 1)).reshape(-1, 1)
+    idx = np.concatenate([i, i + n, i + 1, i + 1, i + n, i + n + 1], 1).reshape(-1).astype(np.uint32)
+    prim = {"positions": p, "normals": np.tile(np.float32([0, 1, 0]), (n * n, 1)), "texcoords": None, "tangents": None,
+            "indices": idx, "material": 0}
+    mat = {"base_color": (1.0, 1.0, 1.0, 1.0), "metallic": 0.0, "roughness": 0.5}
+    scene = sr.SceneData([prim], [(0, 1)], [(np.eye(4, dtype=np.float32), 0)], [mat], [], name="floor")
+    light = np.repeat(np.float32([0.0, 1.0]), 2)[None].repeat(2, 0).reshape(-1)      # [z][y][x]: by y
+    scene.attach(dark_environment(sr), sr.VoxelGrid((2, 2, 2), np.float32([-3, 0, -3]), np.float32([3, 3.4567, 3]), light))
+    cam = scenes.make_camera(scenes.camera_spec((0, 1.5, 3), 0.0, 0.5, np.pi / 3, W, H, 50.0))
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = np.ascontiguousarray(o.read_frame()["rgb"], np.float32)
+    r = sr.Renderer(W, H)
+    r.render_scene(sr.Scene(scene), cam)
+    ids, rgb = r.read_vbuffer()[0], r.read_color()
+    r.close()
+    lit = rgb[ids != sr.NO_ID]
+    assert len(lit) > 1000 and 0 < lit.max() < 10 * y
+    assert np.array_equal(rgb.view(np.uint32), want.view(np.uint32)), int((rgb != want).any(-1).sum())
