@@ -259,7 +259,7 @@ int gi_bake_host(const GiHost &h, const std::vector<uint8_t> &active, const std:
         float rad[GI_SAMPLES * 3];
         uint32_t sky_hits = 0;
         bool ov = false;
-        GiLocalStack st;
+        GiStack st;
         for (int s = 0; s < GI_SAMPLES; s++) {
             bool sky = false;
             G3 r = gi_primary_ray(S, c, g3(dirs[3 * s], dirs[3 * s + 1], dirs[3 * s + 2]), h.primary_bias, h.params, sky,

@@ -66,7 +66,7 @@ struct GiScene {
 
 // Traversal stack in a private array (host).  The device walks a copy of the
 // tree in the same order (gi.hip).
-struct GiLocalStack {
+struct GiStack {
     int32_t s[GI_STACK];
     int n = 0;
     GI_HD void push(int32_t v) { s[n++] = v; }
@@ -143,8 +143,7 @@ struct GiHit {
 
 // RayTracer::trace_nearest (src/raytracer.rs:135-172): depth-first, right
 // child first; boxes beyond the current nearest distance are skipped.
-template <class Stack>
-GI_HD bool gi_trace_nearest(const GiScene &S, G3 o, G3 d, float tmin, GiHit &hit, Stack &st) {
+GI_HD bool gi_trace_nearest(const GiScene &S, G3 o, G3 d, float tmin, GiHit &hit, GiStack &st) {
     if (S.nnodes == 0) return false;
     G3 inv = g3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     st.n = 0;
@@ -182,8 +181,7 @@ GI_HD bool gi_trace_nearest(const GiScene &S, G3 o, G3 d, float tmin, GiHit &hit
 
 // RayTracer::trace_transmittance (src/raytracer.rs:174-207).  over is set if
 // more than GI_HIT_CAP translucent surfaces lie on the ray.
-template <class Stack>
-GI_HD float gi_trace_transmittance(const GiScene &S, G3 o, G3 d, float tmin, bool &over, Stack &st) {
+GI_HD float gi_trace_transmittance(const GiScene &S, G3 o, G3 d, float tmin, bool &over, GiStack &st) {
     if (S.nnodes == 0) return 1.0f;
     G3 inv = g3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     st.n = 0;
@@ -303,9 +301,8 @@ GI_HD G3 gi_sky_dir(G3 normal, int k) {
 }
 
 // sky_visibility_hemisphere4 (src/gi.rs:549-570)
-template <class Stack>
 GI_HD float gi_sky_visibility(const GiScene &S, G3 origin, G3 normal, float dir_bias, float tmin, bool &over,
-                              Stack &st) {
+                              GiStack &st) {
     float vis = 0.0f;
     for (int k = 0; k < 4; k++) {
         G3 dir = gi_sky_dir(normal, k);
@@ -359,9 +356,8 @@ GI_HD G3 gi_bounce_finish(const GiScene &S, G3 normal, G3 albedo, G3 emissive, f
 }
 
 // estimate_surface_bounce_radiance (src/gi.rs:450-547)
-template <class Stack>
 GI_HD G3 gi_bounce(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const GiRayParams &P, bool &over,
-                   Stack &st) {
+                   GiStack &st) {
     G3 normal, albedo, emissive, shading_origin;
     if (!gi_bounce_surface(S, hit, o, incoming, P, normal, albedo, emissive, shading_origin)) return g3(0.0f, 0.0f, 0.0f);
     float dir_bias = P.hit_bias * 0.5f;
@@ -377,9 +373,8 @@ GI_HD G3 gi_bounce(const GiScene &S, const GiHit &hit, G3 o, G3 incoming, const 
 
 // Incident radiance along primary direction dir from the voxel centre
 // (one iteration of the ray loop of bake_voxel_gi, src/gi.rs:372-388).
-template <class Stack>
 GI_HD G3 gi_primary_ray(const GiScene &S, G3 center, G3 dir, float primary_bias, const GiRayParams &P, bool &sky,
-                        bool &over, Stack &st) {
+                        bool &over, GiStack &st) {
     G3 o = gadd(center, gscale(dir, primary_bias));
     GiHit hit;
     if (gi_trace_nearest(S, o, dir, P.tmin, hit, st)) {
