@@ -234,7 +234,7 @@ typedef struct sr_batch_stats {
     uint64_t binned_pairs;
     uint64_t pixels;
     uint32_t views;
-    uint32_t work_items;      /* (view, tile) items drained by the persistent kernel */
+    uint32_t work_items;      /* (view, tile) items of the raster */
     float ms_total;
 } sr_batch_stats;
 
@@ -503,8 +503,10 @@ SR_API int sr_batch_create(const sr_batch_opts *opts, sr_batch **out);
 SR_API int sr_batch_destroy(sr_batch *batch);
 /* Changes the persistent raster workgroup count (> 0; 0 keeps it; -1 launches
  * one raster workgroup per (view, tile) instead) and hipGraph use of an
- * existing batch; the tile size is fixed at creation.  Used by the autotuner
- * (no reference counterpart). */
+ * existing batch; the tile size is fixed at creation.  Launches whose overdraw
+ * selects the raster that takes entries nearest first (16-px tiles) have one
+ * wave per (view, tile) whatever the count.  Used by the autotuner (no
+ * reference counterpart). */
 SR_API int sr_batch_configure(sr_batch *batch, int32_t persistent_blocks, int32_t use_graph);
 /* Renders every view; per-view outputs are written to device memory owned
  * by the batch and read back with sr_batch_read_*. */

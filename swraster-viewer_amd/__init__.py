@@ -856,7 +856,9 @@ class Batch:
         self.sizes = []
 
     def configure(self, persistent_blocks=0, use_graph=False):
-        """Persistent raster workgroup count (0 keeps it) and hipGraph use."""
+        """Persistent raster workgroup count (0 keeps it, -1: one per (view, tile))
+        and hipGraph use.  Launches with high overdraw at 16-px tiles have one
+        wave per (view, tile) whatever the count."""
         check(lib().sr_batch_configure(self.handle, int(persistent_blocks), int(use_graph)))
 
     def render(self, views):

@@ -2,7 +2,8 @@
 
 Picks the screen-tile size (8, 16 or 32 px) and the number of persistent
 raster workgroups (or -1: one raster workgroup per (view, tile), which wins
-for few large views) for a set of views by timing the real batch, and keeps the
+for few large views; it has no effect on launches whose overdraw selects the
+near-first raster, at 16-px tiles) for a set of views by timing the real batch, and keeps the
 choice in a JSON cache keyed by device and a coarse workload signature (view
 count, log2 of total pixels and of total triangles).  Numerics do not depend
 on either knob; only time does.  The bin lists hold one 4-byte entry per
