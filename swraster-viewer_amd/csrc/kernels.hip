@@ -2808,7 +2808,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(T == 32
 // instructions a wave; in this order with four waves sharing a tile (one
 // setting up at a time, barriers in each round) 396 us at 1286, which is 0.69
 // of the issue rate; one wave a tile needs no barrier and took 195 us at
-// 3420, 0.94 of it (182 with shorter scans and without the alpha test).
+// 3420, 0.94 of it (181 at 3137 with shorter scans and without the alpha
+// test, 189 at 3161 with bounds as wide as the edge values' rounding).
 // Pixels off the screen must not hold quadrants open: with the last row of
 // tiles half below a 640x360 view, 92,727 triangles (5841 entries a tile) took
 // 740 us, and the frame 1141 (without 478).  Frames of small triangles (the
