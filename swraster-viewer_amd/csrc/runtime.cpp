@@ -410,9 +410,13 @@ int Pipeline::run(const std::vector<DevView> &hv, const std::vector<DevDraw> &hd
         // many of them (high overdraw); judged from the last frame.  Whole
         // frames of 40-px triangles over the view, by k_raster and
         // k_raster_near: 246 and 249 us at 14 pairs a tile, 307 and 251 at
-        // 48, 565 and 315 at 207 (1920x1080); 150 and 153 at 48, 182 and 164
-        // at 210 (320x240, where a wave a tile leaves SIMDs idle)
-        a.overdraw = tile_size == 16 && last_pairs > 32ull * total_items && last_pairs > 4ull * last_records;
+        // 48, 565 and 315 at 207 (1920x1080).  With few tiles one wave each
+        // leaves SIMDs idle and the line is higher: 320x240, 320 tiles, 128
+        // and 145 us at 44 pairs, 149 and 157 at 66, 157 and 163 at 106, 182
+        // and 164 at 197; over half the view only 163 and 164 at 65, 171 and
+        // 152 at 76
+        const uint64_t line = total_items < 512 ? 56 : 32;
+        a.overdraw = tile_size == 16 && last_pairs > line * total_items && last_pairs > 4ull * last_records;
         last_near = a.overdraw != 0;
         if (use_graph) {
             if ((r = launch_graph(a, vbytes, upload))) return r;

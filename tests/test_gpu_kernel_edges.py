@@ -207,6 +207,40 @@ def test_overdraw_raster_list_lengths(sr, orc, n, kind):
     r.close()
 
 
+# pairs a tile on both sides of the overdraw raster's line: 56 with fewer than
+# 512 tiles (320 here), 32 from there on (512)
+@pytest.mark.parametrize("W,H,pairs,near", [(320, 240, 45, 0), (320, 240, 80, 1), (512, 256, 24, 0), (512, 256, 45, 1)])
+def test_overdraw_raster_line(sr, orc, W, H, pairs, near):
+    """The raster that a second frame takes follows the pairs a tile, and both
+    frames have the oracle's visibility buffer."""
+    from util import attach_dummy, screen_triangle_scene
+    import swraster_viewer_amd.scenes as sc
+    rng = np.random.default_rng(pairs)
+    n = pairs * W * H // 256 // 25                 # 40-px triangles take about 25 tiles each
+    c = rng.uniform([0, 0], [W * 16, H * 16], (n, 1, 2))
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0.0, 2.1, 4.2])
+    tris = np.round(c + np.stack([np.cos(ang), np.sin(ang)], -1) * 640)
+    a = (tris[:, 1, 0] - tris[:, 0, 0]) * (tris[:, 2, 1] - tris[:, 0, 1]) - \
+        (tris[:, 2, 0] - tris[:, 0, 0]) * (tris[:, 1, 1] - tris[:, 0, 1])
+    tris[a > 0] = tris[a > 0][:, ::-1]
+    scene, spec = screen_triangle_scene(sr, tris, rng.uniform(2.0, 90.0, n), W, H)
+    attach_dummy(sr, scene)
+    cam = sc.make_camera(spec)
+    o = orc.OracleRenderer(W, H)
+    o.render_scene(orc.OracleScene(scene), cam)
+    want = o.read_frame()
+    gscene = sr.Scene(scene)
+    r = sr.Renderer(W, H)
+    for k in range(2):
+        r.render_scene(gscene, cam)
+        ids, depth = r.read_vbuffer()
+        assert np.array_equal(ids, want["ids"]), f"frame {k}"
+        assert np.array_equal(depth.view(np.uint32), want["depth"].view(np.uint32)), f"frame {k}"
+    st = r.stats()
+    r.close()
+    assert st["depth_rejection"] == near, st["binned_pairs"] / st["tiles"]
+
+
 # sizes that leave part of a tile, whole quadrants or whole tiles off the
 # screen, the centre quad of a 64-px tile among them (32 rows: just off it)
 @pytest.mark.parametrize("size", [(64, 32), (70, 40), (33, 97), (47, 34), (640, 360)])
